@@ -578,6 +578,8 @@ struct lbm_batch {
     void ensure_dense(size_t n) {
         if (dense_elems < n) {
             if (dense) (void)hipFree(dense);
+            dense = nullptr;
+            dense_elems = 0;
             dense = dalloc<float>(n);
             dense_elems = n;
         }
@@ -742,13 +744,16 @@ int lbm_batch_set_mask(lbm_batch *b, uint32_t d, const uint8_t *solid) {
     return bguard(b, [&] {
         bcheck(d < b->table.size() && solid, "bad domain or null mask");
         const DomainDev &dd = b->table[d];
-        std::vector<uint8_t> m((size_t)dd.g.X * dd.g.Y);
-        for (size_t i = 0; i < m.size(); ++i) m[i] = solid[i] == 1 ? 1 : 0;
         b->flush();  // the pending stream uses the old mask
-        HIPCHK(hipMemcpy2DAsync(b->mask + dd.aux_off, dd.g.pitch, m.data(), dd.g.X, dd.g.X, dd.g.Y,
-                                hipMemcpyHostToDevice, b->stream));
-        HIPCHK(hipStreamSynchronize(b->stream));
+        // the host's bytes go through the domain's flag plane, which is rebuilt
+        // (with the lists) before the next step
         b->dirty = true;
+        HIPCHK(hipMemcpyAsync(b->flags + dd.aux_off, solid, (size_t)dd.g.X * dd.g.Y, hipMemcpyHostToDevice,
+                              b->stream));
+        hipLaunchKernelGGL(k_place_mask, dim3((dd.g.X + 255) / 256, dd.g.Y), dim3(256), 0, b->stream,
+                           b->flags + dd.aux_off, b->mask + dd.aux_off, dd.g.X, dd.g.pitch);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipStreamSynchronize(b->stream));
     });
 }
 
@@ -943,11 +948,32 @@ int lbm_batch_read_moments(lbm_batch *b, uint32_t d, float *jx, float *jy, float
         const DomainDev &dd = b->table[d];
         const float *base = b->lag + 3 * dd.aux_off;
         float *dst[3] = {jx, jy, rho};
-        for (int c = 0; c < 3; ++c)
-            if (dst[c])
+        const size_t dn = (size_t)dd.g.X * dd.g.Y;
+        // padded planes are made dense on the device and copied in one piece
+        // each (row by row only where there is no memory to stage them)
+        const bool packed = dd.g.pitch == dd.g.X;
+        if (!packed) {
+            try {
+                b->ensure_dense(3 * dn);
+            } catch (const HipError &) {
+            }
+        }
+        const bool staged = !packed && b->dense_elems >= 3 * dn;
+        if (staged) {
+            hipLaunchKernelGGL(k_dense_planes, dim3((dd.g.X + 255) / 256, dd.g.Y, 3), dim3(256), 0, b->stream, base,
+                               b->dense, dd.g.X, dd.g.Y, dd.g.pitch, dd.g.pstride);
+            HIPCHK(hipGetLastError());
+        }
+        for (int c = 0; c < 3; ++c) {
+            if (!dst[c]) continue;
+            if (packed || staged)
+                HIPCHK(hipMemcpyAsync(dst[c], staged ? b->dense + c * dn : base + c * dd.g.pstride,
+                                      dn * sizeof(float), hipMemcpyDeviceToHost, b->stream));
+            else
                 HIPCHK(hipMemcpy2DAsync(dst[c], sizeof(float) * dd.g.X, base + c * dd.g.pstride,
                                         sizeof(float) * dd.g.pitch, sizeof(float) * dd.g.X, dd.g.Y,
                                         hipMemcpyDeviceToHost, b->stream));
+        }
         HIPCHK(hipStreamSynchronize(b->stream));
     });
 }

@@ -297,7 +297,8 @@ struct lbm_grid {
     float *lag = nullptr;   // jx, jy, rho planes: the renderer's density bind group
     float *now = nullptr;   // moments of the current state (scratch)
     float *out = nullptr;   // summary output plane (persistent)
-    float *dense = nullptr; // dense f32 staging (4 planes)
+    float *dense = nullptr; // dense f32 staging (dense_planes planes)
+    int dense_planes = 0;
     float *rgb = nullptr;   // colour-map output (3 floats per cell), allocated on first use
     size_t rgb_elems = 0;
     double *partials = nullptr;
@@ -542,8 +543,13 @@ struct lbm_grid {
     void ensure_now() {
         if (!now) now = dalloc<float>(3 * (size_t)geom.pstride);
     }
-    void ensure_dense() {
-        if (!dense) dense = dalloc<float>(4 * (size_t)X * Y);
+    void ensure_dense(int planes) {
+        if (dense_planes >= planes) return;
+        if (dense) (void)hipFree(dense);
+        dense = nullptr;
+        dense_planes = 0;
+        dense = dalloc<float>((size_t)planes * X * Y);
+        dense_planes = planes;
     }
     void ensure_partials() {
         if (!partials) {
@@ -622,7 +628,7 @@ struct lbm_grid {
 
     void copy_plane_out(const void *dev_plane, float *host, int k) {
         // decode one pitched population plane into a dense f32 host plane
-        ensure_dense();
+        ensure_dense(1);
         dim3 grid((X + 255) / 256, Y);
         by_store(precision, [&]<class St>() {
             hipLaunchKernelGGL(k_decode_plane<St>, grid, dim3(256), 0, stream, (const typename St::T *)dev_plane,
@@ -634,7 +640,7 @@ struct lbm_grid {
     }
 
     void copy_plane_in(const float *host, void *dev_plane, int k) {
-        ensure_dense();
+        ensure_dense(1);
         HIPCHK(hipMemcpyAsync(dense, host, sizeof(float) * X * Y, hipMemcpyHostToDevice, stream));
         dim3 grid((X + 255) / 256, Y);
         by_store(precision, [&]<class St>() {
@@ -651,9 +657,36 @@ struct lbm_grid {
         return ((size_t)y * geom.ys + (size_t)k * geom.ks + x) * esize;
     }
 
-    void copy_f32_plane_out(const float *dev, float *host) {
-        HIPCHK(hipMemcpy2DAsync(host, sizeof(float) * X, dev, sizeof(float) * geom.pitch, sizeof(float) * X, Y,
-                                hipMemcpyDeviceToHost, stream));
+    // n dense staging planes, or null where there is no memory for them
+    float *try_dense(int n) {
+        try {
+            ensure_dense(n);
+        } catch (const HipError &) {
+        }
+        return dense;
+    }
+
+    // n <= 3 pitched planes (pstride apart) to host planes, null ones left out:
+    // made dense on the device and copied in one piece each; row by row only
+    // where there is no memory to stage them
+    void copy_f32_planes_out(const float *dev, float *const *host, int n) {
+        const size_t bytes = sizeof(float) * X * Y;
+        const bool packed = geom.pitch == (int)X;
+        if (!packed && try_dense(n)) {
+            hipLaunchKernelGGL(k_dense_planes, dim3((X + 255) / 256, Y, n), dim3(256), 0, stream, dev, dense, (int)X,
+                               (int)Y, geom.pitch, geom.pstride);
+            HIPCHK(hipGetLastError());
+        }
+        for (int i = 0; i < n; ++i) {
+            if (!host[i]) continue;
+            const float *src = dev + (size_t)i * geom.pstride;
+            if (packed) HIPCHK(hipMemcpyAsync(host[i], src, bytes, hipMemcpyDeviceToHost, stream));
+            else if (dense)
+                HIPCHK(hipMemcpyAsync(host[i], dense + (size_t)i * X * Y, bytes, hipMemcpyDeviceToHost, stream));
+            else
+                HIPCHK(hipMemcpy2DAsync(host[i], sizeof(float) * X, src, sizeof(float) * geom.pitch,
+                                        sizeof(float) * X, Y, hipMemcpyDeviceToHost, stream));
+        }
     }
 };
 
@@ -917,11 +950,17 @@ int lbm_paint(lbm_grid *g, const uint32_t *pairs, size_t n_u32) {
 int lbm_set_mask(lbm_grid *g, const uint8_t *solid) {
     return guarded(g, [&] {
         check(solid != nullptr, "null mask");
-        std::vector<uint8_t> m((size_t)g->X * g->Y);
-        for (size_t i = 0; i < m.size(); ++i) m[i] = solid[i] == 1 ? 1 : 0;
         g->flush();
-        HIPCHK(hipMemcpy2DAsync(g->mask, g->geom.pitch, m.data(), g->X, g->X, g->Y, hipMemcpyHostToDevice,
-                                g->stream));
+        // the host's bytes go through the flag plane, which is rebuilt next
+        try {
+            HIPCHK(hipMemcpyAsync(g->flags, solid, (size_t)g->X * g->Y, hipMemcpyHostToDevice, g->stream));
+            hipLaunchKernelGGL(k_place_mask, dim3((g->X + 255) / 256, g->Y), dim3(256), 0, g->stream, g->flags,
+                               g->mask, (int)g->X, g->geom.pitch);
+            HIPCHK(hipGetLastError());
+        } catch (...) {
+            g->build_flags();  // of the mask as it was
+            throw;
+        }
         g->build_flags();
         HIPCHK(hipStreamSynchronize(g->stream));
     });
@@ -930,8 +969,14 @@ int lbm_set_mask(lbm_grid *g, const uint8_t *solid) {
 int lbm_get_mask(lbm_grid *g, uint8_t *solid) {
     return guarded(g, [&] {
         check(solid != nullptr, "null mask");
-        HIPCHK(hipMemcpy2DAsync(solid, g->X, g->mask, g->geom.pitch, g->X, g->Y, hipMemcpyDeviceToHost, g->stream));
+        // one copy of the pitched plane, its rows then moved on the host (a
+        // copy of separate rows costs 5 us a row)
+        const size_t pitch = (size_t)g->geom.pitch, bytes = pitch * g->Y;
+        std::vector<uint8_t> rows(pitch == g->X ? 0 : bytes);
+        HIPCHK(hipMemcpyAsync(rows.empty() ? solid : rows.data(), g->mask, bytes, hipMemcpyDeviceToHost, g->stream));
         HIPCHK(hipStreamSynchronize(g->stream));
+        if (!rows.empty())
+            for (uint32_t y = 0; y < g->Y; ++y) std::memcpy(solid + (size_t)y * g->X, rows.data() + y * pitch, g->X);
     });
 }
 
@@ -1241,10 +1286,8 @@ int lbm_read_moments(lbm_grid *g, float *jx, float *jy, float *rho, int lagged) 
             g->moments_now(false);
             src = g->now;
         }
-        const size_t ps = g->geom.pstride;
-        if (jx) g->copy_f32_plane_out(src, jx);
-        if (jy) g->copy_f32_plane_out(src + ps, jy);
-        if (rho) g->copy_f32_plane_out(src + 2 * ps, rho);
+        float *const dst[3] = {jx, jy, rho};
+        g->copy_f32_planes_out(src, dst, 3);
         HIPCHK(hipStreamSynchronize(g->stream));
     });
 }
@@ -1256,7 +1299,7 @@ int lbm_read_fields(lbm_grid *g, float *rho, float *ux, float *uy, float *curl, 
             g->moments_now(false);
             src = g->now;
         }
-        g->ensure_dense();
+        g->ensure_dense(4);
         hipLaunchKernelGGL(k_fields, dim3((g->X + 255) / 256, g->Y), dim3(256), 0, g->stream, src, g->dense, g->geom);
         HIPCHK(hipGetLastError());
         const size_t dn = (size_t)g->X * g->Y;
@@ -1271,10 +1314,15 @@ int lbm_read_fields(lbm_grid *g, float *rho, float *ux, float *uy, float *curl, 
 int lbm_summary(lbm_grid *g, int kind, float *out) {
     return guarded(g, [&] {
         check(kind >= 0 && kind <= 4, "unknown summary kind");
+        // a padded plane is also written dense, which the host copies in one piece
+        float *dense = out && g->geom.pitch != (int)g->X ? g->try_dense(1) : nullptr;
         hipLaunchKernelGGL(k_summary, dim3((g->X + 255) / 256, g->Y), dim3(256), 0, g->stream, g->lag, g->out, g->mask,
-                           (float *)nullptr, g->geom, kind, 0);
+                           (float *)nullptr, dense, g->geom, kind, 0);
         HIPCHK(hipGetLastError());
-        if (out) g->copy_f32_plane_out(g->out, out);
+        if (dense)
+            HIPCHK(hipMemcpyAsync(out, dense, sizeof(float) * g->X * g->Y, hipMemcpyDeviceToHost, g->stream));
+        else if (out)
+            g->copy_f32_planes_out(g->out, &out, 1);
         HIPCHK(hipStreamSynchronize(g->stream));
     });
 }
@@ -1292,7 +1340,7 @@ int lbm_render(lbm_grid *g, int kind, int colormap, float *rgb) {
             g->rgb_elems = n;
         }
         hipLaunchKernelGGL(k_summary, dim3((g->X + 255) / 256, g->Y), dim3(256), 0, g->stream, g->lag, g->out, g->mask,
-                           g->rgb, g->geom, kind, colormap);
+                           g->rgb, (float *)nullptr, g->geom, kind, colormap);
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(rgb, g->rgb, n * sizeof(float), hipMemcpyDeviceToHost, g->stream));
         HIPCHK(hipStreamSynchronize(g->stream));

@@ -838,6 +838,18 @@ __global__ void k_pack_input(const float *__restrict__ fields, uint16_t *__restr
     for (int c = 8; c < C; c += 8) *(u16x8 *)(x + p * C + c) = u16x8{};
 }
 
+// the network's three outputs per pixel, of `stride` stored ones, as dense
+// triples for the host (a strided copy of them is one 12-byte transfer a pixel:
+// 930 ms for 256 x 512 pixels, against 0.2 ms for one dense copy)
+__global__ void k_dense_output(const float *__restrict__ out, float *__restrict__ dense, long long P, int stride) {
+    const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= P) return;
+    const float4 v = *(const float4 *)(out + p * stride);
+    dense[3 * p] = v.x;
+    dense[3 * p + 1] = v.y;
+    dense[3 * p + 2] = v.z;
+}
+
 // Adam (Kingma and Ba 2015) on f32 master weights; refreshes the bf16 copy
 __global__ void k_adam(float *__restrict__ w, float *__restrict__ m, float *__restrict__ v,
                        const float *__restrict__ g, uint16_t *__restrict__ wb, size_t n, float lr, float b1, float b2,
@@ -1604,7 +1616,11 @@ int lbm_unet_forward(lbm_unet *n, const float *x, float *y) {
         HIPCHK(hipMemcpyAsync(n->fields, x, P * 32, hipMemcpyHostToDevice, n->stream));
         hipLaunchKernelGGL(k_pack_input, dim3(nblk(P)), dim3(256), 0, n->stream, n->fields, n->x.a, (long long)P, 32);
         n->forward();
-        HIPCHK(hipMemcpy2DAsync(y, 12, n->out32, 128, 12, P, hipMemcpyDeviceToHost, n->stream));
+        // through the host fields' buffer, which the pass has read
+        hipLaunchKernelGGL(k_dense_output, dim3(nblk(P)), dim3(256), 0, n->stream, n->out32, n->fields, (long long)P,
+                           32);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipMemcpyAsync(y, n->fields, P * 12, hipMemcpyDeviceToHost, n->stream));
         HIPCHK(hipStreamSynchronize(n->stream));
     });
 }
