@@ -10,9 +10,9 @@ before the timed region; K steps run between two stream synchronisations.
 
 Printed: ONE JSON line with the FP32 MLUPS as `value`, the roofline of the
 fused step kernel (72 algorithmic bytes per cell update times the updates one
-launch makes -- two for the two-step variants, which read and write the state
-once per pair of steps -- over the average launch duration of that kernel
-from HIP events recorded on the grid's own stream; `frac_hbm` the same with
+launch makes -- six in f32 and five in binary16 for the tile variants, which
+read and write the state once per launch -- over the average launch duration of
+that kernel from HIP events recorded on the grid's own stream; `frac_hbm` the same with
 the launch's measured HBM bytes, calibrated FETCH_SIZE + WRITE_SIZE), the same
 for FP16-shifted storage (36 B per cell update; f - w, and centred on the
 free-stream equilibrium), both again at 4096 x 2048 and 16384 x 8192
@@ -53,19 +53,21 @@ def read_traffic(name):
     return float(m.group(1)) if m else None
 
 
-KERNEL_NAMES = {1: "k_cell (one step per launch)",
-                2: "k_pair (two steps per launch: the state read and written once per pair of steps; its last "
-                   "blocks step the cells that read only themselves)"}
+def kernel_name(steps_per_launch):
+    if steps_per_launch == 1:
+        return "k_cell (one step per launch)"
+    return f"k_tile ({steps_per_launch} steps per launch: the state read and written once per launch)"
 
 
-def updates_per_launch(variant):
+def updates_per_launch(variant, f32=True):
     """Cell updates per cell in one launch of the step kernel: variants 8 and 9
-    run two steps per launch (the state is read and written once per pair)."""
-    return 2 if variant is not None and variant >= 8 else 1
+    (k_tile) run the number of steps a launch that costs least, at the sizes
+    timed here six in f32 and five in binary16."""
+    return (6 if f32 else 5) if variant is not None and variant >= 8 else 1
 
 
 def run_gpu(precision, X, Y, mask, steps, warmup, omega, u_in, variant=None):
-    from lbm_amd import LBM, LbmError
+    from lbm_amd import LBM, PRECISION_F32, LbmError
     g = LBM(omega, X, Y, precision=precision)
     g.mask = mask
     g.custom_speed(u_in)
@@ -87,21 +89,17 @@ def run_gpu(precision, X, Y, mask, steps, warmup, omega, u_in, variant=None):
     except LbmError as e:  # the flow left BGK's stable range: timing stands, sums do not
         log(f"conservation: {e}")
         cons = None
-    tuned["kernel_us"] = launch_us(g, tuned["variant"])
+    tuned["kernel_us"] = launch_us(g, updates_per_launch(tuned["variant"], precision == PRECISION_F32))
     g.close()
     return wall, dev_ms, cons, tuned
 
 
-def launch_us(g, variant, launches=40):
+def launch_us(g, steps_per_launch, launches=40):
     """Average duration of one launch of the step kernel, from HIP events on the
-    grid's stream.  A call of n steps with a two-step variant ends with one-step
-    launches, so the two-step launch is timed as the difference of a call of
-    2 + 2m steps and one of 2 steps (m two-step launches)."""
-    if updates_per_launch(variant) == 2:
-        g.step_timed(2)
-        short = min(g.step_timed(2) for _ in range(3))
-        return round((g.step_timed(2 + 2 * launches) - short) / launches * 1e3, 2)
-    return round(g.step_timed(launches) / launches * 1e3, 2)
+    grid's stream, over a call of `launches` launches (the last of them also
+    writes the other set and the moments)."""
+    g.step_timed(2)
+    return round(g.step_timed(launches * steps_per_launch) / launches * 1e3, 2)
 
 
 SURROGATE_WEIGHTS = os.path.join(ROOT, "lbm_amd", "data", "surrogate_f2.npy")
@@ -217,7 +215,7 @@ def grid_leg(X, Y, steps):
         k = dev_ms / 1e3 / steps
         out[name] = {"mlups": round(X * Y / k / 1e6, 1), "us_per_step": round(k * 1e6, 2),
                      "achieved_gbs": round(bpc * X * Y / k / 1e9, 1), "variant": tuned["variant"],
-                     "steps_per_launch": updates_per_launch(tuned["variant"]), "steps": steps,
+                     "steps_per_launch": updates_per_launch(tuned["variant"], prec == PRECISION_F32), "steps": steps,
                      "state_finite": cons is not None}
     out["f16s_speedup_vs_f32"] = round(out["f16s"]["mlups"] / out["f32"]["mlups"], 3)
     return out
@@ -361,7 +359,7 @@ def main():
         f"{achieved:.0f} GB/s algorithmic")
     traffic = None
     if (X, Y) == (8192, 4096):
-        traffic = read_traffic("traffic_f32_pair_8192x4096.txt" if upl == 2 else "traffic_f32_8192x4096.txt")
+        traffic = read_traffic("traffic_f32_tile_8192x4096.txt" if upl > 1 else "traffic_f32_8192x4096.txt")
 
     out = {
         "metric": METRIC,
@@ -389,7 +387,7 @@ def main():
             "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": traffic,
-            "kernel": KERNEL_NAMES[upl],
+            "kernel": kernel_name(upl),
             "algorithmic_bytes_per_launch": 72 * cells * upl,
             "cell_updates_per_launch": cells * upl,
             "kernel_avg_us": tuned["kernel_us"],
@@ -406,18 +404,18 @@ def main():
         w16, d16, c16, tuned16 = run_gpu(PRECISION_F16S, X, Y, mask, args.steps, args.warmup, omega,
                                         u_in, args.f16_variant)
         m16 = cells * args.steps / w16 / 1e6
-        u16 = updates_per_launch(tuned16["variant"])
+        u16 = updates_per_launch(tuned16["variant"], False)
         k16 = tuned16["kernel_us"] / 1e6 / u16
         a16 = 36.0 * cells / k16 / 1e9
         log(f"f16s: {m16:.0f} MLUPS, {k16 * 1e6:.1f} us per step, {u16} step(s) per launch, "
             f"{a16:.0f} GB/s algorithmic")
-        t16 = (read_traffic("traffic_f16s_8192x4096.txt" if u16 == 1 else "traffic_f16s_pair_8192x4096.txt")
+        t16 = (read_traffic("traffic_f16s_8192x4096.txt" if u16 == 1 else "traffic_f16s_tile_8192x4096.txt")
                if (X, Y) == (8192, 4096) else None)
         out["f16s"] = {
             "mlups": round(m16, 1),
             "speedup_vs_f32": round(m16 / mlups, 3),
             "roofline": {"bound": "hbm", "achieved": round(a16, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                         "frac": round(a16 / HBM_PEAK_GBS, 4), "kernel": KERNEL_NAMES[u16],
+                         "frac": round(a16 / HBM_PEAK_GBS, 4), "kernel": kernel_name(u16),
                          "algorithmic_bytes_per_launch": 36 * cells * u16,
                          "cell_updates_per_launch": cells * u16, "kernel_avg_us": tuned16["kernel_us"],
                          "traffic": t16,

@@ -145,16 +145,20 @@ int lbm_step(lbm_grid *g, uint32_t n);
 int lbm_sync(lbm_grid *g);
 
 /* Step-kernel variants (no reference counterpart): how the fused step moves
- * memory -- cells per thread, non-temporal access, block order, or (8, 9) two
- * steps per launch through LDS, which reads and writes the state once per two
- * steps (row blocks of 8 or 16).  All variants compute the same bits.  The two-step variants need two
+ * memory -- cells per thread, non-temporal access, block order, or (8, 9)
+ * several steps per launch with each block's cells in registers, which reads
+ * and writes the state once per launch (8: one row a wave; 9: two or three).
+ * All variants compute the same bits.  The variants of several steps need two
  * more state sets: lbm_set_variant allocates them when it selects one (and
  * fails, changing nothing, when it cannot) and frees them when it selects
- * another.  lbm_autotune times each variant for `steps` steps on the grid's
+ * another.  A grid for which no variant was ever set or tuned (lbm_get_variant:
+ * 0) runs several steps per launch too where two more sets take at most 512
+ * MiB; they are allocated with the grid, if there is memory for them.
+ * lbm_autotune times each variant for `steps` steps on the grid's
  * own state, restores that state exactly, selects the fastest, and returns it
  * in *best and the per-step time of every variant in ms[LBM_NUM_VARIANTS]
- * (either pointer may be NULL; +inf for a two-step variant whose sets could
- * not be allocated). */
+ * (either pointer may be NULL; +inf for a variant of several steps whose sets
+ * could not be allocated, or with steps < 3). */
 #define LBM_NUM_VARIANTS 10
 int lbm_set_variant(lbm_grid *g, int variant);
 int lbm_get_variant(const lbm_grid *g, int *variant);
@@ -165,8 +169,7 @@ int lbm_autotune(lbm_grid *g, uint32_t steps, int *best, float *ms);
  * variant that was fastest.  A key found in the file selects its variant
  * without timing (*hit = 1); otherwise the call tunes as lbm_autotune and
  * adds the key (*hit = 0), rewriting the file through a temporary file and a
- * rename.  A cached two-step variant that cannot get its spare sets counts as
- * a miss.  LBM_EINVAL when the file cannot be written (the tuned variant is
+ * rename.  A cached variant that cannot get its spare sets counts as a miss.  LBM_EINVAL when the file cannot be written (the tuned variant is
  * selected all the same).  best and hit may be NULL. */
 int lbm_autotune_cached(lbm_grid *g, const char *cache_path, uint32_t steps, int *best, int *hit);
 /* lbm_step(g, n) bracketed by two hipEvents recorded on the grid's stream;

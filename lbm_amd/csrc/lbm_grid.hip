@@ -19,9 +19,9 @@
 //   fused   (P -> P)   S_n := pull(buf[cur]) on streamed cells, buf[1-cur] own
 //                      values elsewhere; buf[1-cur] := collide(S_n); swap.
 //   flush   (P -> S)   buf[1-cur] := S_n (streamed cells only); swap.
-//   pair    (P -> P -> P, variants 8 and 9) two fused steps in one pass, the
-//                      first one's result staged in LDS (k_pair below); its
-//                      last blocks step the cells that read only themselves.
+//   tile    (-> P, by default on all but large grids; variants 8 and 9)
+//                      several steps in one launch, each block's cells held in
+//                      registers (k_tile below, tile.h).
 // Since the pull of step n uses the mask at the time the kernel runs, any mask
 // change first flushes a pending stream, so results are those of the reference
 // step order exactly.  The rest population is stored in both sets (the
@@ -50,7 +50,7 @@
 
 #include "lbm_common.h"
 #include "tune_cache.h"
-#include "pair.h"
+#include "tile.h"
 
 namespace {
 
@@ -77,44 +77,20 @@ __global__ __launch_bounds__(kBlock) void k_cell(const typename St::T *src, type
     if (OP & OP_REDUCE) block_sums(s0, s1, s2, partials, blockIdx.x);
 }
 
-// ---- two steps per launch -------------------------------------------------------
-// (the per-block work is pair_block / fixed_cell in pair.h)
+// ---- several steps per launch (the per-block work is tile_block in tile.h) ----------
 
-// the fixed-cell list: kSlowCell cells per row (one block per row), then the
-// (column, row) entries at each row's offset
-__global__ __launch_bounds__(kFixedBlock) void k_fixed_count(const uint8_t *__restrict__ flags, Geom g,
-                                                             uint32_t *__restrict__ counts) {
-    fixed_row_count(flags + (size_t)blockIdx.x * g.pitch, g.X, counts + blockIdx.x);
-}
-
-__global__ __launch_bounds__(kFixedBlock) void k_fixed_emit(const uint8_t *__restrict__ flags,
-                                                            const uint8_t *__restrict__ mask, Geom g,
-                                                            const uint32_t *__restrict__ offsets,
-                                                            uint2 *__restrict__ list) {
-    const size_t r = (size_t)blockIdx.x * g.pitch;
-    fixed_row_emit(flags + r, mask + r, g.X, (int)blockIdx.x, g.Y, blockIdx.x, list + offsets[blockIdx.x]);
-}
-
-template <class St, int MODE>
-__global__ __launch_bounds__(kBlock) void k_pair(const typename St::T *A, const typename St::T *B,
-                                                 typename St::T *__restrict__ A2, typename St::T *__restrict__ B2,
-                                                 const uint8_t *__restrict__ flags, Geom g, int nstrips, int rows,
-                                                 int nblocks, int remap, const uint2 *__restrict__ fixed,
-                                                 uint32_t n_fixed) {
-    __shared__ typename St::T ring[kRing][8][kBlock];
-    if ((int)blockIdx.x >= nblocks) {
-        // the fixed-cell pass: one thread per list entry (column | streamed << 31, row)
-        const uint32_t i = (blockIdx.x - nblocks) * kBlock + threadIdx.x;
-        if (i < n_fixed) {
-            const uint2 e = fixed[i];
-            fixed_cell<St>(A, B, g, (int)(e.x & 0x7FFFFFFFu), (int)e.y, (e.x >> 31) != 0, A2, B2);
-        }
-        return;
-    }
-    const int L = remap ? xcd_remap(blockIdx.x, nblocks) : (int)blockIdx.x;
-    const int chunk = L / nstrips;
-    const int r0 = chunk * rows;
-    pair_block_any<St, MODE>(ring, A, B, A2, B2, flags, g, L - chunk * nstrips, r0, min(r0 + rows, g.Y));
+// Two blocks of 16 waves share a CU with up to 64 registers a lane, two of 12
+// waves with up to 80.
+template <class St, int MODE, int SHAPE>
+__global__ __launch_bounds__(64 * tile_shape<typename St::T>(SHAPE).waves,
+                             tile_shape<typename St::T>(SHAPE).waves / 2) void
+k_tile(const typename St::T *A, const typename St::T *B, typename St::T *__restrict__ A2,
+       typename St::T *__restrict__ B2, const uint8_t *__restrict__ flags, const uint8_t *__restrict__ mask, Geom g,
+       TileArgs a, float *__restrict__ mom) {
+    extern __shared__ uint32_t ex[];
+    const int L = xcd_remap(blockIdx.x, a.nbx * a.nby);
+    const int by = L / a.nbx;
+    tile_block<St, MODE, SHAPE>(ex, A, B, A2, B2, flags, mask, g, a, L - by * a.nbx, by, mom);
 }
 
 // ---- surrogate support ---------------------------------------------------------
@@ -286,11 +262,7 @@ struct lbm_grid {
         geom.sh = make_f16_shift(precision == LBM_PRECISION_F16E, u);
     }
     void *f[2] = {nullptr, nullptr};
-    void *spare[2] = {nullptr, nullptr};  // output sets of the two-step kernel, allocated on first use
-    uint2 *fixed = nullptr;               // its fixed-cell list: (column | streamed << 31, row) per kSlowCell cell
-    uint32_t *fixed_rows = nullptr;       // the list's offset per row
-    uint32_t n_fixed = 0;
-    bool fixed_dirty = true;              // the list does not follow the flags (a rebuild failed)
+    void *spare[2] = {nullptr, nullptr};  // output sets of k_tile: with a tile variant, or by default (see auto_path)
     int cur = 0;
     bool pform = false;
     uint8_t *mask = nullptr, *flags = nullptr;
@@ -306,6 +278,7 @@ struct lbm_grid {
     size_t npartials = 0;
     uint64_t steps = 0;
     int variant = 0;  // step-kernel variant (cells per thread, non-temporal access)
+    bool auto_path = true;  // no variant was ever set or tuned: steps go through k_tile where `spare` is there
     std::string err;
     // device snapshot of the evolving state (both sets, fields, form, step count)
     char *snap = nullptr;
@@ -327,8 +300,8 @@ struct lbm_grid {
     size_t nvpart = 0;
 
     size_t set_bytes() const { return (size_t)geom.ys * Y * esize; }
-    // a set's allocation: two rows more, which the two-step kernel's loads of
-    // the last rows (wrapped outlet pulls, the relay lanes) read and discard
+    // a set's allocation: two rows more, which k_tile's wrapped outlet pulls of
+    // the last rows read and discard
     size_t alloc_bytes() const { return set_bytes() + 2 * (size_t)geom.ys * esize; }
     struct Shape {
         int blocks_per_row, nblocks;
@@ -341,8 +314,8 @@ struct lbm_grid {
 
     void release() {
         (void)hipSetDevice(dev);
-        for (void *p : {f[0], f[1], spare[0], spare[1], (void *)fixed, (void *)fixed_rows, (void *)mask, (void *)flags,
-                        (void *)lag, (void *)now, (void *)out, (void *)dense, (void *)partials, (void *)sums,
+        for (void *p : {f[0], f[1], spare[0], spare[1], (void *)mask, (void *)flags, (void *)lag,
+                        (void *)now, (void *)out, (void *)dense, (void *)partials, (void *)sums,
                         (void *)snap, (void *)umark, (void *)vpart})
             if (p) (void)hipFree(p);
         snap = nullptr;
@@ -350,8 +323,6 @@ struct lbm_grid {
         vpart = nullptr;
         f[0] = f[1] = nullptr;
         spare[0] = spare[1] = nullptr;
-        fixed = nullptr;
-        fixed_rows = nullptr;
         mask = flags = nullptr;
         lag = now = out = dense = nullptr;
         partials = sums = nullptr;
@@ -385,7 +356,7 @@ struct lbm_grid {
     //   cells    1 1 1 2 2 4 4 4      cells    1 1 1 2 2 4 4 8
     //   nt       1 1 0 1 1 1 1 0      nt       1 1 0 1 1 1 1 1
     //   remap    1 0 0 1 0 1 0 0      remap    1 0 0 1 0 1 0 0
-    // and 8, 9: two steps per launch (k_pair, see pair()).
+    // and 8, 9: several steps per launch (k_tile, shapes 0 and 1; see tile()).
     template <class St, int MODE, bool PFORM, int OP>
     void launch_cell(const void *src, void *dst, float *mom, double *part) {
         constexpr bool f32 = sizeof(typename St::T) == 4;
@@ -402,7 +373,7 @@ struct lbm_grid {
             case 7:
                 if constexpr (f32) return go<St, MODE, PFORM, OP, 4, false>(src, dst, mom, part, 0);
                 else return go<St, MODE, PFORM, OP, 8, true>(src, dst, mom, part, 0);
-            default:  // single steps of the two-step variants: variant 0 (f32) / 4 (f16s)
+            default:  // single steps of the tile variants: variant 0 (f32) / 4 (f16s)
                 if constexpr (f32) return go<St, MODE, PFORM, OP, 1, true>(src, dst, mom, part, 1);
                 else return go<St, MODE, PFORM, OP, 2, true>(src, dst, mom, part, 0);
             }
@@ -410,100 +381,81 @@ struct lbm_grid {
         go<St, MODE, PFORM, OP, (PFORM && !f32 ? 2 : 1), true>(src, dst, mom, part, 0);
     }
 
-    // Variants 8, 9: two P-form steps per launch (k_pair), blocks of 8 or 16 rows
-    // (measured at 8192 x 4096: 2 / 4 / 8 / 16 / 32 rows 362 / 312 / 303 / 314 /
-    // 333 us per step).  Two cells per thread (pairs through the ring, 510-column
-    // strips) measured slower: f32 408 vs 297 us per step (64 KB of ring, 2 waves
-    // per SIMD), binary16 303 vs 255 us.
-    static constexpr int kPairFirst = 8;
-    static bool pair_variant(int v) { return v >= kPairFirst; }
-    int pair_rows() const { return 8 << (variant - kPairFirst); }
+    // Variants 8, 9: several steps per launch, with k_tile's shape 0 or 1.
+    static constexpr int kTileFirst = 8;
+    static bool tile_variant(int v) { return v >= kTileFirst; }
+    // A grid nobody has chosen a variant for has k_tile's two output sets from
+    // the start if they take at most this (7 million cells in f32): there a step
+    // gains most (400 x 160: 3.7 -> 1.6 us; 2048 x 1024: 28 -> 13 us), and
+    // memory for two more sets is not taken unasked on a large grid.
+    static constexpr size_t kAutoSpareBytes = (size_t)512 << 20;
 
-    // the two-step kernel's output sets and fixed-cell list (room for every
-    // cell); allocated when a two-step variant is set, so that stepping itself
-    // does not allocate
-    void ensure_pair_buffers() {
-        if (spare[0] && spare[1] && fixed) return;
-        release_pair_buffers();
+    // two more sets (not in place of the default path's: those stay until the
+    // new ones are there)
+    void make_spare(void *out[2]) {
+        out[0] = out[1] = nullptr;
         try {
-            spare[0] = dalloc<char>(alloc_bytes());
-            spare[1] = dalloc<char>(alloc_bytes());
-            fixed = dalloc<uint2>((size_t)X * Y);
-            fixed_rows = dalloc<uint32_t>((size_t)Y);
-            // the rows' padding is never written by this kernel: keep it defined
-            HIPCHK(hipMemsetAsync(spare[0], 0, set_bytes(), stream));
-            HIPCHK(hipMemsetAsync(spare[1], 0, set_bytes(), stream));
-            build_fixed_list();
+            for (int i = 0; i < 2; ++i) {
+                out[i] = dalloc<char>(alloc_bytes());
+                // the rows' padding is never written by k_tile: keep it defined
+                HIPCHK(hipMemsetAsync(out[i], 0, set_bytes(), stream));
+            }
         } catch (...) {
-            release_pair_buffers();
+            for (int i = 0; i < 2; ++i)
+                if (out[i]) (void)hipFree(out[i]);
             throw;
         }
     }
-
-    // the fixed-cell list from the current flags (after every mask change
-    // while the two-step buffers exist); waits for the stream.  Until it has
-    // succeeded the list is dirty, and a two-step launch rebuilds it first.
-    void build_fixed_list() {
-        fixed_dirty = true;
-        hipLaunchKernelGGL(k_fixed_count, dim3(Y), dim3(kFixedBlock), 0, stream, flags, geom, fixed_rows);
-        HIPCHK(hipGetLastError());
-        std::vector<uint32_t> off(Y);
-        HIPCHK(hipMemcpyAsync(off.data(), fixed_rows, Y * sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
-        HIPCHK(hipStreamSynchronize(stream));
-        uint32_t total = 0;
-        for (uint32_t &o : off) {
-            const uint32_t c = o;
-            o = total;
-            total += c;
-        }
-        HIPCHK(hipMemcpyAsync(fixed_rows, off.data(), Y * sizeof(uint32_t), hipMemcpyHostToDevice, stream));
-        hipLaunchKernelGGL(k_fixed_emit, dim3(Y), dim3(kFixedBlock), 0, stream, flags, mask, geom, fixed_rows, fixed);
-        HIPCHK(hipGetLastError());
-        HIPCHK(hipStreamSynchronize(stream));  // `off` is read by the copy above
-        n_fixed = total;
-        fixed_dirty = false;
-    }
-
-    template <class St, int MODE>
-    void launch_pair() {
-        using T = typename St::T;
-        ensure_pair_buffers();
-        if (fixed_dirty) build_fixed_list();
-        const T *A = (const T *)f[cur], *B = (const T *)f[1 - cur];
-        T *A2 = (T *)spare[0], *B2 = (T *)spare[1];
-        const int rows = pair_rows();
-        const int nstrips = ((int)X + kBlock - 3) / (kBlock - 2);
-        const int nblocks = nstrips * (((int)Y + rows - 1) / rows);
-        const unsigned nfix = (n_fixed + kBlock - 1) / kBlock;
-        hipLaunchKernelGGL((k_pair<St, MODE>), dim3(nblocks + nfix), dim3(kBlock), 0, stream, A, B, A2, B2, flags,
-                           geom, nstrips, rows, nblocks, 1, fixed, n_fixed);
-        HIPCHK(hipGetLastError());
-        spare[0] = f[cur];
-        spare[1] = f[1 - cur];
-        f[cur] = A2;
-        f[1 - cur] = B2;
-    }
-
-    // the two-step kernel's output sets and fixed-cell list (the state itself
-    // is always in f[0], f[1] between calls)
-    void release_pair_buffers() {
+    void release_spare() {
         for (void *&p : spare) {
             if (p) (void)hipFree(p);
             p = nullptr;
         }
-        if (fixed) (void)hipFree(fixed);
-        if (fixed_rows) (void)hipFree(fixed_rows);
-        fixed = nullptr;
-        fixed_rows = nullptr;
-        n_fixed = 0;
+    }
+    // k_tile's sets for a tile variant (setting one does not take over the
+    // default path's: it succeeds exactly when two more sets can be allocated);
+    // the state itself is always in f[0], f[1] between calls
+    void ensure_spare(bool take_over = true) {
+        if (spare[0] && (take_over || !auto_path)) return;
+        void *fresh[2];
+        make_spare(fresh);
+        release_spare();
+        spare[0] = fresh[0];
+        spare[1] = fresh[1];
     }
 
-    // two P-form steps in one launch; the other set is then whole only on the
-    // cells the stream does not write
-    void pair() {
+    template <class St, int MODE, int SHAPE>
+    void launch_tile(int steps, bool final) {
+        using T = typename St::T;
+        constexpr TileShape sh = tile_shape<T>(SHAPE);
+        constexpr size_t lds = tile_lds(sh, sizeof(T));
+        const TileArgs a{steps, tile_nbx((int)X, steps), tile_nby((int)Y, sh.waves * sh.m, steps), pform ? 0 : 1, final};
+        tile_allow_lds<k_tile<St, MODE, SHAPE>>(lds, dev);
+        hipLaunchKernelGGL((k_tile<St, MODE, SHAPE>), dim3(a.nbx * a.nby), dim3(64 * sh.waves), lds, stream,
+                           (const T *)f[cur], (const T *)f[1 - cur], (T *)spare[0], (T *)spare[1], flags, mask, geom, a,
+                           lag);
+        HIPCHK(hipGetLastError());
+        // the sets' parity goes on as with single steps, of which every one but
+        // the collision of an S-form trades them
+        void *const a0 = f[cur], *const b0 = f[1 - cur];
+        cur = (cur + steps - (pform ? 0 : 1)) & 1;
+        f[cur] = spare[0];
+        f[1 - cur] = spare[1];
+        spare[0] = a0;
+        spare[1] = b0;
+        pform = true;
+    }
+
+    // `steps` steps in one launch; unless it is the call's last, the other set is
+    // then whole only on the cells the stream does not write
+    void tile(int shape, int steps, bool final) {
         by_store(precision, [&]<class St>() {
-            if (boundary == LBM_BOUNDARY_REFERENCE) launch_pair<St, LBM_BOUNDARY_REFERENCE>();
-            else launch_pair<St, LBM_BOUNDARY_ZERO_GRADIENT>();
+            auto mode = [&]<int SHAPE>() {
+                if (boundary == LBM_BOUNDARY_REFERENCE) launch_tile<St, LBM_BOUNDARY_REFERENCE, SHAPE>(steps, final);
+                else launch_tile<St, LBM_BOUNDARY_ZERO_GRADIENT, SHAPE>(steps, final);
+            };
+            if (shape == 0) mode.template operator()<0>();
+            else mode.template operator()<1>();
         });
     }
 
@@ -525,7 +477,6 @@ struct lbm_grid {
             hipLaunchKernelGGL(k_build_flags<LBM_BOUNDARY_ZERO_GRADIENT>, grid, dim3(256), 0, stream, mask, flags,
                                geom);
         HIPCHK(hipGetLastError());
-        if (fixed) build_fixed_list();
     }
 
     void fill_both(const float v[9]) {
@@ -567,18 +518,28 @@ struct lbm_grid {
         pform = false;
     }
 
+    // a call's launches of k_tile; none where it is not used
+    TilePlan plan_tile(uint32_t n) const {
+        if (n < 2 || !spare[0] || !(auto_path || tile_variant(variant)) || (uint64_t)geom.ys * esize >= 1ull << 31)
+            return {0, 0};
+        const bool any = !tile_variant(variant);
+        const int first = any ? 0 : variant - kTileFirst, last = any ? 1 : first;
+        return tile_plan(precision, first, last, n, pform, [&](int i, int s) {
+            const TileShape &sh = tile_shape(precision, i);
+            return (int64_t)tile_nbx((int)X, s) * tile_nby((int)Y, sh.waves * sh.m, s);
+        });
+    }
+
     void step(uint32_t n) {
+        if (const TilePlan plan = plan_tile(n); plan.launches) {
+            const uint32_t low = n / plan.launches, more = n % plan.launches;
+            for (uint32_t i = 0; i < plan.launches; ++i)
+                tile(plan.shape, (int)(low + (i < more)), i + 1 == plan.launches);
+            steps += n;
+            return;
+        }
         for (uint32_t i = 0; i < n; ++i) {
             const bool last = i + 1 == n;
-            if (pform && pair_variant(variant) && n - i >= 3) {
-                // after a two-step launch the other set is current only on the
-                // cells the stream does not write, the only ones the next step
-                // reads from it; the last step of a call is always a one-step
-                // launch, which writes that set whole (and the moments)
-                pair();
-                ++i;
-                continue;
-            }
             if (!pform) {
                 if (last)
                     cell<false, OP_COLLIDE | OP_MOMENTS>(f[cur], f[cur], lag, nullptr);
@@ -800,6 +761,12 @@ int lbm_create(const lbm_config *cfg, lbm_grid **out) {
         hipLaunchKernelGGL(k_walls, dim3((g->X + 255) / 256), dim3(256), 0, g->stream, g->mask, g->geom);
         HIPCHK(hipGetLastError());
         g->build_flags();
+        if (2 * g->alloc_bytes() <= lbm_grid::kAutoSpareBytes) {
+            try {
+                g->make_spare(g->spare);
+            } catch (const HipError &) {  // no memory for them: one step per launch
+            }
+        }
         HIPCHK(hipStreamSynchronize(g->stream));
     });
     if (rc != LBM_OK) {
@@ -1014,9 +981,10 @@ int lbm_set_variant(lbm_grid *g, int variant) {
     return guarded(g, [&] {
         check(variant >= 0 && variant < LBM_NUM_VARIANTS, "unknown kernel variant");
         HIPCHK(hipStreamSynchronize(g->stream));
-        if (g->pair_variant(variant)) g->ensure_pair_buffers();  // may fail: then nothing changes
-        else g->release_pair_buffers();
+        if (g->tile_variant(variant)) g->ensure_spare(false);  // may fail: then nothing changes
+        else g->release_spare();
         g->variant = variant;
+        g->auto_path = false;
     });
 }
 
@@ -1036,9 +1004,11 @@ int lbm_autotune(lbm_grid *g, uint32_t steps, int *best, float *ms) {
         const bool pform = g->pform;
         const uint64_t nsteps = g->steps;
         const int variant = g->variant;
+        const bool auto_path = g->auto_path, had_spare = g->spare[0] != nullptr;
         float t[LBM_NUM_VARIANTS];
         int v_best = 0;
         bool saved = false;
+        g->auto_path = false;  // time each variant's own kernel
         try {
             HIPCHK(hipMemcpyAsync(snap, g->f[0], sb, hipMemcpyDeviceToDevice, g->stream));
             HIPCHK(hipMemcpyAsync(snap + sb, g->f[1], sb, hipMemcpyDeviceToDevice, g->stream));
@@ -1048,15 +1018,14 @@ int lbm_autotune(lbm_grid *g, uint32_t steps, int *best, float *ms) {
             HIPCHK(hipEventCreate(&e0));
             HIPCHK(hipEventCreate(&e1));
             for (int v = 0; v < LBM_NUM_VARIANTS; ++v) {
-                if (g->pair_variant(v) && steps < 3) {
-                    // a call of fewer than three steps never launches the
-                    // two-step kernel: it would time the one-step fallback
+                if (g->tile_variant(v) && steps < 3) {
+                    // too few steps a call for what these variants are for
                     t[v] = INFINITY;
                     continue;
                 }
-                if (g->pair_variant(v)) {
+                if (g->tile_variant(v)) {
                     try {
-                        g->ensure_pair_buffers();
+                        g->ensure_spare();
                     } catch (...) {  // no memory for two more sets: not a candidate
                         t[v] = INFINITY;
                         continue;
@@ -1078,9 +1047,9 @@ int lbm_autotune(lbm_grid *g, uint32_t steps, int *best, float *ms) {
             HIPCHK(hipMemcpyAsync(g->lag, snap + 2 * sb, lb, hipMemcpyDeviceToDevice, g->stream));
             HIPCHK(hipStreamSynchronize(g->stream));
         } catch (...) {
-            // put the grid back as it was (the two-step kernel trades the
-            // state sets with its spare pair, so the state may live in any
-            // two of the four: the copies restore whichever two are current)
+            // put the grid back as it was (k_tile trades the state sets with
+            // the spare pair, so the state may live in any two of the four:
+            // the copies restore whichever two are current)
             (void)hipStreamSynchronize(g->stream);
             if (saved) {
                 (void)hipMemcpyAsync(g->f[0], snap, sb, hipMemcpyDeviceToDevice, g->stream);
@@ -1093,7 +1062,8 @@ int lbm_autotune(lbm_grid *g, uint32_t steps, int *best, float *ms) {
             g->pform = pform;
             g->steps = nsteps;
             g->variant = variant;
-            if (!g->pair_variant(variant)) g->release_pair_buffers();
+            g->auto_path = auto_path;
+            if (!had_spare) g->release_spare();
             throw;
         }
         (void)hipFree(snap);
@@ -1101,7 +1071,7 @@ int lbm_autotune(lbm_grid *g, uint32_t steps, int *best, float *ms) {
         g->pform = pform;
         g->steps = nsteps;
         g->variant = v_best;
-        if (!g->pair_variant(v_best)) g->release_pair_buffers();  // tried, not kept
+        if (!g->tile_variant(v_best)) g->release_spare();  // tried, not kept
         if (best) *best = v_best;
         if (ms)
             for (int v = 0; v < LBM_NUM_VARIANTS; ++v) ms[v] = t[v] / steps;
@@ -1124,7 +1094,7 @@ int lbm_autotune_cached(lbm_grid *g, const char *cache_path, uint32_t steps, int
     });
     if (rc != LBM_OK) return rc;
     if (hit) *hit = 0;
-    // a cached two-step variant whose spare sets cannot be allocated here is a miss
+    // a cached variant whose spare sets cannot be allocated here is a miss
     if (found && lbm_set_variant(g, e.variant) == LBM_OK) {
         if (hit) *hit = 1;
         if (best) *best = e.variant;
