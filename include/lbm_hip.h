@@ -273,12 +273,14 @@ int lbm_batch_info(lbm_batch *b, uint64_t *cells, uint32_t *interior_tiles, uint
 /* hipGraph replay on (default) or off */
 int lbm_batch_set_graph(lbm_batch *b, int enable);
 /* Batch variants: 0..5 the interior kernel's tile (cells per thread 1, 2, 4
- * -- 2, 4, 8 for binary16 -- each in list order or chunked); 6, 7 two steps
- * per launch for every domain (row chunks of 8 / 16), which needs two more
- * state sets: lbm_batch_set_variant allocates them (and fails, changing
- * nothing, when it cannot) and frees them when another variant is selected.
- * All variants give the same bits.  lbm_batch_autotune as lbm_autotune (+inf
- * for a two-step variant without memory or with steps < 3). */
+ * -- twice that for binary16 -- in two list orders), 6 and 7 several steps per
+ * launch (one row a wave; two or three), which need two more state sets:
+ * lbm_batch_set_variant allocates them (and fails, changing nothing, when it
+ * cannot) and frees them when another variant is selected.  A batch for which
+ * no variant was ever set or tuned (lbm_batch_get_variant: 0) runs several
+ * steps per launch too where two more sets take at most 512 MiB.  All variants
+ * give the same bits.  lbm_batch_autotune as lbm_autotune (+inf for a variant
+ * of several steps without memory or with steps < 3). */
 int lbm_batch_set_variant(lbm_batch *b, int variant);
 int lbm_batch_get_variant(const lbm_batch *b, int *variant);
 int lbm_batch_autotune(lbm_batch *b, uint32_t steps, int *best, float *ms);

@@ -284,7 +284,8 @@ struct StoreF16E : StoreF16S {
     // population k's working value from a stored value of population opp(k) when
     // `bounced` (half-way bounce-back hands a cell its own opposite population)
     __device__ __forceinline__ static float load_b(T v, int k, bool bounced, const F16Shift &sh) {
-        return StoreF16S::load(v, k, sh) + (bounced ? sh.d[opp(k)] : sh.d[k]);
+        const float own = sh.d[opp(k)], pulled = sh.d[k];
+        return StoreF16S::load(v, k, sh) + (bounced ? own : pulled);
     }
     __device__ __forceinline__ static T store(float g, int k, const F16Shift &sh) {
         return StoreF16S::store(g - sh.d[k], k, sh);

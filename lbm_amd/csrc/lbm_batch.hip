@@ -1,13 +1,14 @@
 // Batched engine: many independent D2Q9 domains of uneven size and obstacle
-// layout stepped together, one launch pair (interior + boundary) per step for
-// all domains, replayed from a hipGraph.
+// layout stepped together, by default and with the tile variants several steps
+// of all domains per launch (k_batch_tile), otherwise two launches (interior +
+// boundary) per step for all domains, replayed from a hipGraph.
 //
 // Each domain follows exactly the single-grid semantics (the reference step,
 // lbm-wgpu src/lbm.rs:1112-1134, with the S-form / P-form state machine of
 // lbm_grid.hip) and uses the same device code (lbm_common.h), so a domain of a
 // batch equals a single grid of the same size bit for bit.
 //
-// Work decomposition.  Every domain is cut into rows of 64-cell segments.  A
+// Work decomposition of the single steps.  Every domain is cut into rows of 64-cell segments.  A
 // tile is the span of one wave (64 * CPT cells of one row); a tile whose
 // segments are all clear (streamed, no bounce-back, before the outlet column)
 // goes to the interior list, every segment of any other tile to the boundary
@@ -31,7 +32,7 @@
 
 #include "lbm_common.h"
 #include "tune_cache.h"
-#include "pair.h"
+#include "tile.h"
 
 namespace {
 
@@ -103,61 +104,45 @@ __global__ __launch_bounds__(kBlock) void k_batch_boundary(const typename St::T 
     if (OP & OP_REDUCE) block_sums(s0, s1, s2, partials, blockIdx.x);
 }
 
-// Two steps per launch for every domain (the single grid's two-step scheme,
-// pair.h): one block per work item (domain, 254-column strip, row chunk) of
-// the pair list, blocks of one XCD on one contiguous run of it, then the
-// fixed-cell pass's blocks.  A, B: the current sets; A2, B2: the spare sets
-// that receive C_{n+2} and C_{n+1}.
-template <class St, int MODE>
-__global__ __launch_bounds__(kBlock) void k_batch_pair(const typename St::T *A, const typename St::T *B,
-                                                       typename St::T *__restrict__ A2, typename St::T *__restrict__ B2,
-                                                       const uint8_t *__restrict__ flags,
-                                                       const DomainDev *__restrict__ table,
-                                                       const uint2 *__restrict__ list, int n_items, int rows,
-                                                       const uint2 *__restrict__ fixed,
-                                                       const uint2 *__restrict__ rowtab, uint32_t n_fixed) {
-    __shared__ typename St::T ring[kRing][8][kBlock];
-    if ((int)blockIdx.x >= n_items) {
-        // the fixed-cell pass: one thread per list entry (column | streamed << 31, row-table index)
-        const uint32_t i = (blockIdx.x - n_items) * kBlock + threadIdx.x;
-        if (i < n_fixed) {
-            const uint2 f = fixed[i];
-            const uint2 r = rowtab[f.y];
-            const DomainDev d = table[r.x];
-            fixed_cell<St>(A + d.f_off, B + d.f_off, d.g, (int)(f.x & 0x7FFFFFFFu), (int)r.y, (f.x >> 31) != 0,
-                           A2 + d.f_off, B2 + d.f_off);
-        }
-        return;
+// the bounce-back bytes of every domain: blockIdx.y the domain, the blocks
+// across covering the largest one's cells
+template <int MODE>
+__global__ __launch_bounds__(kBlock) void k_batch_flags(const uint8_t *__restrict__ mask, uint8_t *__restrict__ flags,
+                                                        const DomainDev *__restrict__ table) {
+    const DomainDev d = table[blockIdx.y];
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x, y = i / (uint32_t)d.g.pitch, x = i - y * (uint32_t)d.g.pitch;
+    if (y >= (uint32_t)d.g.Y || x >= (uint32_t)d.g.X) return;
+    flags[d.aux_off + i] = flag_byte<MODE>(mask + d.aux_off, d.g, (int)x, (int)y);
+}
+
+// Several steps per launch for every domain (the per-block work is tile_block
+// in tile.h).  A block finds its domain from the domains' running block counts
+// (`start`, n + 1 of them): each lane compares one count in 64, all at once, so
+// that the search costs one load's latency up to 64 domains and a list of
+// blocks for each number of steps (16 MB for 512 domains) is not needed.
+template <class St, int MODE, int SHAPE>
+__global__ __launch_bounds__(64 * tile_shape<typename St::T>(SHAPE).waves,
+                             tile_shape<typename St::T>(SHAPE).waves / 2) void
+k_batch_tile(const typename St::T *A, const typename St::T *B, typename St::T *__restrict__ A2,
+             typename St::T *__restrict__ B2, const uint8_t *__restrict__ flags, const uint8_t *__restrict__ mask,
+             const DomainDev *__restrict__ table, const uint32_t *__restrict__ start, int n, int steps, int sform,
+             int final, float *__restrict__ mom) {
+    extern __shared__ uint32_t ex[];
+    constexpr int rows = tile_shape<typename St::T>(SHAPE).waves * tile_shape<typename St::T>(SHAPE).m;
+    const uint32_t L = (uint32_t)xcd_remap(blockIdx.x, gridDim.x);
+    int dom = -1;  // domains that start at or before block L, less one
+    for (int i = 0; i < n; i += 64) {
+        const int j = i + ((int)threadIdx.x & 63);
+        dom += __popcll(__ballot(j < n && start[j] <= L));
     }
-    const uint2 e = list[xcd_remap((int)blockIdx.x, n_items)];
-    const DomainDev d = table[e.x];
-    const int strip = (int)(e.y >> 16), r0 = (int)(e.y & 0xFFFFu) * rows;
-    pair_block_any<St, MODE>(ring, A + d.f_off, B + d.f_off, A2 + d.f_off, B2 + d.f_off, flags + d.aux_off, d.g,
-                             strip, r0, min(r0 + rows, d.g.Y));
-}
-
-// the fixed-cell list of every domain (pair.h): one block per entry
-// (domain, row) of the row table; entries (column | streamed << 31,
-// row-table index)
-__global__ __launch_bounds__(kFixedBlock) void k_batch_fixed_count(const uint8_t *__restrict__ flags,
-                                                                   const DomainDev *__restrict__ table,
-                                                                   const uint2 *__restrict__ rowtab,
-                                                                   uint32_t *__restrict__ counts) {
-    const uint2 e = rowtab[blockIdx.x];
-    const DomainDev d = table[e.x];
-    fixed_row_count(flags + d.aux_off + (size_t)e.y * d.g.pitch, d.g.X, counts + blockIdx.x);
-}
-
-__global__ __launch_bounds__(kFixedBlock) void k_batch_fixed_emit(const uint8_t *__restrict__ flags,
-                                                                  const uint8_t *__restrict__ mask,
-                                                                  const DomainDev *__restrict__ table,
-                                                                  const uint2 *__restrict__ rowtab,
-                                                                  const uint32_t *__restrict__ offsets,
-                                                                  uint2 *__restrict__ list) {
-    const uint2 e = rowtab[blockIdx.x];
-    const DomainDev d = table[e.x];
-    const size_t r = d.aux_off + (size_t)e.y * d.g.pitch;
-    fixed_row_emit(flags + r, mask + r, d.g.X, (int)e.y, d.g.Y, blockIdx.x, list + offsets[blockIdx.x]);
+    dom = __builtin_amdgcn_readfirstlane(dom);
+    const long long f = table[dom].f_off, aux = table[dom].aux_off;
+    Geom g = table[dom].g;
+    if constexpr (!St::shifted) g.sh = F16Shift{};
+    const TileArgs a{steps, tile_nbx(g.X, steps), tile_nby(g.Y, rows, steps), sform, final};
+    const int local = (int)(L - start[dom]), by = local / a.nbx;
+    tile_block<St, MODE, SHAPE>(ex, A + f, B + f, A2 + f, B2 + f, flags + aux, mask + aux, g, a, local - by * a.nbx, by,
+                                mom + 3 * aux);
 }
 
 thread_local std::string g_batch_create_error;
@@ -180,16 +165,14 @@ struct lbm_batch {
     DomainDev *dtable = nullptr;
     uint2 *ilist = nullptr, *blist = nullptr, *alist = nullptr;
     uint32_t n_interior = 0, n_boundary = 0, n_all = 0;
-    // two-step variants: the output sets and the (domain, strip, row chunk)
-    // work list for `plist_rows`-row chunks
-    void *spare[2] = {nullptr, nullptr};
-    uint2 *plist = nullptr;
-    uint32_t n_pair = 0;
-    uint2 *fixed = nullptr, *rowtab = nullptr;  // fixed-cell list (column | streamed << 31, row-table index); (domain, row)
-    uint32_t *fixed_rows = nullptr;             // the list's offset per row-table entry
-    uint32_t n_fixed = 0, n_rows = 0;
-    bool fixed_dirty = true;
-    int plist_rows = 0;
+    void *spare[2] = {nullptr, nullptr};  // output sets of k_batch_tile: with a tile variant, or by default
+    bool auto_path = true;                // no variant was ever set or tuned
+    // running block counts of the domains for each shape and number of steps
+    // (n + 1 a combination, the last one the launch's blocks)
+    uint32_t *starts = nullptr;
+    std::vector<uint32_t> tile_blocks;  // the launch's blocks by combination
+    uint32_t max_cells = 0;             // pitch * ny of the largest domain
+    bool flags_dirty = true;            // masks changed since the bounce-back bytes were built
     int list_cpt = 0;  // tile width (cells per thread) the interior list was built for
     bool dirty = true;  // masks changed since the lists were built
     int cur = 0;
@@ -197,31 +180,27 @@ struct lbm_batch {
     uint64_t steps = 0;
     int variant = 0;
     bool use_graph = true;
-    // fused steps starting from cur = 0 / 1 and, for the two-step variants, from
-    // either arrangement of the state and spare sets (each two-step launch
-    // trades them; a graph holds the pointers it was captured with)
-    hipGraphExec_t graph[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
-    int pair_parity = 0;  // flips with every two-step launch
+    hipGraphExec_t graph[2] = {nullptr, nullptr};  // two one-step launches from cur = 0 / 1
+    void *graph_sets[2] = {nullptr, nullptr};  // the state sets it was captured with
     int graph_variant = -1;
     int grid_blocks = 1024;
     std::string err;
     uint64_t cells = 0;
 
     void drop_graphs() {
-        for (auto &row : graph)
-            for (auto &gx : row)
-                if (gx) {
-                    (void)hipGraphExecDestroy(gx);
-                    gx = nullptr;
-                }
+        for (auto &gx : graph)
+            if (gx) {
+                (void)hipGraphExecDestroy(gx);
+                gx = nullptr;
+            }
         graph_variant = -1;
     }
 
     void release() {
         (void)hipSetDevice(dev);
         drop_graphs();
-        release_pair_buffers();
-        for (void *p : {f[0], f[1], (void *)mask, (void *)flags, (void *)segs, (void *)lag, (void *)dense,
+        release_spare();
+        for (void *p : {f[0], f[1], (void *)starts, (void *)mask, (void *)flags, (void *)segs, (void *)lag, (void *)dense,
                         (void *)dtable, (void *)ilist, (void *)blist, (void *)alist})
             if (p) (void)hipFree(p);
         if (stream) (void)hipStreamDestroy(stream);
@@ -232,13 +211,13 @@ struct lbm_batch {
     //   v        0  1  2  3  4  5
     //   cells    1  1  2  2  4  4      (f16s: 2 2 4 4 8 8)
     //   chunked  0  1  0  1  0  1
-    // variants 6, 7: two steps per launch (k_batch_pair) in chunks of 8 / 16
-    // rows; their one-step launches (the first and last steps of a call) run
-    // as the two-cells-per-thread variant (f32 2, binary16 0)
-    static constexpr int kPairFirst = 6;
-    static bool pair_variant(int v) { return v >= kPairFirst; }
+    // variants 6, 7: several steps per launch (k_batch_tile, shapes 0 and 1);
+    // their calls of one step run as the two-cells-per-thread variant (f32 2,
+    // binary16 0)
+    static constexpr int kTileFirst = 6;
+    static bool tile_variant(int v) { return v >= kTileFirst; }
     int one_step_variant() const {
-        return pair_variant(variant) ? (precision == LBM_PRECISION_F32 ? 2 : 0) : variant;
+        return tile_variant(variant) ? (precision == LBM_PRECISION_F32 ? 2 : 0) : variant;
     }
     int cpt_of(int v) const {
         const int c = v / 2 == 0 ? 1 : (v / 2 == 1 ? 2 : 4);
@@ -248,19 +227,28 @@ struct lbm_batch {
     char *fptr(int s, const DomainDev &d) const { return (char *)f[s] + (size_t)d.f_off * esize; }
 
     // ---- lists -----------------------------------------------------------------
+    // the bounce-back bytes of the current masks
+    void ensure_flags() {
+        if (!flags_dirty) return;
+        // (blockIdx.y holds at most 65535 domains)
+        for (size_t i = 0; i < table.size(); i += 65535) {
+            const dim3 grid((max_cells + kBlock - 1) / kBlock, (unsigned)std::min<size_t>(65535, table.size() - i));
+            if (boundary == LBM_BOUNDARY_REFERENCE)
+                hipLaunchKernelGGL(k_batch_flags<LBM_BOUNDARY_REFERENCE>, grid, dim3(kBlock), 0, stream, mask, flags,
+                                   dtable + i);
+            else
+                hipLaunchKernelGGL(k_batch_flags<LBM_BOUNDARY_ZERO_GRADIENT>, grid, dim3(kBlock), 0, stream, mask,
+                                   flags, dtable + i);
+            HIPCHK(hipGetLastError());
+        }
+        flags_dirty = false;
+    }
+
     void rebuild_lists(int cpt) {
-        // bounce-back and segment bytes on the device, lists on the host
-        fixed_dirty = true;
+        // segment bytes on the device, lists on the host
+        ensure_flags();
         for (size_t i = 0; i < table.size(); ++i) {
             const DomainDev &d = table[i];
-            const dim3 gf((d.g.X + 255) / 256, d.g.Y);
-            if (boundary == LBM_BOUNDARY_REFERENCE)
-                hipLaunchKernelGGL(k_build_flags<LBM_BOUNDARY_REFERENCE>, gf, dim3(256), 0, stream, mask + d.aux_off,
-                                   flags + d.aux_off, d.g);
-            else
-                hipLaunchKernelGGL(k_build_flags<LBM_BOUNDARY_ZERO_GRADIENT>, gf, dim3(256), 0, stream,
-                                   mask + d.aux_off, flags + d.aux_off, d.g);
-            HIPCHK(hipGetLastError());
             const int srow = d.g.pitch / 64 + kSegSlack;
             hipLaunchKernelGGL(k_build_segments, dim3((srow + 255) / 256, d.g.Y), dim3(256), 0, stream,
                                flags + d.aux_off, segs + d.seg_off, nullptr, nullptr, d.g);
@@ -364,130 +352,103 @@ struct lbm_batch {
         pform = false;
     }
 
-    // ---- two steps per launch ---------------------------------------------------------
+    // ---- several steps per launch ------------------------------------------------------
     size_t set_bytes() const { return f_elems * esize; }
-    // a set's allocation: two rows of the widest domain more, which the
-    // two-step kernel's loads in the last domain's last rows read and discard
+    // a set's allocation: two rows of the widest domain more, which
+    // k_batch_tile's wrapped outlet pulls of the last domain read and discard
     size_t alloc_bytes() const { return (f_elems + tail_elems) * esize; }
+    // as a single grid's: two more sets of at most this are there from the start
+    static constexpr size_t kAutoSpareBytes = (size_t)512 << 20;
 
-    void release_pair_buffers() {
-        drop_graphs();
-        for (void *&q : spare) {
-            if (q) (void)hipFree(q);
-            q = nullptr;
-        }
-        if (plist) (void)hipFree(plist);
-        plist = nullptr;
-        n_pair = 0;
-        plist_rows = 0;
-        for (void *q : {(void *)fixed, (void *)rowtab, (void *)fixed_rows})
-            if (q) (void)hipFree(q);
-        fixed = rowtab = nullptr;
-        fixed_rows = nullptr;
-        n_fixed = 0;
-    }
-
-    // allocated when a two-step variant is selected, so that stepping itself
-    // does not allocate: the output sets, and the fixed-cell list (room for
-    // every cell) with its row table (domain, row) and per-row offsets
-    void ensure_pair_buffers() {
-        if (spare[0] && spare[1] && fixed) return;
-        release_pair_buffers();
+    void make_spare(void *out[2]) {
+        out[0] = out[1] = nullptr;
         try {
-            spare[0] = dalloc<char>(alloc_bytes());
-            spare[1] = dalloc<char>(alloc_bytes());
-            std::vector<uint2> rt;
-            for (size_t i = 0; i < table.size(); ++i)
-                for (int y = 0; y < table[i].g.Y; ++y) rt.push_back(make_uint2((uint32_t)i, (uint32_t)y));
-            n_rows = (uint32_t)rt.size();
-            fixed = dalloc<uint2>((size_t)cells);
-            rowtab = dalloc<uint2>(rt.size());
-            fixed_rows = dalloc<uint32_t>(rt.size());
-            // the rows' padding is never written by the two-step kernel: keep it defined
-            HIPCHK(hipMemsetAsync(spare[0], 0, set_bytes(), stream));
-            HIPCHK(hipMemsetAsync(spare[1], 0, set_bytes(), stream));
-            HIPCHK(hipMemcpyAsync(rowtab, rt.data(), rt.size() * sizeof(uint2), hipMemcpyHostToDevice, stream));
-            HIPCHK(hipStreamSynchronize(stream));
-            fixed_dirty = true;
+            for (int i = 0; i < 2; ++i) {
+                out[i] = dalloc<char>(alloc_bytes());
+                // the rows' padding is never written by k_batch_tile: keep it defined
+                HIPCHK(hipMemsetAsync(out[i], 0, set_bytes(), stream));
+            }
         } catch (...) {
-            release_pair_buffers();
+            for (int i = 0; i < 2; ++i)
+                if (out[i]) (void)hipFree(out[i]);
             throw;
         }
     }
+    void release_spare() {
+        for (void *&p : spare) {
+            if (p) (void)hipFree(p);
+            p = nullptr;
+        }
+    }
+    // a tile variant's sets; setting one does not take over the default path's
+    void ensure_spare(bool take_over = true) {
+        if (spare[0] && (take_over || !auto_path)) return;
+        void *fresh[2];
+        make_spare(fresh);
+        release_spare();
+        spare[0] = fresh[0];
+        spare[1] = fresh[1];
+    }
 
-    // the fixed-cell list from the current flags; waits for the stream.  Drops
-    // the graphs, whose fixed-cell launches hold the old count.
-    void build_fixed_list() {
-        hipLaunchKernelGGL(k_batch_fixed_count, dim3(n_rows), dim3(kFixedBlock), 0, stream, flags, dtable, rowtab,
-                           fixed_rows);
-        HIPCHK(hipGetLastError());
-        std::vector<uint32_t> off(n_rows);
-        HIPCHK(hipMemcpyAsync(off.data(), fixed_rows, off.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
+    static size_t combination(int shape, int steps) { return (size_t)shape * (kTileMaxSteps + 1) + steps; }
+    // the domains' running block counts, of every shape and number of steps
+    void build_starts() {
+        const size_t n = table.size();
+        tile_blocks.assign(2 * (kTileMaxSteps + 1), 0);
+        std::vector<uint32_t> all(tile_blocks.size() * (n + 1), 0);
+        for (int shape = 0; shape < 2; ++shape) {
+            const TileShape &sh = tile_shape(precision, shape);
+            for (int steps = 2; steps <= kTileMaxSteps; ++steps) {
+                const size_t c = combination(shape, steps);
+                uint64_t total = 0;
+                for (size_t i = 0; i < n; ++i) {
+                    all[c * (n + 1) + i] = (uint32_t)total;
+                    total += (uint64_t)tile_nbx(table[i].g.X, steps) * tile_nby(table[i].g.Y, sh.waves * sh.m, steps);
+                }
+                tile_blocks[c] = (uint32_t)std::min<uint64_t>(total, UINT32_MAX);  // tile_plan leaves that many out
+            }
+        }
+        starts = dalloc<uint32_t>(all.size());
+        HIPCHK(hipMemcpyAsync(starts, all.data(), all.size() * sizeof(uint32_t), hipMemcpyHostToDevice, stream));
         HIPCHK(hipStreamSynchronize(stream));
-        uint32_t total = 0;
-        for (uint32_t &o : off) {
-            const uint32_t c = o;
-            o = total;
-            total += c;
-        }
-        HIPCHK(hipMemcpyAsync(fixed_rows, off.data(), off.size() * sizeof(uint32_t), hipMemcpyHostToDevice, stream));
-        hipLaunchKernelGGL(k_batch_fixed_emit, dim3(n_rows), dim3(kFixedBlock), 0, stream, flags, mask, dtable,
-                           rowtab, fixed_rows, fixed);
-        HIPCHK(hipGetLastError());
-        HIPCHK(hipStreamSynchronize(stream));  // `off` is read by the copy above
-        n_fixed = total;
-        fixed_dirty = false;
-        drop_graphs();
     }
 
-    int pair_rows() const { return 8 << (variant - kPairFirst); }
-
-    void ensure_pair_list() {
-        const int rows = pair_rows();
-        if (plist && plist_rows == rows) return;
-        std::vector<uint2> pl;
-        for (size_t i = 0; i < table.size(); ++i) {
-            const Geom &g = table[i].g;
-            const int nstrips = (g.X + kBlock - 3) / (kBlock - 2), nchunks = (g.Y + rows - 1) / rows;
-            for (int c = 0; c < nchunks; ++c)
-                for (int sx = 0; sx < nstrips; ++sx)
-                    pl.push_back(make_uint2((uint32_t)i, ((uint32_t)sx << 16) | (uint32_t)c));
-        }
-        uint2 *d = dalloc<uint2>(pl.size());
-        try {
-            HIPCHK(hipMemcpyAsync(d, pl.data(), pl.size() * sizeof(uint2), hipMemcpyHostToDevice, stream));
-            HIPCHK(hipStreamSynchronize(stream));
-        } catch (...) {
-            (void)hipFree(d);
-            throw;
-        }
-        if (plist) (void)hipFree(plist);
-        plist = d;
-        n_pair = (uint32_t)pl.size();
-        plist_rows = rows;
-        drop_graphs();
-    }
-
-    // C_n, C_{n-1} in f[cur], f[1 - cur] -> C_{n+2}, C_{n+1} (the latter only
-    // where the next step reads it); the spare sets take the old ones
-    template <class St, int MODE>
-    void launch_pair() {
+    template <class St, int MODE, int SHAPE>
+    void launch_tile(int steps, bool final) {
         using T = typename St::T;
-        const T *A = (const T *)f[cur], *B = (const T *)f[1 - cur];
-        T *A2 = (T *)spare[0], *B2 = (T *)spare[1];
-        const unsigned nfix = (n_fixed + kBlock - 1) / kBlock;
-        hipLaunchKernelGGL((k_batch_pair<St, MODE>), dim3(n_pair + nfix), dim3(kBlock), 0, stream, A, B, A2, B2,
-                           flags, dtable, plist, (int)n_pair, pair_rows(), fixed, rowtab, n_fixed);
+        constexpr TileShape sh = tile_shape<T>(SHAPE);
+        constexpr size_t lds = tile_lds(sh, sizeof(T));
+        const size_t c = combination(SHAPE, steps);
+        tile_allow_lds<k_batch_tile<St, MODE, SHAPE>>(lds, dev);
+        hipLaunchKernelGGL((k_batch_tile<St, MODE, SHAPE>), dim3(tile_blocks[c]), dim3(64 * sh.waves), lds, stream,
+                           (const T *)f[cur], (const T *)f[1 - cur], (T *)spare[0], (T *)spare[1], flags, mask, dtable,
+                           starts + c * (table.size() + 1), (int)table.size(), steps, pform ? 0 : 1, final ? 1 : 0,
+                           lag);
         HIPCHK(hipGetLastError());
-        spare[0] = f[cur];
-        spare[1] = f[1 - cur];
-        f[cur] = A2;
-        f[1 - cur] = B2;
-        pair_parity ^= 1;
+        // the sets' parity goes on as with single steps (see the single grid's)
+        void *const a0 = f[cur], *const b0 = f[1 - cur];
+        cur = (cur + steps - (pform ? 0 : 1)) & 1;
+        f[cur] = spare[0];
+        f[1 - cur] = spare[1];
+        spare[0] = a0;
+        spare[1] = b0;
+        pform = true;
     }
 
-    void pair() {
-        dispatch([&]<class St, int MODE>() { launch_pair<St, MODE>(); });
+    void tile(int shape, int steps, bool final) {
+        dispatch([&]<class St, int MODE>() {
+            if (shape == 0) launch_tile<St, MODE, 0>(steps, final);
+            else launch_tile<St, MODE, 1>(steps, final);
+        });
+    }
+
+    // a call's launches of k_batch_tile; none where it is not used
+    TilePlan plan_tile(uint32_t n) const {
+        if (n < 2 || !spare[0] || !(auto_path || tile_variant(variant))) return {0, 0};
+        const bool any = !tile_variant(variant);
+        const int first = any ? 0 : variant - kTileFirst, last = any ? 1 : first;
+        return tile_plan(precision, first, last, n, pform,
+                         [&](int i, int s) { return (int64_t)tile_blocks[combination(i, s)]; });
     }
 
     template <class F>
@@ -499,29 +460,25 @@ struct lbm_batch {
     }
 
     void flush() {
+        if (pform) ensure_lists();
         dispatch([&]<class St, int MODE>() { flush_t<St, MODE>(); });
     }
 
-    // two fused steps from cur = c (four for the two-step variants), captured
-    // once per arrangement of the sets and replayed
+    // two fused steps from cur = c, captured once and replayed.  (The tile path's
+    // launches carry several steps each and trade the sets: they are launched.)
     hipGraphExec_t pair_graph(int c) {
         if (graph_variant != variant) drop_graphs();
-        hipGraphExec_t &gx = graph[c][pair_parity];
+        hipGraphExec_t &gx = graph[c];
         if (!gx) {
             const int saved = cur;
             cur = c;
             hipGraph_t gr;
             HIPCHK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
             try {
-                if (pair_variant(variant)) {
-                    pair();  // f[] and spare[] trade places ...
-                    pair();  // ... and trade back: the graph leaves them as it found them
-                } else {
-                    dispatch([&]<class St, int MODE>() {
-                        do_step<St, MODE>(false);
-                        do_step<St, MODE>(false);
-                    });
-                }
+                dispatch([&]<class St, int MODE>() {
+                    do_step<St, MODE>(false);
+                    do_step<St, MODE>(false);
+                });
             } catch (...) {
                 hipGraph_t dummy;
                 (void)hipStreamEndCapture(stream, &dummy);
@@ -535,38 +492,35 @@ struct lbm_batch {
             cur = saved;
             HIPCHK(e);
             graph_variant = variant;
+            graph_sets[0] = f[0];
+            graph_sets[1] = f[1];
         }
         return gx;
     }
 
     void step(uint32_t n) {
         if (n == 0) return;
-        ensure_lists();
-        const bool two = pair_variant(variant);
-        if (two) {
-            ensure_pair_buffers();
-            ensure_pair_list();
-            if (fixed_dirty) build_fixed_list();
+        if (const TilePlan plan = plan_tile(n); plan.launches) {
+            ensure_flags();
+            const uint32_t low = n / plan.launches, more = n % plan.launches;
+            for (uint32_t i = 0; i < plan.launches; ++i)
+                tile(plan.shape, (int)(low + (i < more)), i + 1 == plan.launches);
+            steps += n;
+            return;
         }
+        ensure_lists();
         uint32_t left = n;
         if (!pform) {
             dispatch([&]<class St, int MODE>() { do_step<St, MODE>(left == 1); });
             --left;
         }
-        // all but the last step from the graph: two steps at a time, or four
-        // (two two-step launches) for the two-step variants
-        const uint32_t per = two ? 4 : 2;
+        // all but the last step from the graph, two steps at a time
         if (use_graph) {
-            while (left > per) {
+            if (graph_sets[0] != f[0] || graph_sets[1] != f[1]) drop_graphs();
+            while (left > 2) {
                 HIPCHK(hipGraphLaunch(pair_graph(cur), stream));
-                left -= per;  // the graph leaves cur (and the sets) where it started
+                left -= 2;  // the graph leaves cur where it started
             }
-        }
-        // two-step launches while at least one step is left for the closing
-        // one-step launch, which leaves both sets whole
-        while (two && left >= 3) {
-            pair();
-            left -= 2;
         }
         while (left > 0) {
             dispatch([&]<class St, int MODE>() { do_step<St, MODE>(left == 1); });
@@ -669,6 +623,7 @@ int lbm_batch_create(const lbm_domain *doms, uint32_t n, int32_t precision, int3
         so += ((long long)(pitch / 64 + kSegSlack) * Y + 15) / 16 * 16;
         b->cells += (uint64_t)X * Y;
         b->tail_elems = std::max(b->tail_elems, 18 * (size_t)pitch);
+        b->max_cells = std::max(b->max_cells, (uint32_t)((uint64_t)pitch * Y));
     }
     b->f_elems = fo;
     b->aux_elems = ao;
@@ -688,6 +643,13 @@ int lbm_batch_create(const lbm_domain *doms, uint32_t n, int32_t precision, int3
         for (const DomainDev &d : b->table) {
             hipLaunchKernelGGL(k_walls, dim3((d.g.X + 255) / 256), dim3(256), 0, b->stream, b->mask + d.aux_off, d.g);
             HIPCHK(hipGetLastError());
+        }
+        b->build_starts();
+        if (2 * b->alloc_bytes() <= lbm_batch::kAutoSpareBytes) {
+            try {
+                b->make_spare(b->spare);
+            } catch (const HipError &) {  // no memory for them: one step per launch
+            }
         }
         HIPCHK(hipStreamSynchronize(b->stream));
     });
@@ -747,7 +709,7 @@ int lbm_batch_set_mask(lbm_batch *b, uint32_t d, const uint8_t *solid) {
         b->flush();  // the pending stream uses the old mask
         // the host's bytes go through the domain's flag plane, which is rebuilt
         // (with the lists) before the next step
-        b->dirty = true;
+        b->dirty = b->flags_dirty = true;
         HIPCHK(hipMemcpyAsync(b->flags + dd.aux_off, solid, (size_t)dd.g.X * dd.g.Y, hipMemcpyHostToDevice,
                               b->stream));
         hipLaunchKernelGGL(k_place_mask, dim3((dd.g.X + 255) / 256, dd.g.Y), dim3(256), 0, b->stream,
@@ -764,7 +726,8 @@ int lbm_batch_step(lbm_batch *b, uint32_t n) {
 int lbm_batch_step_timed(lbm_batch *b, uint32_t n, float *ms) {
     return bguard(b, [&] {
         bcheck(ms != nullptr, "null output");
-        b->ensure_lists();
+        if (b->plan_tile(n).launches) b->ensure_flags();
+        else b->ensure_lists();
         hipEvent_t e0, e1;
         HIPCHK(hipEventCreate(&e0));
         HIPCHK(hipEventCreate(&e1));
@@ -808,9 +771,10 @@ int lbm_batch_set_variant(lbm_batch *b, int variant) {
     return bguard(b, [&] {
         bcheck(variant >= 0 && variant < LBM_BATCH_NUM_VARIANTS, "unknown variant");
         HIPCHK(hipStreamSynchronize(b->stream));
-        if (lbm_batch::pair_variant(variant)) b->ensure_pair_buffers();  // may fail: then nothing changes
-        else b->release_pair_buffers();
+        if (lbm_batch::tile_variant(variant)) b->ensure_spare(false);  // may fail: then nothing changes
+        else b->release_spare();
         b->variant = variant;
+        b->auto_path = false;
     });
 }
 
@@ -829,8 +793,10 @@ int lbm_batch_autotune(lbm_batch *b, uint32_t steps, int *best, float *ms) {
         const bool pform = b->pform;
         const uint64_t nsteps = b->steps;
         const int variant0 = b->variant;
+        const bool auto_path = b->auto_path, had_spare = b->spare[0] != nullptr;
         float t[LBM_BATCH_NUM_VARIANTS];
         int v_best = 0;
+        b->auto_path = false;  // time each variant's own kernels
         try {
             HIPCHK(hipMemcpyAsync(snap, b->f[0], sb, hipMemcpyDeviceToDevice, b->stream));
             HIPCHK(hipMemcpyAsync(snap + sb, b->f[1], sb, hipMemcpyDeviceToDevice, b->stream));
@@ -839,13 +805,13 @@ int lbm_batch_autotune(lbm_batch *b, uint32_t steps, int *best, float *ms) {
             HIPCHK(hipEventCreate(&e0));
             HIPCHK(hipEventCreate(&e1));
             for (int v = 0; v < LBM_BATCH_NUM_VARIANTS; ++v) {
-                if (lbm_batch::pair_variant(v)) {
-                    if (steps < 3) {  // a call this short never launches two steps at once
+                if (lbm_batch::tile_variant(v)) {
+                    if (steps < 3) {  // too few steps a call for what these variants are for
                         t[v] = INFINITY;
                         continue;
                     }
                     try {
-                        b->ensure_pair_buffers();
+                        b->ensure_spare();
                     } catch (...) {  // no memory for two more sets: not a candidate
                         t[v] = INFINITY;
                         continue;
@@ -873,6 +839,8 @@ int lbm_batch_autotune(lbm_batch *b, uint32_t steps, int *best, float *ms) {
             b->pform = pform;
             b->steps = nsteps;
             b->variant = variant0;
+            b->auto_path = auto_path;
+            if (!had_spare) b->release_spare();
             throw;
         }
         (void)hipFree(snap);
@@ -880,7 +848,7 @@ int lbm_batch_autotune(lbm_batch *b, uint32_t steps, int *best, float *ms) {
         b->pform = pform;
         b->steps = nsteps;
         b->variant = v_best;
-        if (!lbm_batch::pair_variant(v_best)) b->release_pair_buffers();  // tried, not kept
+        if (!lbm_batch::tile_variant(v_best)) b->release_spare();  // tried, not kept
         if (best) *best = v_best;
         if (ms)
             for (int v = 0; v < LBM_BATCH_NUM_VARIANTS; ++v) ms[v] = t[v] / steps;
@@ -904,12 +872,14 @@ int lbm_batch_autotune_cached(lbm_batch *b, const char *cache_path, uint32_t ste
                                     (b->boundary == LBM_BOUNDARY_REFERENCE ? "/ref" : "/zg") + "/v" +
                                     std::to_string(LBM_BATCH_NUM_VARIANTS));
         found = tune_cache::lookup(cache_path, key, e) && e.variant >= 0 && e.variant < LBM_BATCH_NUM_VARIANTS;
-        if (found) b->variant = e.variant;
     });
     if (rc != LBM_OK) return rc;
-    if (hit) *hit = found ? 1 : 0;
-    if (found) {
+    if (hit) *hit = 0;
+    // a cached variant whose spare sets cannot be allocated here is a miss
+    if (found && lbm_batch_set_variant(b, e.variant) == LBM_OK) {
+        if (hit) *hit = 1;
         if (best) *best = e.variant;
+        b->err.clear();
         return LBM_OK;
     }
     e.ms.assign(LBM_BATCH_NUM_VARIANTS, 0.0f);
@@ -923,7 +893,6 @@ int lbm_batch_autotune_cached(lbm_batch *b, const char *cache_path, uint32_t ste
 int lbm_batch_read_f(lbm_batch *b, uint32_t d, float *f9) {
     return bguard(b, [&] {
         bcheck(d < b->table.size() && f9, "bad domain or null output");
-        b->ensure_lists();
         b->flush();
         const DomainDev &dd = b->table[d];
         const size_t dn = (size_t)dd.g.X * dd.g.Y;

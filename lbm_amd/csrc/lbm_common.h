@@ -52,26 +52,29 @@ __host__ __device__ __forceinline__ void upstream(int k, int x, int y, int X, in
     }
 }
 
+// the bounce-back byte of one cell
+template <int MODE>
+__device__ __forceinline__ uint8_t flag_byte(const uint8_t *__restrict__ mask, const Geom &g, int x, int y) {
+    const bool streamed = mask[(size_t)y * g.pitch + x] != 1 && x != 0 && y < g.Y - 1;
+    if (!streamed) return kSlowCell;
+    uint8_t b = 0;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+        if (k == C) continue;
+        int ux, uy;
+        upstream<MODE>(k, x, y, g.X, ux, uy);
+        const bool solid = uy < 0 || uy >= g.Y || ux < 0 || mask[(size_t)uy * g.pitch + ux] == 1;
+        if (solid) b |= (uint8_t)(1u << bit(k));
+    }
+    return b;
+}
+
 template <int MODE>
 __global__ void k_build_flags(const uint8_t *__restrict__ mask, uint8_t *__restrict__ flags, Geom g) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x;
     const int y = blockIdx.y;
     if (x >= g.X) return;
-    const size_t own = (size_t)y * g.pitch + x;
-    const bool streamed = mask[own] != 1 && x != 0 && y < g.Y - 1;
-    uint8_t b = kSlowCell;
-    if (streamed) {
-        b = 0;
-#pragma unroll
-        for (int k = 0; k < 9; ++k) {
-            if (k == C) continue;
-            int ux, uy;
-            upstream<MODE>(k, x, y, g.X, ux, uy);
-            const bool solid = uy < 0 || uy >= g.Y || ux < 0 || mask[(size_t)uy * g.pitch + ux] == 1;
-            if (solid) b |= (uint8_t)(1u << bit(k));
-        }
-    }
-    flags[own] = b;
+    flags[(size_t)y * g.pitch + x] = flag_byte<MODE>(mask, g, x, y);
 }
 
 // The grid is cut into 64-cell segments of a row.  A segment is "clear" when

@@ -40,10 +40,10 @@ namespace {
 // them counting the halo (168 us in f32, 141 in binary16 against 163), and a
 // small grid by the 2 us a launch and the 1 us of a region's step (1.6 us a
 // step).  More rows a wave mean less halo and fewer waves in flight: measured
-// at 8192 x 4096 in f32, us per step, for 1 x 16, 2 x 16, 3 x 12, 5 x 8 rows x
-// waves: 300, 176, 168, 188; two rows of which a block keeps 16 waves twice on
-// a CU are best for binary16 (141; 3 x 12: 150).  2, 4, 6, 8 steps: 245 (3),
-// 196, 168, 178.
+// at 8192 x 4096 in f32, us per step of 6 steps a launch, for 2 x 16, 3 x 12 and
+// 5 x 8 rows x waves: 176, 168, 188; binary16, of 5 steps, 2 x 16 (two blocks a
+// CU, as its values need fewer registers) and 3 x 12: 141, 150.  3, 4, 6, 8
+// steps a launch with 3 x 12 rows in f32: 246, 196, 168, 178.
 struct TileArgs {
     int steps;         // 2 .. kTileMaxSteps
     int nbx, nby;      // regions across and down

@@ -48,3 +48,39 @@ def test_tile_equals_one_step(nx, ny, precision, boundary):
             assert np.array_equal(both_sets(g), want), (walls, v, "after paint")
             g.close()
         grids[0].close()
+
+
+@pytest.mark.parametrize("precision", [0, 1, 2])
+@pytest.mark.parametrize("boundary", [0, 1])
+def test_batch_tile_equals_one_step(precision, boundary):
+    """Seventy domains around the regions' sizes (more than one wave of block
+    counts to search): the default path and both tile variants give the one-step
+    variants' populations and moments, through mask changes between calls."""
+    from lbm_amd import Batch
+    print(f"case: batch tile precision {precision} boundary {boundary}", flush=True)
+    rng = np.random.default_rng(precision * 2 + boundary)
+    sizes = [(3, 3), (62, 15), (63, 14), (64, 16), (65, 31), (121, 37), (200, 70)] * 10
+    doms = [(nx, ny, rng.uniform(1.2, 1.7), rng.uniform(0.02, 0.08)) for nx, ny in sizes]
+    batches = []
+    for variant in (0, None, 6, 7):
+        b = Batch(doms, precision=precision, boundary=boundary)
+        if variant is not None:
+            b.variant = variant
+        batches.append(b)
+    for n in (8, 9, 2, 1, 25, 6):
+        for i in rng.choice(len(doms), 40, replace=False):
+            mask = (rng.random((doms[i][1], doms[i][0])) < 0.06).astype(np.uint8)
+            for b in batches:
+                b.set_mask(i, mask)
+        for b in batches:
+            b.step(n)
+        for i in range(0, len(doms), 3):
+            want = batches[0].moments(i)
+            for b, v in zip(batches[1:], ("default", 6, 7)):
+                assert all(same_bits(p, q) for p, q in zip(b.moments(i), want)), (i, v, n)
+    for i in range(len(doms)):
+        want = batches[0].read_f(i)
+        for b, v in zip(batches[1:], ("default", 6, 7)):
+            assert same_bits(b.read_f(i), want), (i, v)
+    for b in batches:
+        b.close()
