@@ -818,7 +818,7 @@ int lbm_batch_autotune(lbm_batch *b, uint32_t steps, int *best, float *ms) {
                     }
                 }
                 b->variant = v;
-                b->step(2);  // builds lists and graphs, leaves P-form
+                b->step(4);  // builds lists and graphs, leaves P-form; the fewest steps k_batch_tile runs from there
                 HIPCHK(hipEventRecord(e0, b->stream));
                 b->step(steps);
                 HIPCHK(hipEventRecord(e1, b->stream));

@@ -1032,7 +1032,9 @@ int lbm_autotune(lbm_grid *g, uint32_t steps, int *best, float *ms) {
                     }
                 }
                 g->variant = v;
-                g->step(2);  // warm-up (and leaves the grid in P-form)
+                // warm-up (and leaves the grid in P-form); four steps: the
+                // fewest that k_tile runs from there
+                g->step(4);
                 HIPCHK(hipEventRecord(e0, g->stream));
                 g->step(steps);
                 HIPCHK(hipEventRecord(e1, g->stream));

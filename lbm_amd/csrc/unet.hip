@@ -9,10 +9,9 @@
 // have the same lane layout -- lane l holds row l % 32 and k = 8 (l / 32) +
 // 0..7, i.e. 16 contiguous bytes of one pixel's channels or of one row of
 // W[tap][cout][cin] -- so which of them is "A" only decides the layout of the
-// result.  The 1x1 kernel puts pixels in A: D (32 x 32 f32), lane l, value r
-// holds pixel 8 (r / 4) + 4 (l / 32) + r % 4, cout l % 32.  The 3x3 kernels put
-// the weights in A: lane l holds pixel l % 32 and couts 8 (r / 4) + 4 (l / 32)
-// + r % 4, four runs of four consecutive channels that are stored as vectors.
+// result D (32 x 32 f32).  The kernels put the weights in A: lane l, value r
+// holds pixel l % 32 and cout 8 (r / 4) + 4 (l / 32) + r % 4, four runs of four
+// consecutive channels that are stored as vectors.
 // The input gradient is the same forward convolution applied to the output
 // gradient with the weights flipped in space and transposed in channels; the
 // weight gradient reduces over pixels (K), with both operands transposed on
@@ -43,6 +42,13 @@ __device__ __forceinline__ uint16_t f2bf(float v) {  // round to nearest even
     return __builtin_bit_cast(uint16_t, (__bf16)v);
 }
 __device__ __forceinline__ float bf2f(uint16_t v) { return (float)__builtin_bit_cast(__bf16, v); }
+// v > 0 of a bf16 value (false for NaN)
+__device__ __forceinline__ bool positive(uint16_t v) { return (uint16_t)(v - 1) < 0x7F80; }
+// two bf16 values of a pair of activations' gradient: zero where the activation
+// (after its ReLU) is not positive
+__device__ __forceinline__ uint32_t gate2(uint32_t g, uint32_t y) {
+    return (positive((uint16_t)y) ? g & 0xFFFFu : 0u) | (positive((uint16_t)(y >> 16)) ? g & 0xFFFF0000u : 0u);
+}
 
 // ---- convolution forward (and input gradient) ------------------------------------
 // Input of a convolution, NHWC bf16: channels [0, ca) come from a, channels
@@ -64,11 +70,14 @@ typedef uint16_t u16x16 __attribute__((ext_vector_type(16)));  // 32 B: one lane
 // eight and the second k-step their last eight (the same permutation of K for
 // A and B).  The next chunk's operands are loaded while the current one is
 // multiplied.  Requirements: P % (32 * MI) == 0, Cin % 32 == 0,
-// Cout % (32 * NI) == 0.  Only channels co < co_store are stored.
+// Cout % (32 * NI) == 0.  Only channels co < co_store, rounded up to a multiple
+// of four, are stored: the weights are the A operand, as in the 3x3 kernels, so
+// that a lane holds runs of four channels of one pixel (with the pixels in A it
+// held one channel and stored two bytes at a time).
 template <int MI, int NI, bool RELU, bool OUT_F32>
 __global__ __launch_bounds__(256) void k_conv1x1(const uint16_t *__restrict__ in, const uint16_t *__restrict__ w,
                                                  const float *__restrict__ bias, void *__restrict__ out, long long P,
-                                                 int Cin, int Cout, int co_store) {
+                                                 int Cin, int Cout, int co_store, const uint16_t *__restrict__ gate) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int half = lane >> 5, l32 = lane & 31;
     const long long p0 = ((long long)blockIdx.x * 4 + wave) * (32 * MI);
@@ -98,8 +107,8 @@ __global__ __launch_bounds__(256) void k_conv1x1(const uint16_t *__restrict__ in
                 for (int j = 0; j < NI; ++j) {
                     const u16x8 b8 = s == 0 ? __builtin_shufflevector(b[j], b[j], 0, 1, 2, 3, 4, 5, 6, 7)
                                             : __builtin_shufflevector(b[j], b[j], 8, 9, 10, 11, 12, 13, 14, 15);
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a8),
-                                                                        __builtin_bit_cast(bf16x8, b8), acc[i][j],
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, b8),
+                                                                        __builtin_bit_cast(bf16x8, a8), acc[i][j],
                                                                         0, 0, 0);
                 }
             }
@@ -114,20 +123,33 @@ __global__ __launch_bounds__(256) void k_conv1x1(const uint16_t *__restrict__ in
         if (kk + 2 < nk) load(kk + 2, A0, B0);
         mma(A1, B1);
     }
+    // lane l holds pixel l % 32 and channels 8 g + 4 (l / 32) .. + 3: four at a time
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
+        const long long p = p0 + 32 * i + l32;
 #pragma unroll
         for (int j = 0; j < NI; ++j) {
-            const int co = co0 + 32 * j + l32;
-            const float bv = bias ? bias[co] : 0.0f;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const long long p = p0 + 32 * i + 8 * (r / 4) + 4 * half + (r % 4);
-                float v = acc[i][j][r] + bv;
-                if (RELU) v = fmaxf(v, 0.0f);
-                if (co < co_store) {
-                    if (OUT_F32) ((float *)out)[p * Cout + co] = v;
-                    else ((uint16_t *)out)[p * Cout + co] = f2bf(v);
+            for (int g = 0; g < 4; ++g) {
+                const int co = co0 + 32 * j + 8 * g + 4 * half;
+                if (co >= co_store) continue;
+                const float4 bv = bias ? *(const float4 *)&bias[co] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                float v[4] = {acc[i][j][4 * g] + bv.x, acc[i][j][4 * g + 1] + bv.y, acc[i][j][4 * g + 2] + bv.z,
+                              acc[i][j][4 * g + 3] + bv.w};
+                if (RELU)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = fmaxf(v[e], 0.0f);
+                if (OUT_F32) {
+                    *(float4 *)&((float *)out)[p * Cout + co] = make_float4(v[0], v[1], v[2], v[3]);
+                } else {
+                    uint32_t lo = f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16),
+                             hi = f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
+                    if (gate) {
+                        const uint2 y = *(const uint2 *)&gate[p * Cout + co];
+                        lo = gate2(lo, y.x);
+                        hi = gate2(hi, y.y);
+                    }
+                    *(uint2 *)&((uint16_t *)out)[p * Cout + co] = make_uint2(lo, hi);
                 }
             }
         }
@@ -138,16 +160,21 @@ __global__ __launch_bounds__(256) void k_conv1x1(const uint16_t *__restrict__ in
 // the A operand and the pixels as B, so a wave's 32 x 32 result is
 // [cout][pixel]: lane l holds pixel l % 32 and output channels
 // 8 (r / 4) + 4 (l / 32) + r % 4, r = 0..15 -- four runs of four consecutive
-// channels, stored as four 8-byte (bf16) or 16-byte (f32) pieces.  A wave
+// channels, stored as four 8-byte (bf16) or 16-byte (f32) pieces.  gate (input
+// gradients, bf16): the activation the gradient belongs to, of the output's
+// shape; where it is not positive its ReLU passes nothing on and 0 is stored
+// (a pass of its own read and wrote every gradient once more: 17 launches,
+// 230 us of one 8 x 256 x 256 minibatch).  A wave
 // covers MI rows (from y_first) x 32 columns (from x0) x NI tiles of 32
 // output channels (from co_first).  With a K split (gridDim.z > 1) the raw
 // sums go to part[z][p][co]; otherwise bias, ReLU and the store of channels
 // co < co_store.
 template <int MI, int NI>
 __device__ __forceinline__ void conv_store_tile(const f32x16 (&acc)[MI][NI], const float *__restrict__ bias,
-                                                void *__restrict__ out, float *__restrict__ part, int N, int H, int W,
-                                                int Cout, int co_store, int relu, int out_f32, long long n, int x0,
-                                                int y_first, int co_first, int half, int l32) {
+                                                void *__restrict__ out, float *__restrict__ part,
+                                                const uint16_t *__restrict__ gate, int N, int H, int W, int Cout,
+                                                int co_store, int relu, int out_f32, long long n, int x0, int y_first,
+                                                int co_first, int half, int l32) {
     const long long P = (long long)N * H * W;
     const bool split = gridDim.z > 1;
 #pragma unroll
@@ -179,8 +206,13 @@ __device__ __forceinline__ void conv_store_tile(const f32x16 (&acc)[MI][NI], con
                     if (out_f32) {
                         *(float4 *)&((float *)out)[p * Cout + co] = make_float4(v[0], v[1], v[2], v[3]);
                     } else {
-                        const uint32_t lo = f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16),
-                                       hi = f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
+                        uint32_t lo = f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16),
+                                 hi = f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
+                        if (gate) {
+                            const uint2 y2 = *(const uint2 *)&gate[p * Cout + co];
+                            lo = gate2(lo, y2.x);
+                            hi = gate2(hi, y2.y);
+                        }
                         *(uint2 *)&((uint16_t *)out)[p * Cout + co] = make_uint2(lo, hi);
                     }
                 } else {
@@ -363,8 +395,8 @@ __device__ __forceinline__ void conv_head_tile(const f32x16 (&acc)[MI][1], const
 template <int MI, int NI, int WN>
 __global__ __launch_bounds__(256) void k_conv3_lds(ConvIn src, const uint16_t *__restrict__ w,
                                                    const float *__restrict__ bias, void *__restrict__ out,
-                                                   float *__restrict__ part, uint16_t *__restrict__ pout, ConvHead hd, int N, int H,
-                                                   int W, int Cout,
+                                                   float *__restrict__ part, uint16_t *__restrict__ pout, ConvHead hd,
+                                                   const uint16_t *__restrict__ gate, int N, int H, int W, int Cout,
                                                    int co_store, int relu, int out_f32) {
     constexpr int WM = 4 / WN, TH = WM * MI, HR = TH + 2, HC = 34, PS = 40;
     constexpr int NPIECE = HR * HC * 4;  // 16-byte pieces of one chunk's halo
@@ -465,7 +497,7 @@ __global__ __launch_bounds__(256) void k_conv3_lds(ConvIn src, const uint16_t *_
         if (ck + 1 < ck1) swrite(buf ^ 1);
         __syncthreads();
     }
-    conv_store_tile<MI, NI>(acc, bias, out, part, N, H, W, Cout, co_store, relu, out_f32, n, x0, y0 + wm * MI, co0,
+    conv_store_tile<MI, NI>(acc, bias, out, part, gate, N, H, W, Cout, co_store, relu, out_f32, n, x0, y0 + wm * MI, co0,
                             half, l32);
     if constexpr (MI == 2 || (MI == 1 && WN == 1))
         if (pout) conv_pool_tile<MI, NI, WN>(acc, bias, pout, &lds[0][0], H, W, Cout, relu, n, x0, y0 + wm * MI, wm, co0, lane);
@@ -488,8 +520,8 @@ __global__ __launch_bounds__(256) void k_conv3_lds(ConvIn src, const uint16_t *_
 template <int MI, int NI, int WN, int KC = 32>
 __global__ __launch_bounds__(256) void k_conv3_lw(ConvIn src, const uint16_t *__restrict__ w,
                                                   const float *__restrict__ bias, void *__restrict__ out,
-                                                  float *__restrict__ part, uint16_t *__restrict__ pout, int N, int H,
-                                                   int W, int Cout,
+                                                  float *__restrict__ part, uint16_t *__restrict__ pout,
+                                                  const uint16_t *__restrict__ gate, int N, int H, int W, int Cout,
                                                   int co_store, int relu, int out_f32) {
     constexpr int WM = 4 / WN, TH = WM * MI, HR = TH + 2, HC = 34;
     constexpr int PS = KC + 8;           // element stride of a pixel / a weight row: 16 bytes of padding
@@ -596,7 +628,7 @@ __global__ __launch_bounds__(256) void k_conv3_lw(ConvIn src, const uint16_t *__
         if (ck + 1 < ck1) swrite(buf ^ 1);
         __syncthreads();
     }
-    conv_store_tile<MI, NI>(acc, bias, out, part, N, H, W, Cout, co_store, relu, out_f32, n, x0, y0 + wm * MI,
+    conv_store_tile<MI, NI>(acc, bias, out, part, gate, N, H, W, Cout, co_store, relu, out_f32, n, x0, y0 + wm * MI,
                             cb0 + wn * NI * 32, half, l32);
     if constexpr (MI == 2 || (MI == 1 && WN == 1))
         if (pout)
@@ -607,7 +639,7 @@ __global__ __launch_bounds__(256) void k_conv3_lw(ConvIn src, const uint16_t *__
 // out = act(bias + sum of the split partials), four channels per thread
 template <bool RELU, bool OUT_F32>
 __global__ void k_conv_finish(const float *__restrict__ part, const float *__restrict__ bias, void *__restrict__ out,
-                              long long n, int Cout, int splits) {
+                              const uint16_t *__restrict__ gate, long long n, int Cout, int splits) {
     const long long i = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
     if (i >= n) return;
     float4 s = *(const float4 *)(part + i);
@@ -628,7 +660,12 @@ __global__ void k_conv_finish(const float *__restrict__ part, const float *__res
     if (OUT_F32) {
         *(float4 *)((float *)out + i) = make_float4(v[0], v[1], v[2], v[3]);
     } else {
-        const uint32_t lo = f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16), hi = f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
+        uint32_t lo = f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16), hi = f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
+        if (gate) {
+            const uint2 y = *(const uint2 *)(gate + i);
+            lo = gate2(lo, y.x);
+            hi = gate2(hi, y.y);
+        }
         *(uint2 *)((uint16_t *)out + i) = make_uint2(lo, hi);
     }
 }
@@ -885,12 +922,6 @@ __global__ void k_flip_transpose(const uint16_t *__restrict__ w, uint16_t *__res
     wt[i] = w[((size_t)(taps - 1 - tp) * Cout + co) * Cin + ci];
 }
 
-// gradient through ReLU: g *= (y > 0)
-__global__ void k_relu_bwd(uint16_t *__restrict__ g, const uint16_t *__restrict__ y, size_t n) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n && !(bf2f(y[i]) > 0.0f)) g[i] = 0;
-}
-
 // 2x2 average pool, NHWC, eight channels per thread
 __global__ void k_pool2(const uint16_t *__restrict__ in, uint16_t *__restrict__ out, int N, int H, int W, int C) {
     const size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * 8;
@@ -912,9 +943,10 @@ __global__ void k_pool2(const uint16_t *__restrict__ in, uint16_t *__restrict__ 
 
 // Gradient of a convolution input built as [up2(a) | b] (see ConvIn):
 // ga[q] = sum of gk's first ca channels over the 2x2 fine pixels of coarse pixel
-// q; gb[p] = gk's last cb channels.  H, W: the fine size; eight channels per thread.
-__global__ void k_split_up(const uint16_t *__restrict__ gk, uint16_t *__restrict__ ga, uint16_t *__restrict__ gb,
-                           int N, int H, int W, int ca, int cb) {
+// q, through a's ReLU (ya: its activation); gb[p] = gk's last cb channels.  H, W:
+// the fine size; eight channels per thread.
+__global__ void k_split_up(const uint16_t *__restrict__ gk, const uint16_t *__restrict__ ya, uint16_t *__restrict__ ga,
+                           uint16_t *__restrict__ gb, int N, int H, int W, int ca, int cb) {
     const size_t t = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * 8;
     const size_t na = (size_t)N * (H / 2) * (W / 2) * ca, nb = (size_t)N * H * W * cb;
     const int C = ca + cb;
@@ -930,6 +962,9 @@ __global__ void k_split_up(const uint16_t *__restrict__ gk, uint16_t *__restrict
         u16x8 o;
 #pragma unroll
         for (int k = 0; k < 8; ++k) o[k] = f2bf((bf2f(v0[k]) + bf2f(v1[k])) + (bf2f(v2[k]) + bf2f(v3[k])));
+        const u16x8 y8 = *(const u16x8 *)(ya + t);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) o[k] = positive(y8[k]) ? o[k] : 0;
         *(u16x8 *)(ga + t) = o;
     } else if (t - na < nb) {
         const size_t j = t - na;
@@ -938,40 +973,89 @@ __global__ void k_split_up(const uint16_t *__restrict__ gk, uint16_t *__restrict
     }
 }
 
-// gin (+)= the pool gradient; H, W: the input (fine) size
-__global__ void k_pool2_bwd(const uint16_t *__restrict__ gout, uint16_t *__restrict__ gin, int N, int H, int W, int C,
-                            int accumulate) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+// gin = (gin + the pool gradient) through the ReLU of the pooled activation y;
+// H, W: the input (fine) size; eight channels per thread (36 -> 12 us a layer,
+// the ReLU's own pass gone)
+__global__ void k_pool2_bwd(const uint16_t *__restrict__ gout, const uint16_t *__restrict__ y,
+                            uint16_t *__restrict__ gin, int N, int H, int W, int C) {
+    const size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * 8;
     if (i >= (size_t)N * H * W * C) return;
     const int c = (int)(i % C);
     const size_t q = i / C;
-    const int x = (int)(q % W), y = (int)((q / W) % H);
+    const int x = (int)(q % W), yy = (int)((q / W) % H);
     const size_t n = q / ((size_t)W * H);
-    float v = 0.25f * bf2f(gout[((n * (H / 2) + y / 2) * (W / 2) + x / 2) * C + c]);
-    if (accumulate) v += bf2f(gin[i]);
-    gin[i] = f2bf(v);
+    const u16x8 g8 = *(const u16x8 *)(gout + ((n * (H / 2) + yy / 2) * (W / 2) + x / 2) * C + c);
+    const u16x8 y8 = *(const u16x8 *)(y + i), o8 = *(const u16x8 *)(gin + i);
+    u16x8 r;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) r[k] = positive(y8[k]) ? f2bf(0.25f * bf2f(g8[k]) + bf2f(o8[k])) : 0;
+    *(u16x8 *)(gin + i) = r;
 }
 
-// masked mean-square loss on the first three output channels and its gradient:
-// loss = sum_p wm[p] sum_{c<3} (out[p][c] - tgt[p][c])^2 / sum_p wm[p]
-__global__ void k_mse(const float *__restrict__ out, const float *__restrict__ tgt, const float *__restrict__ wm,
-                      uint16_t *__restrict__ gout, float *__restrict__ loss, long long P, int C, float inv_wsum) {
-    const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+// Sum of the loss weights in double, block by block, then its reciprocal:
+// sums[0] the sum, *inv = 1 / sum rounded once.  (Added up on the host the sum
+// of 524288 weights took 0.6 ms before the GPU had anything to do.)
+constexpr int kSumBlocks = 256;
+__global__ __launch_bounds__(256) void k_weight_sum(const float *__restrict__ wm, double *__restrict__ part, size_t n) {
+    double s = 0.0;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)kSumBlocks * 256) s += wm[i];
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    __shared__ double red[4];
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) part[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+}
+__global__ __launch_bounds__(kSumBlocks) void k_weight_inverse(const double *__restrict__ part,
+                                                               double *__restrict__ sum, float *__restrict__ inv,
+                                                               float *__restrict__ loss) {
+    double s = part[threadIdx.x];
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    __shared__ double red[kSumBlocks / 64];
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const double t = (red[0] + red[1]) + (red[2] + red[3]);
+        *sum = t;
+        *inv = (float)(1.0 / t);
+        *loss = 0.0f;
+    }
+}
+
+// masked mean-square loss on the first three of 32 output channels and its
+// gradient: loss = sum_p wm[p] sum_{c<3} (out[p][c] - tgt[p][c])^2 / sum_p wm[p].
+// Four threads a pixel, each one 16-byte store of the gradient's 32 channels;
+// kMseBlocks blocks walk over the pixels and end in one atomic each.  (Channel by
+// channel a thread wrote two bytes at a time, and an atomic a wave on the one
+// address of the loss took most of 122 us for 524288 pixels; now 25.)
+constexpr int kMseBlocks = 512;
+__global__ __launch_bounds__(256) void k_mse(const float *__restrict__ out, const float *__restrict__ tgt,
+                                             const float *__restrict__ wm, uint16_t *__restrict__ gout,
+                                             float *__restrict__ loss, long long P,
+                                             const float *__restrict__ inv_wsum) {
+    const float inv = *inv_wsum;
     float l = 0.0f;
-    if (p < P) {
-        const float w = wm[p];
-        for (int c = 0; c < C; ++c) {
-            float gv = 0.0f;
-            if (c < 3) {
-                const float d = out[p * C + c] - tgt[p * 3 + c];
+    for (long long t = (long long)blockIdx.x * 256 + threadIdx.x; t < 4 * P; t += (long long)gridDim.x * 256) {
+        const long long p = t >> 2;
+        const int part = (int)(t & 3);
+        u16x8 g = u16x8{};
+        if (part == 0) {
+            const float w = wm[p];
+            const float4 o = *(const float4 *)(out + p * 32);
+            const float v[3] = {o.x, o.y, o.z};
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const float d = v[c] - tgt[p * 3 + c];
                 l += w * d * d;
-                gv = 2.0f * w * d * inv_wsum;
+                g[c] = f2bf(2.0f * w * d * inv);
             }
-            gout[p * C + c] = f2bf(gv);
         }
+        *(u16x8 *)(gout + p * 32 + 8 * part) = g;
     }
     for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off, 64);
-    if ((threadIdx.x & 63) == 0) atomicAdd(loss, l * inv_wsum);
+    __shared__ float red[4];
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = l;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(loss, ((red[0] + red[1]) + (red[2] + red[3])) * inv);
 }
 
 // network input from host fields: x[p] = (the kNetIn host channels, then zeros)
@@ -1146,24 +1230,30 @@ size_t conv_split_elems(int ks, long long P, int N, int H, int W, int Cin, int C
 // k_conv3_lw (conv3_plan), 1x1 on k_conv1x1.  Only channels co < co_store are
 // stored (all of them when the K split is taken).  pool_out: also the output's
 // 2 x 2 average pool; head: also a 1x1 head on the output (ConvHead); both in
-// the epilogue where the block shape allows, else as passes of their own.
+// the epilogue where the block shape allows, else as passes of their own.  gate:
+// see conv_store_tile.
 void conv_fwd(hipStream_t s, int ks, const ConvIn &in, const uint16_t *w, const float *bias, void *out, int N, int H,
               int W, int Cout, bool relu, bool out_f32, int co_store, float *ws, size_t ws_elems,
-              ConvTile force = ConvTile{}, uint16_t *pool_out = nullptr, ConvHead head = ConvHead{}) {
+              ConvTile force = ConvTile{}, uint16_t *pool_out = nullptr, ConvHead head = ConvHead{},
+              const uint16_t *gate = nullptr) {
     const long long P = (long long)N * H * W;
     const int Cin = in.ca + in.cb;
     ucheck(W % 32 == 0 && in.ca % 32 == 0 && in.cb % 32 == 0 && Cin > 0 && Cout % 32 == 0,
            "convolution shape: W, channel counts must be multiples of 32");
     ucheck(!in.a_up || H % 2 == 0, "upsampled input needs an even height");
+    ucheck(!gate || (!out_f32 && !relu && co_store == Cout && ((uintptr_t)gate & 7) == 0),
+           "gate: a whole bf16 gradient's activation");
     if (ks == 1) {
         ucheck(!in.a_up && in.cb == 0 && !pool_out && !head.w, "1x1 convolutions take one plain input only");
+        ucheck(((uintptr_t)bias & 15) == 0 && ((uintptr_t)out & (out_f32 ? 15 : 7)) == 0,
+               "convolution buffers must be 16-byte aligned (8 for bf16 outputs)");
         int mi = 1, ni = 1;
         if (P % 64 == 0 && P / 64 * (Cout / 32) >= 4096) mi = 2;
         else if (Cout % 64 == 0 && P / 32 * (Cout / 64) >= 4096) ni = 2;
         const dim3 grid((unsigned)((P + 128 * mi - 1) / (128 * mi)), (unsigned)(Cout / (32 * ni)), 1);
 #define K1(MI, NI, R, F)                                                                                     \
     hipLaunchKernelGGL((k_conv1x1<MI, NI, R, F>), grid, dim3(256), 0, s, in.a, w, bias, out, P, Cin, Cout, \
-                       co_store)
+                       co_store, gate)
 #define PICK(R, F)                       \
     do {                                 \
         if (mi == 2) K1(2, 1, R, F);     \
@@ -1218,14 +1308,14 @@ void conv_fwd(hipStream_t s, int ks, const ConvIn &in, const uint16_t *w, const 
 #define L3(MI, NI, WN)                                                                                             \
     do {                                                                                                           \
         if (kind == 2)                                                                                             \
-            hipLaunchKernelGGL((k_conv3_lw<1, 1, 1, 64>), grid, dim3(256), 0, s, in, w, bias, out, ws, pout, N, H, \
-                               W, Cout, co_store, r, f);                                                           \
+            hipLaunchKernelGGL((k_conv3_lw<1, 1, 1, 64>), grid, dim3(256), 0, s, in, w, bias, out, ws, pout, gate, N, \
+                               H, W, Cout, co_store, r, f);                                                           \
         else if (kind == 1 && 32 * (NI) * (WN) <= 64)                                                              \
             hipLaunchKernelGGL((k_conv3_lw<MI, NI, (32 * NI * WN <= 64 ? WN : 1)>), grid, dim3(256), 0, s, in, w,   \
-                               bias, out, ws, pout, N, H, W, Cout, co_store, r, f);                                \
+                               bias, out, ws, pout, gate, N, H, W, Cout, co_store, r, f);                                \
         else                                                                                                       \
-            hipLaunchKernelGGL((k_conv3_lds<MI, NI, WN>), grid, dim3(256), 0, s, in, w, bias, out, ws, pout, hd, N, \
-                               H, W, Cout, co_store, r, f);                                                        \
+            hipLaunchKernelGGL((k_conv3_lds<MI, NI, WN>), grid, dim3(256), 0, s, in, w, bias, out, ws, pout, hd, gate, \
+                               N, H, W, Cout, co_store, r, f);                                                        \
     } while (0)
     switch (t) {
         case 0: L3(1, 1, 1); break;
@@ -1248,11 +1338,11 @@ void conv_fwd(hipStream_t s, int ks, const ConvIn &in, const uint16_t *w, const 
         const long long n = P * Cout;
         const dim3 fg(nblk((size_t)(n / 4)));
         if (out_f32)
-            hipLaunchKernelGGL((k_conv_finish<false, true>), fg, dim3(256), 0, s, ws, bias, out, n, Cout, pl.split);
+            hipLaunchKernelGGL((k_conv_finish<false, true>), fg, dim3(256), 0, s, ws, bias, out, gate, n, Cout, pl.split);
         else if (relu)
-            hipLaunchKernelGGL((k_conv_finish<true, false>), fg, dim3(256), 0, s, ws, bias, out, n, Cout, pl.split);
+            hipLaunchKernelGGL((k_conv_finish<true, false>), fg, dim3(256), 0, s, ws, bias, out, gate, n, Cout, pl.split);
         else
-            hipLaunchKernelGGL((k_conv_finish<false, false>), fg, dim3(256), 0, s, ws, bias, out, n, Cout, pl.split);
+            hipLaunchKernelGGL((k_conv_finish<false, false>), fg, dim3(256), 0, s, ws, bias, out, gate, n, Cout, pl.split);
         HIPCHK(hipGetLastError());
     }
     if (pool_out && !fuse_pool) {
@@ -1353,7 +1443,8 @@ struct lbm_unet {
     size_t nparam = 0, nweight = 0;
     float *w32 = nullptr, *m = nullptr, *v = nullptr, *g32 = nullptr;
     uint16_t *wb = nullptr, *wt = nullptr;
-    float *out32 = nullptr, *tgt = nullptr, *wm = nullptr, *fields = nullptr, *loss = nullptr;
+    float *out32 = nullptr, *tgt = nullptr, *wm = nullptr, *fields = nullptr, *loss = nullptr, *inv_wsum = nullptr;
+    double *wsums = nullptr;  // partial sums of the loss weights, then their sum
     uint16_t *gout = nullptr;
     Act x, e1a, e1, p1, e2a, e2, p2, e3a, e3, p3, e4a, e4, d3u, k3, d3a, d3, d2u, k2, d2a, d2, d1u, k1, d1a, d1;
     float *ws = nullptr;  // split-K partial sums
@@ -1468,6 +1559,8 @@ struct lbm_unet {
         wm = (float *)alloc(P * 4);
         fields = (float *)alloc(P * 8 * 4);
         loss = (float *)alloc(4);
+        inv_wsum = (float *)alloc(4);
+        wsums = (double *)alloc((kSumBlocks + 1) * sizeof(double));
         // split-K workspace: the largest need over the forward and input-gradient convolutions
         for (const Conv &c : convs) {
             // level of the layer from its output (forward) / input (gradient) channel count
@@ -1574,73 +1667,60 @@ struct lbm_unet {
         HIPCHK(hipGetLastError());
     }
 
-    // gradients of conv i: weights and bias into g32; input gradient into gin (if any)
-    void bwd_conv(int i, const ConvIn &in, int h, int w, const uint16_t *gout_, uint16_t *gin) {
+    // gradients of conv i: weights and bias into g32; input gradient into gin
+    // (if any), through the ReLU of the activation `gate` (if any)
+    void bwd_conv(int i, const ConvIn &in, int h, int w, const uint16_t *gout_, uint16_t *gin,
+                  const uint16_t *gate = nullptr) {
         const Conv &c = convs[i];
         conv_wgrad(stream, c.ks, in, gout_, g32 + c.woff, true, B, h, w, c.cout, wgrad_ws, wgrad_ws_elems);
         if (gin)
             conv_fwd(stream, c.ks, one_input(gout_, c.cout), wt + c.wboff, nullptr, gin, B, h, w, c.cin, false, false,
-                     c.cin, ws, ws_elems);
+                     c.cin, ws, ws_elems, ConvTile{}, nullptr, ConvHead{}, gate);
     }
-    void bwd_conv(int i, const Act &in, const uint16_t *gout_, uint16_t *gin) {
-        bwd_conv(i, one_input(in.a, in.C), in.H, in.W, gout_, gin);
+    // into the gradient of the layer's input, through that input's ReLU
+    void bwd_conv(int i, const Act &in, const uint16_t *gout_) {
+        bwd_conv(i, one_input(in.a, in.C), in.H, in.W, gout_, in.g, in.a);
     }
-    void relu_bwd(const Act &t) {
-        hipLaunchKernelGGL(k_relu_bwd, dim3(nblk(t.n())), dim3(256), 0, stream, t.g, t.a, t.n());
+    // into the gradient of a pooled layer (no ReLU of its own)
+    void bwd_conv_pooled(int i, const Act &in, const uint16_t *gout_) {
+        bwd_conv(i, one_input(in.a, in.C), in.H, in.W, gout_, in.g);
     }
-    // gradient of [up2(coarse) | fine] -> coarse.g (assigned), fine.g (assigned)
+    // gradient of [up2(coarse) | fine] -> coarse.g (assigned, through its ReLU), fine.g (assigned)
     void split_up(const Act &k, const Act &coarse, const Act &fine) {
         const size_t n = coarse.n() + fine.n();
-        hipLaunchKernelGGL(k_split_up, dim3(nblk(n / 8)), dim3(256), 0, stream, k.g, coarse.g, fine.g, B, k.H, k.W,
-                           coarse.C, fine.C);
+        hipLaunchKernelGGL(k_split_up, dim3(nblk(n / 8)), dim3(256), 0, stream, k.g, coarse.a, coarse.g, fine.g, B, k.H,
+                           k.W, coarse.C, fine.C);
     }
-    void pool_bwd(const Act &coarse, const Act &fine) {  // accumulates into fine.g
-        hipLaunchKernelGGL(k_pool2_bwd, dim3(nblk(fine.n())), dim3(256), 0, stream, coarse.g, fine.g, B, fine.H,
-                           fine.W, fine.C, 1);
+    void pool_bwd(const Act &coarse, const Act &fine) {  // accumulates into fine.g, then fine's ReLU
+        hipLaunchKernelGGL(k_pool2_bwd, dim3(nblk(fine.n() / 8)), dim3(256), 0, stream, coarse.g, fine.a, fine.g, B,
+                           fine.H, fine.W, fine.C);
     }
 
     void backward() {
-        bwd_conv(17, d1, gout, d1.g);
-        relu_bwd(d1);
-        bwd_conv(16, d1a, d1.g, d1a.g);
-        relu_bwd(d1a);
+        bwd_conv(17, d1, gout);
+        bwd_conv(16, d1a, d1.g);
         bwd_conv(15, cat_up(d1u, e1), H, W, d1a.g, k1.g);
         split_up(k1, d1u, e1);
-        relu_bwd(d1u);
-        bwd_conv(14, d2, d1u.g, d2.g);
-        relu_bwd(d2);
-        bwd_conv(13, d2a, d2.g, d2a.g);
-        relu_bwd(d2a);
+        bwd_conv(14, d2, d1u.g);
+        bwd_conv(13, d2a, d2.g);
         bwd_conv(12, cat_up(d2u, e2), e2.H, e2.W, d2a.g, k2.g);
         split_up(k2, d2u, e2);
-        relu_bwd(d2u);
-        bwd_conv(11, d3, d2u.g, d3.g);
-        relu_bwd(d3);
-        bwd_conv(10, d3a, d3.g, d3a.g);
-        relu_bwd(d3a);
+        bwd_conv(11, d3, d2u.g);
+        bwd_conv(10, d3a, d3.g);
         bwd_conv(9, cat_up(d3u, e3), e3.H, e3.W, d3a.g, k3.g);
         split_up(k3, d3u, e3);
-        relu_bwd(d3u);
-        bwd_conv(8, e4, d3u.g, e4.g);
-        relu_bwd(e4);
-        bwd_conv(7, e4a, e4.g, e4a.g);
-        relu_bwd(e4a);
-        bwd_conv(6, p3, e4a.g, p3.g);
+        bwd_conv(8, e4, d3u.g);
+        bwd_conv(7, e4a, e4.g);
+        bwd_conv_pooled(6, p3, e4a.g);
         pool_bwd(p3, e3);
-        relu_bwd(e3);
-        bwd_conv(5, e3a, e3.g, e3a.g);
-        relu_bwd(e3a);
-        bwd_conv(4, p2, e3a.g, p2.g);
+        bwd_conv(5, e3a, e3.g);
+        bwd_conv_pooled(4, p2, e3a.g);
         pool_bwd(p2, e2);
-        relu_bwd(e2);
-        bwd_conv(3, e2a, e2.g, e2a.g);
-        relu_bwd(e2a);
-        bwd_conv(2, p1, e2a.g, p1.g);
+        bwd_conv(3, e2a, e2.g);
+        bwd_conv_pooled(2, p1, e2a.g);
         pool_bwd(p1, e1);
-        relu_bwd(e1);
-        bwd_conv(1, e1a, e1.g, e1a.g);
-        relu_bwd(e1a);
-        bwd_conv(0, x, e1a.g, nullptr);
+        bwd_conv(1, e1a, e1.g);
+        bwd_conv(0, one_input(x.a, x.C), H, W, e1a.g, nullptr);
         HIPCHK(hipGetLastError());
     }
 
@@ -1650,19 +1730,21 @@ struct lbm_unet {
         HIPCHK(hipMemcpyAsync(fields, hx, P * 32, hipMemcpyHostToDevice, stream));
         HIPCHK(hipMemcpyAsync(tgt, hy, P * 12, hipMemcpyHostToDevice, stream));
         HIPCHK(hipMemcpyAsync(wm, hwm, P * 4, hipMemcpyHostToDevice, stream));
-        double wsum = 0.0;
-        for (size_t i = 0; i < P; ++i) wsum += hwm[i];
-        ucheck(wsum > 0.0, "loss weights sum to zero");
         hipLaunchKernelGGL(k_pack_input, dim3(nblk(P)), dim3(256), 0, stream, fields, x.a, (long long)P, 32);
         forward();
-        HIPCHK(hipMemsetAsync(loss, 0, 4, stream));
-        hipLaunchKernelGGL(k_mse, dim3(nblk(P)), dim3(256), 0, stream, out32, tgt, wm, gout, loss, (long long)P, 32,
-                           (float)(1.0 / wsum));
+        hipLaunchKernelGGL(k_weight_sum, dim3(kSumBlocks), dim3(256), 0, stream, wm, wsums, P);
+        hipLaunchKernelGGL(k_weight_inverse, dim3(1), dim3(kSumBlocks), 0, stream, wsums, wsums + kSumBlocks, inv_wsum,
+                           loss);
+        hipLaunchKernelGGL(k_mse, dim3(std::min<unsigned>(kMseBlocks, nblk(4 * P))), dim3(256), 0, stream, out32, tgt, wm, gout, loss, (long long)P,
+                           inv_wsum);
         HIPCHK(hipGetLastError());
         backward();
         float l = 0.0f;
+        double wsum = 0.0;
         HIPCHK(hipMemcpyAsync(&l, loss, 4, hipMemcpyDeviceToHost, stream));
+        HIPCHK(hipMemcpyAsync(&wsum, wsums + kSumBlocks, 8, hipMemcpyDeviceToHost, stream));
         HIPCHK(hipStreamSynchronize(stream));
+        ucheck(wsum > 0.0, "loss weights sum to zero");
         return l;
     }
 

@@ -41,3 +41,35 @@ def test_head_bias_gradient(B, H):
     bound = B * H * 256 * 2.0 ** -24 * np.abs(gout).sum((0, 1, 2))
     assert (np.abs(grads[-32:-29] - gout.sum((0, 1, 2))) <= bound).all()
     assert not grads[-29:].any()
+
+
+def test_minibatch_gradient_is_the_mean_of_its_images():
+    """Loss and gradients of two images are the means of each image's own (equal
+    weight sums), at a height that leaves one row at the coarsest level; the two
+    runs split their sums differently, and bf16 rounding of the loss gradient
+    (scaled by the weight sum, here a power of two apart) is the same in both."""
+    from lbm_amd.surrogate import UNet
+    print("case: minibatch gradient", flush=True)
+    rng = np.random.default_rng(3)
+    one, two = UNet(1, 8, 256, seed=9), UNet(2, 8, 256, seed=9)
+    x = rng.standard_normal((2, 8, 256, 8)).astype(np.float32)
+    t = rng.standard_normal((2, 8, 256, 3)).astype(np.float32)
+    w = np.ones((2, 8, 256), np.float32)
+    loss, grad = two.loss_grad(x, t, w)
+    single = [one.loss_grad(x[i:i + 1], t[i:i + 1], w[i:i + 1]) for i in range(2)]
+    mean = (single[0][1].astype(np.float64) + single[1][1]) / 2
+    assert abs(loss - (single[0][0] + single[1][0]) / 2) < 1e-5 * loss
+    assert np.linalg.norm(grad - mean) < 1e-5 * np.linalg.norm(mean)
+
+
+def test_zero_loss_weights_are_refused():
+    from lbm_amd._native import LbmError, LBM_EINVAL
+    from lbm_amd.surrogate import UNet
+    print("case: zero loss weights", flush=True)
+    net = UNet(1, 8, 256, seed=2)
+    before = net.get_params()
+    x, t = np.zeros((1, 8, 256, 8), np.float32), np.zeros((1, 8, 256, 3), np.float32)
+    with pytest.raises(LbmError) as e:
+        net.train_step(x, t, np.zeros((1, 8, 256), np.float32), 1e-3)
+    assert e.value.code == LBM_EINVAL
+    assert np.array_equal(net.get_params(), before)
