@@ -31,6 +31,7 @@
 #include <vector>
 
 #include "lbm_common.h"
+#include "staging.h"
 #include "tune_cache.h"
 #include "tile.h"
 
@@ -162,6 +163,7 @@ struct lbm_batch {
     float *lag = nullptr;  // per domain 3 moment planes at 3 * aux_off
     float *dense = nullptr;
     size_t dense_elems = 0;
+    Staging staging;
     DomainDev *dtable = nullptr;
     uint2 *ilist = nullptr, *blist = nullptr, *alist = nullptr;
     uint32_t n_interior = 0, n_boundary = 0, n_all = 0;
@@ -199,6 +201,7 @@ struct lbm_batch {
     void release() {
         (void)hipSetDevice(dev);
         drop_graphs();
+        staging.release();
         release_spare();
         for (void *p : {f[0], f[1], (void *)starts, (void *)mask, (void *)flags, (void *)segs, (void *)lag, (void *)dense,
                         (void *)dtable, (void *)ilist, (void *)blist, (void *)alist})
@@ -819,11 +822,14 @@ int lbm_batch_autotune(lbm_batch *b, uint32_t steps, int *best, float *ms) {
                 }
                 b->variant = v;
                 b->step(4);  // builds lists and graphs, leaves P-form; the fewest steps k_batch_tile runs from there
+                // (k_batch_tile over enough steps for the launches of a long call)
+                const uint32_t timed = lbm_batch::tile_variant(v) ? std::max(steps, kTileTimedSteps) : steps;
                 HIPCHK(hipEventRecord(e0, b->stream));
-                b->step(steps);
+                b->step(timed);
                 HIPCHK(hipEventRecord(e1, b->stream));
                 HIPCHK(hipEventSynchronize(e1));
                 HIPCHK(hipEventElapsedTime(&t[v], e0, e1));
+                t[v] *= (float)steps / (float)timed;
                 if (t[v] < t[v_best]) v_best = v;
             }
             (void)hipEventDestroy(e0);
@@ -933,17 +939,18 @@ int lbm_batch_read_moments(lbm_batch *b, uint32_t d, float *jx, float *jy, float
                                b->dense, dd.g.X, dd.g.Y, dd.g.pitch, dd.g.pstride);
             HIPCHK(hipGetLastError());
         }
+        Piece p[3];
+        int np = 0;
         for (int c = 0; c < 3; ++c) {
             if (!dst[c]) continue;
             if (packed || staged)
-                HIPCHK(hipMemcpyAsync(dst[c], staged ? b->dense + c * dn : base + c * dd.g.pstride,
-                                      dn * sizeof(float), hipMemcpyDeviceToHost, b->stream));
+                p[np++] = {dst[c], (void *)(staged ? b->dense + c * dn : base + c * dd.g.pstride), dn * sizeof(float)};
             else
                 HIPCHK(hipMemcpy2DAsync(dst[c], sizeof(float) * dd.g.X, base + c * dd.g.pstride,
                                         sizeof(float) * dd.g.pitch, sizeof(float) * dd.g.X, dd.g.Y,
                                         hipMemcpyDeviceToHost, b->stream));
         }
-        HIPCHK(hipStreamSynchronize(b->stream));
+        HIPCHK(b->staging.copy(b->dev, b->stream, p, np, true));
     });
 }
 

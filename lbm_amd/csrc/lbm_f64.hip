@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "../../include/lbm_hip.h"
+#include "staging.h"
 
 namespace {
 
@@ -202,10 +203,12 @@ struct lbm_f64 {
     double *f = nullptr, *g = nullptr, *scratch = nullptr;
     uint8_t *solid = nullptr;
     uint64_t steps = 0;
+    Staging staging;
 
     size_t n() const { return (size_t)X * Y; }
     void release() {
         (void)hipSetDevice(dev);
+        staging.release();
         for (void *p : {(void *)f, (void *)g, (void *)scratch, (void *)solid})
             if (p) (void)hipFree(p);
         f = g = scratch = nullptr;
@@ -365,10 +368,11 @@ int lbm_f64_macro(lbm_f64 *h, double *rho, double *ux, double *uy) {
                            n);
         H64(hipGetLastError());
         double *dst[3] = {rho, ux, uy};
+        Piece p[3];
+        int np = 0;
         for (int c = 0; c < 3; ++c)
-            if (dst[c]) H64(hipMemcpyAsync(dst[c], h->scratch + c * n, n * sizeof(double), hipMemcpyDeviceToHost,
-                                           h->stream));
-        H64(hipStreamSynchronize(h->stream));
+            if (dst[c]) p[np++] = {dst[c], h->scratch + c * n, n * sizeof(double)};
+        H64(h->staging.copy(h->dev, h->stream, p, np, true));
     });
 }
 
@@ -376,8 +380,8 @@ int lbm_f64_read_f(lbm_f64 *h, double *f9) {
     return fguard([&] {
         fcheck(h && f9, "null argument");
         H64(hipSetDevice(h->dev));
-        H64(hipMemcpyAsync(f9, h->f, 9 * h->n() * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-        H64(hipStreamSynchronize(h->stream));
+        const Piece p{f9, h->f, 9 * h->n() * sizeof(double)};
+        H64(h->staging.copy(h->dev, h->stream, &p, 1, true));
     });
 }
 

@@ -49,6 +49,7 @@
 #include <vector>
 
 #include "lbm_common.h"
+#include "staging.h"
 #include "tune_cache.h"
 #include "tile.h"
 
@@ -271,6 +272,9 @@ struct lbm_grid {
     float *out = nullptr;   // summary output plane (persistent)
     float *dense = nullptr; // dense f32 staging (dense_planes planes)
     int dense_planes = 0;
+    Staging staging;
+    void to_host(const Piece *p, int n) { HIPCHK(staging.copy(dev, stream, p, n, true)); }
+    void to_device(const Piece *p, int n) { HIPCHK(staging.copy(dev, stream, p, n, false)); }
     float *rgb = nullptr;   // colour-map output (3 floats per cell), allocated on first use
     size_t rgb_elems = 0;
     double *partials = nullptr;
@@ -314,6 +318,7 @@ struct lbm_grid {
 
     void release() {
         (void)hipSetDevice(dev);
+        staging.release();
         for (void *p : {f[0], f[1], spare[0], spare[1], (void *)mask, (void *)flags, (void *)lag,
                         (void *)now, (void *)out, (void *)dense, (void *)partials, (void *)sums,
                         (void *)snap, (void *)umark, (void *)vpart})
@@ -596,13 +601,14 @@ struct lbm_grid {
                                dense, geom, k);
         });
         HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpyAsync(host, dense, sizeof(float) * X * Y, hipMemcpyDeviceToHost, stream));
-        HIPCHK(hipStreamSynchronize(stream));
+        const Piece p{host, dense, sizeof(float) * X * Y};
+        to_host(&p, 1);
     }
 
     void copy_plane_in(const float *host, void *dev_plane, int k) {
         ensure_dense(1);
-        HIPCHK(hipMemcpyAsync(dense, host, sizeof(float) * X * Y, hipMemcpyHostToDevice, stream));
+        const Piece p{(void *)host, dense, sizeof(float) * X * Y};
+        to_device(&p, 1);
         dim3 grid((X + 255) / 256, Y);
         by_store(precision, [&]<class St>() {
             hipLaunchKernelGGL(k_encode_plane<St>, grid, dim3(256), 0, stream, dense, (typename St::T *)dev_plane,
@@ -638,16 +644,18 @@ struct lbm_grid {
                                (int)Y, geom.pitch, geom.pstride);
             HIPCHK(hipGetLastError());
         }
+        Piece p[3];
+        int np = 0;
         for (int i = 0; i < n; ++i) {
             if (!host[i]) continue;
             const float *src = dev + (size_t)i * geom.pstride;
-            if (packed) HIPCHK(hipMemcpyAsync(host[i], src, bytes, hipMemcpyDeviceToHost, stream));
-            else if (dense)
-                HIPCHK(hipMemcpyAsync(host[i], dense + (size_t)i * X * Y, bytes, hipMemcpyDeviceToHost, stream));
+            if (packed || dense)
+                p[np++] = {host[i], packed ? (void *)src : (void *)(dense + (size_t)i * X * Y), bytes};
             else
                 HIPCHK(hipMemcpy2DAsync(host[i], sizeof(float) * X, src, sizeof(float) * geom.pitch,
                                         sizeof(float) * X, Y, hipMemcpyDeviceToHost, stream));
         }
+        to_host(p, np);
     }
 };
 
@@ -1035,11 +1043,14 @@ int lbm_autotune(lbm_grid *g, uint32_t steps, int *best, float *ms) {
                 // warm-up (and leaves the grid in P-form); four steps: the
                 // fewest that k_tile runs from there
                 g->step(4);
+                // (k_tile over enough steps for the launches of a long call)
+                const uint32_t timed = g->tile_variant(v) ? std::max(steps, kTileTimedSteps) : steps;
                 HIPCHK(hipEventRecord(e0, g->stream));
-                g->step(steps);
+                g->step(timed);
                 HIPCHK(hipEventRecord(e1, g->stream));
                 HIPCHK(hipEventSynchronize(e1));
                 HIPCHK(hipEventElapsedTime(&t[v], e0, e1));
+                t[v] *= (float)steps / (float)timed;
                 if (t[v] < t[v_best]) v_best = v;
             }
             (void)hipEventDestroy(e0);
@@ -1276,10 +1287,11 @@ int lbm_read_fields(lbm_grid *g, float *rho, float *ux, float *uy, float *curl, 
         HIPCHK(hipGetLastError());
         const size_t dn = (size_t)g->X * g->Y;
         float *dst[4] = {rho, ux, uy, curl};
+        Piece p[4];
+        int np = 0;
         for (int i = 0; i < 4; ++i)
-            if (dst[i])
-                HIPCHK(hipMemcpyAsync(dst[i], g->dense + i * dn, sizeof(float) * dn, hipMemcpyDeviceToHost, g->stream));
-        HIPCHK(hipStreamSynchronize(g->stream));
+            if (dst[i]) p[np++] = {dst[i], g->dense + i * dn, sizeof(float) * dn};
+        g->to_host(p, np);
     });
 }
 
@@ -1291,11 +1303,10 @@ int lbm_summary(lbm_grid *g, int kind, float *out) {
         hipLaunchKernelGGL(k_summary, dim3((g->X + 255) / 256, g->Y), dim3(256), 0, g->stream, g->lag, g->out, g->mask,
                            (float *)nullptr, dense, g->geom, kind, 0);
         HIPCHK(hipGetLastError());
-        if (dense)
-            HIPCHK(hipMemcpyAsync(out, dense, sizeof(float) * g->X * g->Y, hipMemcpyDeviceToHost, g->stream));
-        else if (out)
-            g->copy_f32_planes_out(g->out, &out, 1);
-        HIPCHK(hipStreamSynchronize(g->stream));
+        const Piece p{out, dense, sizeof(float) * g->X * g->Y};
+        if (dense) g->to_host(&p, 1);
+        else if (out) g->copy_f32_planes_out(g->out, &out, 1);
+        else HIPCHK(hipStreamSynchronize(g->stream));
     });
 }
 
@@ -1314,8 +1325,8 @@ int lbm_render(lbm_grid *g, int kind, int colormap, float *rgb) {
         hipLaunchKernelGGL(k_summary, dim3((g->X + 255) / 256, g->Y), dim3(256), 0, g->stream, g->lag, g->out, g->mask,
                            g->rgb, (float *)nullptr, g->geom, kind, colormap);
         HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpyAsync(rgb, g->rgb, n * sizeof(float), hipMemcpyDeviceToHost, g->stream));
-        HIPCHK(hipStreamSynchronize(g->stream));
+        const Piece p{rgb, g->rgb, n * sizeof(float)};
+        g->to_host(&p, 1);
     });
 }
 
@@ -1458,16 +1469,13 @@ int lbm_save_state(lbm_grid *g, void *buf, size_t bytes) {
         std::memcpy(p, &h, sizeof h);
         p += sizeof h;
         const size_t ps = (size_t)g->geom.pstride;
-        HIPCHK(hipMemcpyAsync(p, g->f[0], g->set_bytes(), hipMemcpyDeviceToHost, g->stream));
-        p += g->set_bytes();
-        HIPCHK(hipMemcpyAsync(p, g->f[1], g->set_bytes(), hipMemcpyDeviceToHost, g->stream));
-        p += g->set_bytes();
-        HIPCHK(hipMemcpyAsync(p, g->mask, ps, hipMemcpyDeviceToHost, g->stream));
-        p += ps;
-        HIPCHK(hipMemcpyAsync(p, g->lag, 3 * ps * sizeof(float), hipMemcpyDeviceToHost, g->stream));
-        p += 3 * ps * sizeof(float);
-        HIPCHK(hipMemcpyAsync(p, g->out, ps * sizeof(float), hipMemcpyDeviceToHost, g->stream));
-        HIPCHK(hipStreamSynchronize(g->stream));
+        const size_t sb = g->set_bytes();
+        const Piece pieces[5] = {{p, g->f[0], sb},
+                                 {p + sb, g->f[1], sb},
+                                 {p + 2 * sb, g->mask, ps},
+                                 {p + 2 * sb + ps, g->lag, 3 * ps * sizeof(float)},
+                                 {p + 2 * sb + ps + 3 * ps * sizeof(float), g->out, ps * sizeof(float)}};
+        g->to_host(pieces, 5);
     });
 }
 
@@ -1487,15 +1495,14 @@ int lbm_load_state(lbm_grid *g, const void *buf, size_t bytes) {
               "corrupt state image header");
         const char *p = (const char *)buf + sizeof h;
         const size_t ps = (size_t)g->geom.pstride;
-        HIPCHK(hipMemcpyAsync(g->f[0], p, g->set_bytes(), hipMemcpyHostToDevice, g->stream));
-        p += g->set_bytes();
-        HIPCHK(hipMemcpyAsync(g->f[1], p, g->set_bytes(), hipMemcpyHostToDevice, g->stream));
-        p += g->set_bytes();
-        HIPCHK(hipMemcpyAsync(g->mask, p, ps, hipMemcpyHostToDevice, g->stream));
-        p += ps;
-        HIPCHK(hipMemcpyAsync(g->lag, p, 3 * ps * sizeof(float), hipMemcpyHostToDevice, g->stream));
-        p += 3 * ps * sizeof(float);
-        HIPCHK(hipMemcpyAsync(g->out, p, ps * sizeof(float), hipMemcpyHostToDevice, g->stream));
+        char *const src = (char *)p;  // (only read)
+        const size_t sb = g->set_bytes();
+        const Piece pieces[5] = {{src, g->f[0], sb},
+                                 {src + sb, g->f[1], sb},
+                                 {src + 2 * sb, g->mask, ps},
+                                 {src + 2 * sb + ps, g->lag, 3 * ps * sizeof(float)},
+                                 {src + 2 * sb + ps + 3 * ps * sizeof(float), g->out, ps * sizeof(float)}};
+        g->to_device(pieces, 5);
         g->omega = h.omega;
         g->geom.omega = h.omega;
         g->set_inflow(h.u_in);

@@ -51,6 +51,9 @@ struct TileArgs {
 };
 
 constexpr int kTileMaxSteps = 8;
+// steps an autotuner times a tile variant for at least: launches of a few steps
+// (two of three in a call of six) say little about those of a long call
+constexpr uint32_t kTileTimedSteps = 48;
 
 // Block shapes: rows a wave, waves, where the unstreamed cells' previous
 // populations live, and the launch's cost.  Without `chain` every cell has a

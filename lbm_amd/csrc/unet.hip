@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "lbm_common.h"
+#include "staging.h"
 
 namespace {
 
@@ -1452,6 +1453,7 @@ struct lbm_unet {
     float *wgrad_ws = nullptr;  // partial sums of the weight gradients
     size_t wgrad_ws_elems = 0;
     std::vector<void *> mem;
+    Staging staging;
     int adam_t = 0;
     // the forward pass as a hipGraph (captured once; a graph runs on any stream)
     bool use_graph = true;
@@ -1499,6 +1501,7 @@ struct lbm_unet {
             used = nullptr;
         }
         drop_graph();
+        staging.release();
         for (void *p : mem) (void)hipFree(p);
         mem.clear();
         if (stream) (void)hipStreamDestroy(stream);
@@ -1727,9 +1730,8 @@ struct lbm_unet {
     // host inputs -> device; returns the loss
     float loss_and_grad(const float *hx, const float *hy, const float *hwm) {
         const size_t P = (size_t)B * H * W;
-        HIPCHK(hipMemcpyAsync(fields, hx, P * 32, hipMemcpyHostToDevice, stream));
-        HIPCHK(hipMemcpyAsync(tgt, hy, P * 12, hipMemcpyHostToDevice, stream));
-        HIPCHK(hipMemcpyAsync(wm, hwm, P * 4, hipMemcpyHostToDevice, stream));
+        const Piece in[3] = {{(void *)hx, fields, P * 32}, {(void *)hy, tgt, P * 12}, {(void *)hwm, wm, P * 4}};
+        HIPCHK(staging.copy(dev, stream, in, 3, false));
         hipLaunchKernelGGL(k_pack_input, dim3(nblk(P)), dim3(256), 0, stream, fields, x.a, (long long)P, 32);
         forward();
         hipLaunchKernelGGL(k_weight_sum, dim3(kSumBlocks), dim3(256), 0, stream, wm, wsums, P);
@@ -1882,15 +1884,15 @@ int lbm_unet_forward(lbm_unet *n, const float *x, float *y) {
         HIPCHK(hipSetDevice(n->dev));
         n->order_after_last_use(n->stream);
         const size_t P = (size_t)n->B * n->H * n->W;
-        HIPCHK(hipMemcpyAsync(n->fields, x, P * 32, hipMemcpyHostToDevice, n->stream));
+        const Piece in{(void *)x, n->fields, P * 32}, res{y, n->fields, P * 12};
+        HIPCHK(n->staging.copy(n->dev, n->stream, &in, 1, false));
         hipLaunchKernelGGL(k_pack_input, dim3(nblk(P)), dim3(256), 0, n->stream, n->fields, n->x.a, (long long)P, 32);
         n->forward();
         // through the host fields' buffer, which the pass has read
         hipLaunchKernelGGL(k_dense_output, dim3(nblk(P)), dim3(256), 0, n->stream, n->out32, n->fields, (long long)P,
                            32);
         HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpyAsync(y, n->fields, P * 12, hipMemcpyDeviceToHost, n->stream));
-        HIPCHK(hipStreamSynchronize(n->stream));
+        HIPCHK(n->staging.copy(n->dev, n->stream, &res, 1, true));
     });
 }
 
@@ -1902,8 +1904,8 @@ int lbm_unet_loss_grad(lbm_unet *n, const float *x, const float *y, const float 
         const float l = n->loss_and_grad(x, y, weights);
         if (loss) *loss = l;
         if (grad) {
-            HIPCHK(hipMemcpyAsync(grad, n->g32, n->nparam * 4, hipMemcpyDeviceToHost, n->stream));
-            HIPCHK(hipStreamSynchronize(n->stream));
+            const Piece p{grad, n->g32, n->nparam * 4};
+            HIPCHK(n->staging.copy(n->dev, n->stream, &p, 1, true));
         }
     });
 }
