@@ -459,8 +459,35 @@ __global__ __launch_bounds__(256) void k_conv3_lds(ConvIn src, const uint16_t *_
                 b[j][s2] = *(const u16x8 *)(w + ((size_t)tap * Cout + co0 + 32 * j + l32) * Cin + c0 + 16 * s2 +
                                             8 * half);
     };
+    // with one 32-channel tile a wave, a chunk's weights for all nine taps fit in
+    // registers: they are loaded with the chunk's halo, in one latency instead of
+    // nine (one tap ahead, each tap waited for L2)
+    constexpr bool kAllTaps = NI == 1;
+    [[maybe_unused]] u16x8 wt[kAllTaps ? 9 : 1][NI][2];
+    auto wload = [&](int ck) {
+        if constexpr (kAllTaps)
+#pragma unroll
+            for (int tap = 0; tap < 9; ++tap) bload(tap, ck << 5, wt[tap]);
+    };
     auto compute = [&](int buf, int ck) {
         const int c0 = ck << 5;
+        if constexpr (kAllTaps) {
+#pragma unroll
+            for (int tap = 0; tap < 9; ++tap) {
+                const int dy = tap / 3, dx = tap % 3;
+#pragma unroll
+                for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+                    for (int i = 0; i < MI; ++i) {
+                        const int r = wm * MI + i + dy;
+                        const u16x8 a = *(const u16x8 *)&lds[buf][(r * HC + l32 + dx) * PS + 16 * s2 + 8 * half];
+                        acc[i][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, wt[tap][0][s2]),
+                                                                            __builtin_bit_cast(bf16x8, a), acc[i][0], 0,
+                                                                            0, 0);
+                    }
+            }
+            return;
+        }
         u16x8 bc[NI][2], bn[NI][2];
         bload(0, c0, bc);
 #pragma unroll
@@ -489,13 +516,17 @@ __global__ __launch_bounds__(256) void k_conv3_lds(ConvIn src, const uint16_t *_
         }
     };
     gload(ck0);
+    wload(ck0);
     swrite(0);
     __syncthreads();
     for (int ck = ck0; ck < ck1; ++ck) {
         const int buf = (ck - ck0) & 1;
         if (ck + 1 < ck1) gload(ck + 1);
         compute(buf, ck);
-        if (ck + 1 < ck1) swrite(buf ^ 1);
+        if (ck + 1 < ck1) {
+            wload(ck + 1);
+            swrite(buf ^ 1);
+        }
         __syncthreads();
     }
     conv_store_tile<MI, NI>(acc, bias, out, part, gate, N, H, W, Cout, co_store, relu, out_f32, n, x0, y0 + wm * MI, co0,
