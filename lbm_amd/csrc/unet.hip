@@ -1193,62 +1193,39 @@ long long conv3_blocks(int t, int N, int H, int W, int Cout) {
     return (long long)N * ((H + th - 1) / th) * (W / 32) * (Cout / (32 * kTiles3[t][1] * kTiles3[t][2]));
 }
 
-// Block shape and split by layer shape, from timings of every shape on MI355X
-// for the network's layers (batch 1 at 512 x 1024 and batch 8 at 256 x 256):
-// few output channels favour short, single-wave-column tiles; wide layers
-// favour spreading the channels over the four waves.  A shape that leaves
-// fewer than 256 blocks (one per CU) falls back to a narrower one, then to a
-// split of the input chunks.
-ConvPlan conv3_plan(int N, int H, int W, int Cin, int Cout) {
-    // Weights staged in LDS (k_conv3_lw) on one-row-per-wave, 32-channel
-    // blocks: fastest for every layer shape of the network except 32 -> 32
-    // channels (one input chunk, where the halo-only kernel keeps twice the
-    // blocks resident); K split while the blocks cover fewer than half the
-    // CUs (at 128..255 blocks the split's extra pass costs more than it gains).
-    // Where those blocks leave at most one per CU anyway, 64-channel chunks.
-    if (!(Cin == 32 && Cout == 32)) {
-        const int kind = Cin % 64 == 0 && conv3_blocks(0, N, H, W, Cout) <= 256 ? 2 : 1;
-        int split = 1;
-        const int nck = Cin / (kind == 2 ? 64 : 32);
-        while (split < 4 && 2 * split <= nck && conv3_blocks(0, N, H, W, Cout) * split < 128) split *= 2;
-        return {0, split, kind};
-    }
-    // preference lists, indices into kTiles3
-    static const int p32a[] = {1, 0, 2};           // Cout 32, Cin 32
-    static const int p32b[] = {1, 2, 0};           // Cout 32, Cin > 32
-    static const int p64a[] = {5, 4, 0};           // Cout 64, Cin 32
-    static const int p64b[] = {4, 6, 1, 0};        // Cout 64, Cin > 32
-    static const int p128a[] = {10, 6, 1, 0};      // Cout 128, Cin <= 128
-    static const int p128b[] = {2, 10, 6, 1, 0};   // Cout 128, Cin > 128
-    static const int pwide[] = {10, 6, 1, 9, 0};   // Cout >= 256 (multiples of 128)
-    const int *list;
-    int len;
-    if (Cout == 32) {
-        list = Cin == 32 ? p32a : p32b;
-        len = 3;
-    } else if (Cout == 64) {
-        list = Cin == 32 ? p64a : p64b;
-        len = Cin == 32 ? 3 : 4;
-    } else if (Cout == 128) {
-        list = Cin <= 128 ? p128a : p128b;
-        len = Cin <= 128 ? 4 : 5;
-    } else if (Cout % 128 == 0) {
-        list = pwide;
-        len = 5;
-    } else {
-        list = p64b;  // other multiples of 32 (64 k + 32): shapes with 32 channels per block column
-        len = 4;
-    }
-    int best = -1;
-    for (int i = 0; i < len && best < 0; ++i) {
-        const int t = list[i];
-        if (Cout % (32 * kTiles3[t][1] * kTiles3[t][2]) == 0 && conv3_blocks(t, N, H, W, Cout) >= 256) best = t;
-    }
-    if (best < 0) best = 0;
+// Block shape, kernel and split by layer shape, from timings of every shape for
+// the network's layers at batches of 1, 3 and 8 (us, old choice -> this one).
+// Choices differ in how the work is laid out, not in the order of an output's
+// products (32-channel chunk, tap, half chunk; 64-channel chunks for kind 2,
+// where it is the only choice).
+//  - 32 -> 32 channels: one input chunk, the halo-only kernel, which keeps twice
+//    the blocks resident; two rows a wave where that leaves a block per CU.
+//  - 32 -> wider, many pixels: the same kernel with two rows and two channel
+//    tiles a wave (8 x 256 x 256, 32 -> 64: 75.6 -> 49.5), or two rows and two
+//    waves across the channels (3 x 128 x 128: 10.4 -> 8.4; with 256 blocks of
+//    it, 1 x 128 x 256, the LDS weights are as fast: 6.9 against 6.3).
+//  - otherwise weights in LDS.  Two rows and two channel tiles a wave read half
+//    the LDS bytes a product (8 x 64 x 64, 256 -> 128: 32.6 -> 27.9; 1 x 128 x
+//    256, 64 -> 128: 14.5 -> 13.0) but need four times the pixels to fill the
+//    chip: from 192 blocks on (3 x 128 x 128, 64 -> 64: 12.5 either way; with
+//    96, 3 x 64 x 64, 128 -> 128: 10.5 against 13), and not with a pooled output,
+//    whose epilogue takes it longer than it saves.  Else one row and tile a
+//    wave, 64-channel chunks where that leaves at most a block a CU anyway, and
+//    the input chunks split over blocks while those cover fewer than half the
+//    CUs (at 128..255 blocks the split's extra pass costs more than it gains).
+ConvPlan conv3_plan(int N, int H, int W, int Cin, int Cout, bool pooled = false) {
+    constexpr int k111 = 0, k211 = 1, k221 = 4, k212 = 6;  // indices into kTiles3
+    if (Cin == 32 && Cout == 32) return {conv3_blocks(k211, N, H, W, Cout) >= 256 ? k211 : k111, 1, 0};
+    const bool wide = Cout % 64 == 0;
+    if (Cin == 32 && wide && conv3_blocks(k221, N, H, W, Cout) >= 1024) return {k221, 1, 0};
+    if (Cin == 32 && wide && conv3_blocks(k212, N, H, W, Cout) >= 384) return {k212, 1, 0};
+    if (wide && !pooled && conv3_blocks(k221, N, H, W, Cout) >= 192) return {k221, 1, 1};
+    const long long blocks = conv3_blocks(k111, N, H, W, Cout);
+    const int kind = Cin % 64 == 0 && blocks <= 256 ? 2 : 1;
     int split = 1;
-    const int nck = Cin / 32;
-    while (split < 4 && 2 * split <= nck && conv3_blocks(best, N, H, W, Cout) * split < 256) split *= 2;
-    return {best, split, 0};
+    const int nck = Cin / (kind == 2 ? 64 : 32);
+    while (split < 4 && 2 * split <= nck && blocks * split < 128) split *= 2;
+    return {k111, split, kind};
 }
 
 // f32 elements of split-K partial sums a 3x3 convolution needs (0: no split)
@@ -1306,7 +1283,7 @@ void conv_fwd(hipStream_t s, int ks, const ConvIn &in, const uint16_t *w, const 
     ucheck((!bias || aligned(bias, 16)) && aligned(out, out_f32 ? 16 : 8) && (!ws || aligned(ws, 16)) &&
                (!pool_out || aligned(pool_out, 8)),
            "convolution buffers must be 16-byte aligned (8 for bf16 outputs)");
-    ConvPlan pl = conv3_plan(N, H, W, Cin, Cout);
+    ConvPlan pl = conv3_plan(N, H, W, Cin, Cout, pool_out != nullptr);
     if (force.tile) {  // a forced block shape runs on the halo-only kernel unless the kind is forced too
         pl.tile = force.tile - 1;
         pl.kind = 0;
