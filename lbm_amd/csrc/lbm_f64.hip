@@ -26,35 +26,62 @@
 
 #include "../../include/lbm_hip.h"
 #include "staging.h"
+#include "tile.h"
 
 namespace {
 
-__constant__ int kCx[9] = {-1, 0, 1, -1, 0, 1, -1, 0, 1};
-__constant__ int kCy[9] = {-1, -1, -1, 0, 0, 0, 1, 1, 1};
-__constant__ double kW[9] = {1.0 / 36, 1.0 / 9, 1.0 / 36, 1.0 / 9, 4.0 / 9, 1.0 / 9, 1.0 / 36, 1.0 / 9, 1.0 / 36};
-
-__device__ __forceinline__ void feq64(double rho, double ux, double uy, double out[9]) {
-    const double uu = ux * ux + uy * uy;
-#pragma unroll
-    for (int k = 0; k < 9; ++k) {
-        const double cu = kCx[k] * ux + kCy[k] * uy;
-        out[k] = kW[k] * rho * (1.0 + 3.0 * cu + 4.5 * cu * cu - 1.5 * uu);
-    }
+// sum + c v for c = -1, 0, 1 (0 v is exact: the fused form has the bits of the
+// two operations, also where v is not finite)
+template <int c>
+__device__ __forceinline__ double plus(double sum, double v) {
+    return c == 0 ? fma(0.0, v, sum) : c > 0 ? sum + v : sum - v;
 }
 
-// f := f + om (feq - f) of one cell, in the textbook solver's order
+// jx / rho and jy / rho, each correctly rounded: as velocity() in d2q9.h, with
+// the second Newton step on the reciprocal that a double takes before the
+// quotient's residual (12 instead of 22 instructions, one reciprocal instead of
+// two, four for the test).  The residual is exact for numerators down to
+// 2^-900; a smaller quotient changes no bit of the collision's sums.
+__device__ __forceinline__ void velocity64(double jx, double jy, double rho, double &ux, double &uy) {
+    const double top = fmax(fmax(fabs(jx), fabs(jy)), fabs(rho));
+    if (__builtin_expect(__all(rho >= 0x1p-20 && top <= 0x1p20), 1)) {
+        double r = __builtin_amdgcn_rcp(rho);
+        r = fma(fma(-rho, r, 1.0), r, r);
+        r = fma(fma(-rho, r, 1.0), r, r);
+        ux = jx * r;
+        ux = fma(fma(-rho, ux, jx), r, ux);
+        uy = jy * r;
+        uy = fma(fma(-rho, uy, jy), r, uy);
+        return;
+    }
+    ux = jx / rho;
+    uy = jy / rho;
+}
+
+// f := f + om (feq - f) of one cell, in the textbook solver's order.  c.u of
+// opposite directions are each other's negatives, so their even term is the
+// same and 1 + 3 c.u becomes 1 - 3 c.u with the same bits.
 __device__ __forceinline__ void collide64(double fl[9], double om) {
     double rho = 0.0, jx = 0.0, jy = 0.0;
-#pragma unroll
-    for (int k = 0; k < 9; ++k) {
-        rho += fl[k];
-        jx += kCx[k] * fl[k];
-        jy += kCy[k] * fl[k];
-    }
-    double e[9];
-    feq64(rho, jx / rho, jy / rho, e);
-#pragma unroll
-    for (int k = 0; k < 9; ++k) fl[k] = fl[k] + om * (e[k] - fl[k]);
+    [&]<int... K>(std::integer_sequence<int, K...>) {
+        ((rho += fl[K], jx = plus<cx(K)>(jx, fl[K]), jy = plus<cy(K)>(jy, fl[K])), ...);
+    }(std::make_integer_sequence<int, 9>());
+    double ux, uy;
+    velocity64(jx, jy, rho, ux, uy);
+    const double uu15 = 1.5 * (ux * ux + uy * uy);
+    const double rho36 = 1.0 / 36 * rho, rho9 = 1.0 / 9 * rho;
+    auto relax = [&](int k, double wrho, double t) { fl[k] = fl[k] + om * (wrho * (t - uu15) - fl[k]); };
+    auto pair = [&](int k, double wrho, double cu) {  // k and its opposite
+        const double c3 = 3.0 * cu, even = 4.5 * cu * cu;
+        relax(k, wrho, 1.0 + c3 + even);
+        relax(opp(k), wrho, 1.0 - c3 + even);
+    };
+    pair(E, rho9, fma(0.0, uy, ux));
+    pair(S, rho9, fma(0.0, ux, uy));
+    pair(SE, rho36, ux + uy);
+    pair(NE, rho36, ux - uy);
+    // (c.u = 0 u: 1 + 3 c.u + 4.5 (c.u)^2 is 1, or NaN)
+    relax(C, 4.0 / 9 * rho, 1.0 + fma(0.0, ux, 0.0 * uy));
 }
 
 __global__ void k64_collide(const double *__restrict__ f, double *__restrict__ g, size_t n, double om) {
@@ -68,94 +95,258 @@ __global__ void k64_collide(const double *__restrict__ f, double *__restrict__ g
     for (int k = 0; k < 9; ++k) g[k * n + i] = fl[k];
 }
 
-// One step between two post-collision states in one pass: pull from src and
-// collide into dst (streamed cells only).  Column 0 and the last row, which
-// the stream does not write, have the same post-collision value at every step:
-// pulls from them read `fixed`, the state of the call's first collision, which
-// the passes leave alone there (as they leave the solid cells, which nothing
-// pulls from), whichever buffer is the source.
+// ---- the steps after the first collision: several per launch ----------------------
 //
-// Bound by HBM: 144 bytes a cell instead of 288 for a collide and a stream pass
-// (2048 x 1024: 125 -> 65 us a step, 4.7 TB/s).  Every pull is issued before the
-// upstream cells' solid bytes are looked at; a bounced one is read again.
-__global__ __launch_bounds__(256) void k64_step(const double *__restrict__ src, double *__restrict__ dst,
-                                                const double *__restrict__ fixed, const uint8_t *__restrict__ solid,
-                                                int X, int Y, int mode, double om) {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    const int y = blockIdx.y;
-    if (x == 0 || x >= X || y >= Y - 1) return;
-    const size_t n = (size_t)X * Y;
-    const size_t i = (size_t)y * X + x;
-    const uint8_t own = solid[i];
-    double fl[9];
-    unsigned bounced = 0;
-#pragma unroll
-    for (int k = 0; k < 9; ++k) {
-        constexpr int cxk[9] = {-1, 0, 1, -1, 0, 1, -1, 0, 1}, cyk[9] = {-1, -1, -1, 0, 0, 0, 1, 1, 1};
-        int ux = x - cxk[k], uy = y - cyk[k];
-        if (ux >= X) {
-            if (mode == LBM_BOUNDARY_REFERENCE) {
-                ux = 0;
-                uy += 1;
-            } else {
-                ux = X - 1;
-            }
-        }
-        const bool outside = uy < 0 || uy >= Y;
-        const size_t u = (size_t)(outside ? y : uy) * X + ux;
-        if (k != 4 && (outside || solid[u] != 0)) bounced |= 1u << k;
-        const double *from = ux == 0 || uy == Y - 1 ? fixed : src;
-        fl[k] = from[k * n + u];
-    }
-    if (own) return;
-    if (bounced) {
-#pragma unroll
-        for (int k = 0; k < 9; ++k)
-            if ((bounced >> k) & 1u) fl[k] = src[(8 - k) * n + i];
-    }
-    collide64(fl, om);
-#pragma unroll
-    for (int k = 0; k < 9; ++k) dst[k * n + i] = fl[k];
-}
+// Between two post-collision states a step is a pull and a collision; the
+// call's last one is the pull alone.  As in tile.h a block owns a region of 64
+// columns x (waves x M) rows, every population of a cell in registers: the
+// first pull reads memory, the others take columns through lane shifts, rows
+// inside a wave directly and the rows between two waves through LDS (one
+// barrier a step).  Cells whose pulls leave the region turn invalid, one ring a
+// step, so a region writes its inner cells, steps - 1 in from each edge.
+//
+// Column 0 and the last row, which the stream does not write, have the same
+// post-collision value at every step: pulls from them read `fixed`, the state
+// of the call's first collision, which the launches leave alone there (as they
+// leave the solid cells, which nothing pulls from), whichever buffer is the
+// source.  Lane X of a region in reference mode holds column 0 one row on, what
+// the outlet's west-moving populations pull.
+//
+// A step a launch was bound by HBM (2048 x 1024: 65 us a step, 4.7 TB/s).  Here
+// a step moves 37 bytes a cell (6 steps a launch, halo included) and takes about
+// 130 FP64 instructions and 25 to shift and select, 1.5 times counting the
+// halo: 20 us, of which either alone is about 15, as two blocks a CU overlap the
+// one's loads with the other's steps in part.  Select instructions keep an
+// unstreamed cell's value: a version of the steps without them for waves that
+// hold none took 154 instead of 100 registers at three rows a wave, and with
+// them the second block (37 against 21 us).
+// a cell's bounced populations (bits as in d2q9.h), or kFixed: not streamed
+constexpr uint32_t kFixed = 0x100u;
 
-__global__ void k64_stream(const double *__restrict__ g, double *__restrict__ f, const uint8_t *__restrict__ solid,
-                           int X, int Y, int mode, double u_in) {
+template <int MODE>
+__global__ void k64_flags(const uint8_t *__restrict__ solid, uint16_t *__restrict__ flags, int X, int Y) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x;
     const int y = blockIdx.y;
     if (x >= X) return;
-    const size_t n = (size_t)X * Y;
     const size_t i = (size_t)y * X + x;
-    if (x == 0) {
-        double in[9];
-        feq64(1.0, u_in, 0.0, in);
+    uint32_t b = 0;
+    if (x == 0 || y == Y - 1 || solid[i]) {
+        b = kFixed;
+    } else {
 #pragma unroll
-        for (int k = 0; k < 9; ++k) f[k * n + i] = in[k];
-        return;
-    }
-    if (solid[i] || y >= Y - 1) return;
-#pragma unroll
-    for (int k = 0; k < 9; ++k) {
-        if (k == 4) {
-            f[4 * n + i] = g[4 * n + i];
-            continue;
+        for (int k = 0; k < 9; ++k) {
+            if (k == C) continue;
+            int ux, uy;
+            upstream<MODE>(k, x, y, X, ux, uy);
+            if (uy < 0 || uy >= Y || solid[(size_t)uy * X + ux]) b |= 1u << bit(k);
         }
-        int ux = x - kCx[k], uy = y - kCy[k];
-        if (ux >= X) {
-            if (mode == LBM_BOUNDARY_REFERENCE) {
-                ux = 0;
-                uy += 1;
-            } else {
-                ux = X - 1;
+    }
+    flags[i] = (uint16_t)b;
+}
+
+struct Tile64Args {
+    int steps;     // 1 .. kTileMaxSteps
+    int nbx, nby;  // regions across and down
+    int last;      // the call's last step is among them: f = the pulled state
+};
+
+template <int CX>
+__device__ __forceinline__ double shift64(double v) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = from_west_east<CX>((uint32_t)b), hi = from_west_east<CX>((uint32_t)(b >> 32));
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+
+template <int MODE, int M, int NW>
+__global__ __launch_bounds__(64 * NW, NW / 2) void k64_tile(const double *__restrict__ src, double *__restrict__ dst,
+                                                    const double *fixed, const uint16_t *__restrict__ flags, int X,
+                                                    int Y, double om, Tile64Args a) {
+    extern __shared__ double ex64[];
+    constexpr bool wrap = MODE == LBM_BOUNDARY_REFERENCE;
+    constexpr int rows = NW * M;
+    const int L = xcd_remap(blockIdx.x, a.nbx * a.nby);
+    const int by = L / a.nbx, bx = L - by * a.nbx;
+    const int lane = (int)threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int h = a.steps - 1;
+    const int x = bx * (64 - 2 * h) + lane;
+    const int ry0 = w * M, y0 = by * (rows - 2 * h) - 1 + ry0;  // the wave's first row in the region, in the grid
+    const size_t n = (size_t)X * Y;
+    const bool virt = wrap && x == X, outlet = x == X - 1;
+    const bool owner_x = (bx == 0 || lane >= h) && (bx == a.nbx - 1 || lane < 64 - h) && x < X;
+
+    double cur[M][9];
+    uint32_t kind[M];
+    const int x0 = bx * (64 - 2 * h);
+    const uint32_t col = (uint32_t)lane * 8;  // (a row's address is uniform: no address of a lane's own to keep)
+    if (bx > 0 && x0 + 64 < X && y0 > 0 && y0 + M < Y - 1) {
+        // every upstream cell is inside the grid and streamed, or solid and
+        // bounced (an unstreamed cell here is solid: nothing reads its value)
+#pragma unroll
+        for (int j = 0; j < M; ++j) {
+            const ptrdiff_t at = (ptrdiff_t)(y0 + j) * X + x0;
+#pragma unroll
+            for (int k = 0; k < 9; ++k)
+                cur[j][k] = *(const double *)((const char *)(src + k * n + (at - cy(k) * X - cx(k))) + col);
+            kind[j] = *(const uint16_t *)((const char *)(flags + at) + col / 4);
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < M; ++j) {
+            const int y = y0 + j;
+            const bool in = x < X && y >= 0 && y < Y;
+            kind[j] = in ? flags[(size_t)y * X + x] : kFixed;
+            // an unstreamed cell keeps its value; past the grid nothing is read
+            const bool keep = kind[j] == kFixed;
+            const size_t own = virt ? (size_t)min(y + 1, Y - 1) * X : (size_t)min(max(y, 0), Y - 1) * X + min(x, X - 1);
+#pragma unroll
+            for (int k = 0; k < 9; ++k) {
+                int ux, uy;
+                upstream<MODE>(k, x, y, X, ux, uy);
+                uy = min(max(uy, 0), Y - 1);  // (bounced where it is outside)
+                const double *from = keep || ux <= 0 || uy == Y - 1 ? fixed : src;
+                cur[j][k] = from[k * n + (keep ? own : (size_t)uy * X + ux)];
             }
         }
-        bool bounce = uy < 0 || uy >= Y;
-        size_t u = 0;
-        if (!bounce) {
-            u = (size_t)uy * X + ux;
-            bounce = solid[u] != 0;
-        }
-        f[k * n + i] = bounce ? g[(8 - k) * n + i] : g[k * n + u];
     }
+    uint32_t live = 0;  // bit j: the row has streamed cells
+    bool any_bounce = false;
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+        if (!__all(kind[j] == kFixed)) live |= 1u << j;
+        any_bounce = any_bounce || (kind[j] & 0xFFu) != 0;
+    }
+    any_bounce = __any(any_bounce);
+    if (any_bounce)
+#pragma unroll
+        for (int j = 0; j < M; ++j) {
+            if (!(kind[j] & 0xFFu)) continue;
+            const ptrdiff_t at = (ptrdiff_t)(y0 + j) * X + x0;
+#pragma unroll
+            for (int k = 0; k < 9; ++k)
+                if (k != C && ((kind[j] >> bit(k)) & 1u))
+                    cur[j][k] = *(const double *)((const char *)(src + opp(k) * n + at) + col);
+        }
+
+    // does a later step or the store need step s (from 1) of row j, of any of the wave's rows?
+    auto row_needed = [&](int s, int j) {
+        return (by == 0 || ry0 + j >= s - 1) && (by == a.nby - 1 || ry0 + j < rows - (s - 1)) && ((live >> j) & 1u);
+    };
+    auto needed = [&](int s) {
+        return (by == 0 || ry0 + M - 1 >= s - 1) && (by == a.nby - 1 || ry0 < rows - (s - 1)) && live;
+    };
+    if (!(a.last && a.steps == 1))
+#pragma unroll
+        for (int j = 0; j < M; ++j) {
+            if (!row_needed(1, j)) continue;
+            double f[9];
+#pragma unroll
+            for (int k = 0; k < 9; ++k) f[k] = cur[j][k];
+            collide64(f, om);
+#pragma unroll
+            for (int k = 0; k < 9; ++k) cur[j][k] = kind[j] == kFixed ? cur[j][k] : f[k];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+
+    auto advance = [&]<bool COLLIDE>(int s) {
+        double *e = ex64 + (size_t)(s & 1) * NW * 6 * 64;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            e[(w * 6 + i) * 64 + lane] = cur[0][i];              // NW, N, NE
+            e[(w * 6 + 3 + i) * 64 + lane] = cur[M - 1][6 + i];  // SW, S, SE
+        }
+        __syncthreads();
+        if (!needed(s)) return;
+        double south[3], north[3];  // S-movers of the row above, N-movers of the row below the wave
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            south[i] = e[(max(w - 1, 0) * 6 + 3 + i) * 64 + lane];
+            north[i] = e[(min(w + 1, NW - 1) * 6 + i) * 64 + lane];
+        }
+#pragma unroll
+        for (int j = 0; j < M; ++j) {
+            if (!row_needed(s, j)) {
+#pragma unroll
+                for (int i = 0; i < 3; ++i) south[i] = cur[j][6 + i];
+                continue;
+            }
+            double p[9];
+            [&]<int... K>(std::integer_sequence<int, K...>) {
+                (
+                    [&] {
+                        const double v = cy(K) > 0   ? south[K >= 6 ? K - 6 : 0]
+                                         : cy(K) < 0 ? (j + 1 < M ? cur[j + 1 < M ? j + 1 : j][K] : north[K < 3 ? K : 0])
+                                                     : cur[j][K];
+                        const double sh = shift64<cx(K)>(v);
+                        p[K] = !wrap && cx(K) < 0 && outlet ? v : sh;
+                    }(),
+                    ...);
+            }(std::make_integer_sequence<int, 9>());
+            if (any_bounce) {
+                // (opaque: the tests of every row are otherwise kept in 16 M
+                // scalar registers over the steps)
+                uint32_t kd = kind[j];
+                asm volatile("" : "+v"(kd));
+#pragma unroll
+                for (int k = 0; k < 9; ++k)
+                    if (k != C && ((kd >> bit(k)) & 1u)) p[k] = cur[j][opp(k)];
+            }
+#pragma unroll
+            for (int i = 0; i < 3; ++i) south[i] = cur[j][6 + i];
+            if constexpr (COLLIDE) collide64(p, om);
+#pragma unroll
+            for (int k = 0; k < 9; ++k) cur[j][k] = kind[j] == kFixed ? cur[j][k] : p[k];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    const int collided = a.steps - (a.last ? 1 : 0);
+    for (int s = 2; s <= collided; ++s) advance.template operator()<true>(s);
+    if (a.last && a.steps > 1) advance.template operator()<false>(a.steps);
+
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+        const int r = ry0 + j;
+        const bool own = (by == 0 || r >= h) && (by == a.nby - 1 || r < rows - h) && y0 + j < Y;
+        if (!(own && owner_x && kind[j] != kFixed)) continue;
+        double *const row = dst + ((ptrdiff_t)(y0 + j) * X + x0);
+#pragma unroll
+        for (int k = 0; k < 9; ++k) *(double *)((char *)(row + k * n) + col) = cur[j][k];
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// Block shapes as in tile.h, fitted to launches of 1 to 8 steps over 0.006 to 4
+// million cells (within 20% / 38% / 44%, the largest errors where a round is
+// barely begun).  Best us per step of each: 300 x 150 1.95 / 2.71 / 3.88, 640 x
+// 320 4.24 / 3.65 / 4.05, 2048 x 1024 32.4 / 22.7 / 20.2.  Taller regions of
+// three and four rows a wave leave one block a CU, whose loads nothing then
+// hides (3 x 12: 25.9, 4 x 12: 25.7).
+constexpr TileShape kTile64[3] = {{1, 16, false, 0.0f, 0.37f, 5.47f, 0.66f},
+                                  {2, 12, false, 0.0f, 0.93f, 6.67f, 0.95f},
+                                  {4, 8, false, 0.0f, 1.17f, 8.21f, 1.48f}};
+
+// A call's launches: their number is odd, as they go from g to f to g ... and
+// the last one has to end in f, which holds the cells the stream does not write.
+TilePlan plan64(int X, int Y, uint32_t n) {
+    TilePlan best{0, 0};
+    float least = 0.0f;
+    for (int i = 0; i < 3; ++i) {
+        const TileShape &sh = kTile64[i];
+        float cost[kTileMaxSteps + 2] = {};
+        for (int s = 1; s <= kTileMaxSteps; ++s)
+            cost[s] = tile_cost(sh, s, (double)tile_nbx(X, s) * tile_nby(Y, sh.waves * sh.m, s));
+        for (int s = 1; s <= kTileMaxSteps; ++s) {
+            const uint32_t launches = ((n + s - 1) / s) | 1u;
+            if (launches > n) continue;
+            const uint32_t low = n / launches, more = n % launches;
+            const float c = cost[low] * (float)(launches - more) + cost[low + 1] * (float)more;
+            if (!best.launches || c < least) {
+                best = TilePlan{i, launches};
+                least = c;
+            }
+        }
+    }
+    return best;
 }
 
 // rho, u = j / rho (uy north-positive, as the reference's uy field)
@@ -167,8 +358,8 @@ __global__ void k64_macro(const double *__restrict__ f, double *__restrict__ out
     for (int k = 0; k < 9; ++k) {
         const double v = f[k * n + i];
         r += v;
-        jx += kCx[k] * v;
-        jy += kCy[k] * v;
+        jx += cx(k) * v;
+        jy += cy(k) * v;
     }
     out[i] = r;
     out[n + i] = jx / r;
@@ -202,6 +393,7 @@ struct lbm_f64 {
     double omega = 1.0, u_in = 0.0;
     double *f = nullptr, *g = nullptr, *scratch = nullptr;
     uint8_t *solid = nullptr;
+    uint16_t *flags = nullptr;
     uint64_t steps = 0;
     Staging staging;
 
@@ -209,10 +401,11 @@ struct lbm_f64 {
     void release() {
         (void)hipSetDevice(dev);
         staging.release();
-        for (void *p : {(void *)f, (void *)g, (void *)scratch, (void *)solid})
+        for (void *p : {(void *)f, (void *)g, (void *)scratch, (void *)solid, (void *)flags})
             if (p) (void)hipFree(p);
         f = g = scratch = nullptr;
         solid = nullptr;
+        flags = nullptr;
         if (stream) (void)hipStreamDestroy(stream);
         stream = nullptr;
     }
@@ -226,6 +419,9 @@ int fguard(F &&fn) {
         fn();
         return LBM_OK;
     } catch (const HErr &e) {
+        g_f64_error = std::string(e.what) + ": " + hipGetErrorString(e.e);
+        return e.e == hipErrorOutOfMemory ? LBM_ENOMEM : LBM_EHIP;
+    } catch (const HipError &e) {
         g_f64_error = std::string(e.what) + ": " + hipGetErrorString(e.e);
         return e.e == hipErrorOutOfMemory ? LBM_ENOMEM : LBM_EHIP;
     } catch (const AErr &e) {
@@ -242,6 +438,37 @@ int fguard(F &&fn) {
 
 void fcheck(bool ok, const char *msg) {
     if (!ok) throw AErr{msg};
+}
+
+void flags64(lbm_f64 *h) {
+    const dim3 grid((h->X + 255) / 256, h->Y);
+    if (h->mode == LBM_BOUNDARY_REFERENCE)
+        hipLaunchKernelGGL(k64_flags<LBM_BOUNDARY_REFERENCE>, grid, dim3(256), 0, h->stream, h->solid, h->flags, h->X,
+                           h->Y);
+    else
+        hipLaunchKernelGGL(k64_flags<LBM_BOUNDARY_ZERO_GRADIENT>, grid, dim3(256), 0, h->stream, h->solid, h->flags,
+                           h->X, h->Y);
+    H64(hipGetLastError());
+}
+
+// one launch, from g to f or back
+void tile64(lbm_f64 *h, int shape, int steps, bool to_f, bool last) {
+    auto launch = [&]<int MODE, int SHAPE>() {
+        constexpr TileShape sh = kTile64[SHAPE];
+        constexpr auto kernel = &k64_tile<MODE, sh.m, sh.waves>;
+        constexpr size_t lds = (size_t)sh.waves * 64 * 2 * 6 * sizeof(double);
+        const Tile64Args a{steps, tile_nbx(h->X, steps), tile_nby(h->Y, sh.waves * sh.m, steps), last};
+        tile_allow_lds<kernel>(lds, h->dev);
+        hipLaunchKernelGGL(kernel, dim3(a.nbx * a.nby), dim3(64 * sh.waves), lds, h->stream, to_f ? h->g : h->f,
+                           to_f ? h->f : h->g, h->g, h->flags, h->X, h->Y, h->omega, a);
+    };
+    auto shapes = [&]<int MODE>() {
+        if (shape == 0) launch.template operator()<MODE, 0>();
+        else if (shape == 1) launch.template operator()<MODE, 1>();
+        else launch.template operator()<MODE, 2>();
+    };
+    if (h->mode == LBM_BOUNDARY_REFERENCE) shapes.template operator()<LBM_BOUNDARY_REFERENCE>();
+    else shapes.template operator()<LBM_BOUNDARY_ZERO_GRADIENT>();
 }
 
 }  // namespace
@@ -271,6 +498,7 @@ int lbm_f64_create(uint32_t nx, uint32_t ny, double omega, double u_in, int32_t 
             H64(hipMalloc(&h->f, 9 * n * sizeof(double)));
             H64(hipMalloc(&h->g, 9 * n * sizeof(double)));
             H64(hipMalloc(&h->solid, n));
+            H64(hipMalloc(&h->flags, n * sizeof(uint16_t)));
             // walls on the first and last rows; everything at feq(1, (u_in, 0))
             std::vector<uint8_t> s(n, 0);
             for (uint32_t x = 0; x < nx; ++x) {
@@ -278,6 +506,7 @@ int lbm_f64_create(uint32_t nx, uint32_t ny, double omega, double u_in, int32_t 
                 s[(size_t)(ny - 1) * nx + x] = 1;
             }
             H64(hipMemcpy(h->solid, s.data(), n, hipMemcpyHostToDevice));
+            flags64(h);
             const int cx[9] = {-1, 0, 1, -1, 0, 1, -1, 0, 1};
             const double w[9] = {1.0 / 36, 1.0 / 9, 1.0 / 36, 1.0 / 9, 4.0 / 9, 1.0 / 9, 1.0 / 36, 1.0 / 9, 1.0 / 36};
             std::vector<double> plane(n);
@@ -311,6 +540,7 @@ int lbm_f64_set_mask(lbm_f64 *h, const uint8_t *solid) {
         std::vector<uint8_t> s(solid, solid + h->n());
         for (auto &v : s) v = v == 1 ? 1 : 0;
         H64(hipMemcpyAsync(h->solid, s.data(), h->n(), hipMemcpyHostToDevice, h->stream));
+        flags64(h);
         H64(hipStreamSynchronize(h->stream));
     });
 }
@@ -319,33 +549,14 @@ int lbm_f64_step(lbm_f64 *h, uint32_t n) {
     return fguard([&] {
         fcheck(h != nullptr, "null handle");
         H64(hipSetDevice(h->dev));
+        if (n == 0) return;
         const size_t cells = h->n();
-        const dim3 sg((h->X + 255) / 256, h->Y);
-        auto collide = [&] {
-            hipLaunchKernelGGL(k64_collide, dim3((unsigned)((cells + 255) / 256)), dim3(256), 0, h->stream, h->f,
-                               h->g, cells, h->omega);
-        };
-        auto stream = [&] {
-            hipLaunchKernelGGL(k64_stream, sg, dim3(256), 0, h->stream, h->g, h->f, h->solid, h->X, h->Y, h->mode,
-                               h->u_in);
-        };
-        // collide, n - 1 fused passes, stream.  The fused passes go g -> f ->
-        // g ..., so their number is made even (a separate step first): the
-        // last stream then reads g and finds in f the cells it does not write.
-        if (n % 2 == 0 && n > 0) {
-            collide();
-            stream();
-        }
-        if (n > 0) {
-            collide();
-            for (uint32_t s = 0; s + 2 < n; s += 2) {
-                hipLaunchKernelGGL(k64_step, sg, dim3(256), 0, h->stream, h->g, h->f, h->g, h->solid, h->X, h->Y,
-                                   h->mode, h->omega);
-                hipLaunchKernelGGL(k64_step, sg, dim3(256), 0, h->stream, h->f, h->g, h->g, h->solid, h->X, h->Y,
-                                   h->mode, h->omega);
-            }
-            stream();
-        }
+        hipLaunchKernelGGL(k64_collide, dim3((unsigned)((cells + 255) / 256)), dim3(256), 0, h->stream, h->f, h->g,
+                           cells, h->omega);
+        const TilePlan plan = plan64(h->X, h->Y, n);
+        const uint32_t low = n / plan.launches, more = n % plan.launches;
+        for (uint32_t i = 0; i < plan.launches; ++i)
+            tile64(h, plan.shape, (int)(low + (i < more)), i % 2 == 0, i + 1 == plan.launches);
         H64(hipGetLastError());
         h->steps += n;
     });
