@@ -537,6 +537,91 @@ __global__ __launch_bounds__(256) void k_conv3_lds(ConvIn src, const uint16_t *_
         if (hd.w) conv_head_tile<MI>(acc, bias, relu, hd, H, W, n, x0, y0 + wm * MI, lane);
 }
 
+// The same convolution for one plain 32-channel input, two rows and one channel
+// tile a wave.  A layer of so few channels has one chunk, so the kernel above
+// waits for every halo and reads 18 KB of weights a wave for 36 products; here a
+// block keeps the weights in registers and walks down a run of `rows` row tiles, the
+// next one's halo on its way while this one is multiplied (8 x 256 x 256, a
+// forward pass: 458 -> 434 us; one row tile a block 445, twice the run 480, as it
+// leaves one block a CU).  Same products in the same order.
+template <int WN>
+__global__ __launch_bounds__(256, 2) void k_conv3_rows(const uint16_t *__restrict__ src, const uint16_t *__restrict__ w,
+                                                       const float *__restrict__ bias, void *__restrict__ out,
+                                                       uint16_t *__restrict__ pout, ConvHead hd,
+                                                       const uint16_t *__restrict__ gate, int N, int H, int W, int Cout,
+                                                       int co_store, int relu, int out_f32, int rows) {
+    constexpr int MI = 2, WM = 4 / WN, TH = WM * MI, HR = TH + 2, HC = 34, PS = 40;
+    constexpr int NPIECE = HR * HC * 4, PER_T = (NPIECE + 255) / 256;
+    __shared__ __align__(16) uint16_t lds[2][HR * HC * PS];
+    const int tiles_x = W >> 5, tiles_y = (H + TH - 1) / TH, runs = (tiles_y + rows - 1) / rows;
+    int bid = blockIdx.x;
+    const int tx = bid % tiles_x;
+    bid /= tiles_x;
+    const int ty0 = bid % runs * rows, ty1 = min(ty0 + rows, tiles_y);
+    const long long n = bid / runs;
+    const int x0 = tx * 32;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wm = wave / WN, wn = wave % WN;
+    const int half = lane >> 5, l32 = lane & 31;
+    const int co0 = (blockIdx.y * WN + wn) * 32;
+    const uint16_t *img = src + n * H * W * 32;
+
+    u16x8 stage[PER_T];
+    auto gload = [&](int y0) {
+#pragma unroll
+        for (int t = 0; t < PER_T; ++t) {
+            const int q = threadIdx.x + 256 * t, pi = q >> 2;
+            const int y = y0 - 1 + pi / HC, x = x0 - 1 + pi % HC;
+            stage[t] = u16x8{};
+            if (q < NPIECE && y >= 0 && y < H && x >= 0 && x < W)
+                stage[t] = *(const u16x8 *)(img + (y * W + x) * 32 + ((q & 3) << 3));
+        }
+    };
+    auto swrite = [&](int buf) {
+#pragma unroll
+        for (int t = 0; t < PER_T; ++t) {
+            const int q = threadIdx.x + 256 * t;
+            if (q < NPIECE) *(u16x8 *)&lds[buf][(q >> 2) * PS + ((q & 3) << 3)] = stage[t];
+        }
+    };
+    gload(ty0 * TH);
+    u16x8 wt[9][2];
+#pragma unroll
+    for (int tap = 0; tap < 9; ++tap)
+#pragma unroll
+        for (int s2 = 0; s2 < 2; ++s2)
+            wt[tap][s2] = *(const u16x8 *)(w + ((size_t)tap * Cout + co0 + l32) * 32 + 16 * s2 + 8 * half);
+    swrite(0);
+    __syncthreads();
+    int buf = 0;
+    for (int ty = ty0; ty < ty1; ++ty, buf ^= 1) {
+        if (ty + 1 < ty1) gload((ty + 1) * TH);
+        f32x16 acc[MI][1];
+#pragma unroll
+        for (int i = 0; i < MI; ++i) acc[i][0] = f32x16{};
+#pragma unroll
+        for (int tap = 0; tap < 9; ++tap)
+#pragma unroll
+            for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+                for (int i = 0; i < MI; ++i) {
+                    const int r = wm * MI + i + tap / 3;
+                    const u16x8 a = *(const u16x8 *)&lds[buf][(r * HC + l32 + tap % 3) * PS + 16 * s2 + 8 * half];
+                    acc[i][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, wt[tap][s2]),
+                                                                        __builtin_bit_cast(bf16x8, a), acc[i][0], 0, 0,
+                                                                        0);
+                }
+        if (ty + 1 < ty1) swrite(buf ^ 1);
+        const int y = ty * TH + wm * MI;
+        conv_store_tile<MI, 1>(acc, bias, out, nullptr, gate, N, H, W, Cout, co_store, relu, out_f32, n, x0, y, co0, half,
+                               l32);
+        if (pout) conv_pool_tile<MI, 1, WN>(acc, bias, pout, &lds[0][0], H, W, Cout, relu, n, x0, y, wm, co0, lane);
+        if constexpr (WN == 1)
+            if (hd.w) conv_head_tile<MI>(acc, bias, relu, hd, H, W, n, x0, y, lane);
+        __syncthreads();
+    }
+}
+
 // The same convolution with the weights staged in LDS too.  Per chunk the
 // block loads the B operands of all nine taps for its 32 * WN * NI output
 // channels once, with 16-byte loads along input channels (64 contiguous bytes
@@ -1314,6 +1399,21 @@ void conv_fwd(hipStream_t s, int ks, const ConvIn &in, const uint16_t *w, const 
            "head: a bf16 32-channel layer, 32 x 32 weights, 32 f32 outputs per pixel");
     const bool fuse_head = head.w && kind == 0 && !split && kTiles3[t][1] == 1 && kTiles3[t][2] == 1;
     const ConvHead hd = fuse_head ? head : ConvHead{};
+    // one plain 32-channel input, two rows a wave: k_conv3_rows, in runs that
+    // leave two blocks a CU (its index of a pixel's channels is 32 bits)
+    const bool in_rows = kind == 0 && (t == 1 || t == 6) && in.ca == 32 && in.cb == 0 && !in.a_up &&
+                         (long long)H * W <= 1 << 25;
+    if (in_rows) {
+        const int th = t == 1 ? 8 : 4, tiles_y = (H + th - 1) / th;
+        const int rows = (int)std::max(1ll, std::min<long long>(tiles_y, (long long)grid.x * grid.y / 512));
+        const dim3 rgrid((unsigned)(N * (W / 32) * ((tiles_y + rows - 1) / rows)), grid.y);
+        if (t == 1)
+            hipLaunchKernelGGL(k_conv3_rows<1>, rgrid, dim3(256), 0, s, in.a, w, bias, out, pout, hd, gate, N, H, W,
+                               Cout, co_store, r, f, rows);
+        else
+            hipLaunchKernelGGL(k_conv3_rows<2>, rgrid, dim3(256), 0, s, in.a, w, bias, out, pout, hd, gate, N, H, W,
+                               Cout, co_store, r, f, rows);
+    }
 #define L3(MI, NI, WN)                                                                                             \
     do {                                                                                                           \
         if (kind == 2)                                                                                             \
@@ -1326,7 +1426,7 @@ void conv_fwd(hipStream_t s, int ks, const ConvIn &in, const uint16_t *w, const 
             hipLaunchKernelGGL((k_conv3_lds<MI, NI, WN>), grid, dim3(256), 0, s, in, w, bias, out, ws, pout, hd, gate, \
                                N, H, W, Cout, co_store, r, f);                                                        \
     } while (0)
-    switch (t) {
+    if (!in_rows) switch (t) {
         case 0: L3(1, 1, 1); break;
         case 1: L3(2, 1, 1); break;
         case 2: L3(4, 1, 1); break;
