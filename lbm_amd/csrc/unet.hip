@@ -61,6 +61,59 @@ struct ConvIn {
     int ca = 0, cb = 0, a_up = 0;
 };
 
+// Bias, ReLU, rounding, gate (see conv_store_tile) and store of a wave's whole
+// 32-pixel x 32-channel tile of products, [cout][pixel], into the bf16 pixels
+// from p0 on, channels from co0 on.  Lane l holds four runs of four channels of
+// pixel l % 32; the two lanes of a pixel and then the pixels 16 apart trade
+// theirs, so that four lanes hold a pixel's 64 bytes and a store writes whole
+// segments of 64 bytes.  Stored as the products lie, 8 bytes a lane 64 apart, the
+// partial lines bounded the layers of few channels (forward pass 8 x 256 x 256:
+// 436 us, with runs of 32 bytes 386, of 64 bytes 380; in order of lanes too,
+// through LDS, 377 and slower at 1 x 128 x 256).
+__device__ __forceinline__ void store_bf16_tile(const f32x16 &acc, const float *__restrict__ bias, bool relu,
+                                                const uint16_t *__restrict__ gate, uint16_t *__restrict__ out,
+                                                long long p0, int Cout, int co0, int half, int l32) {
+    uint32_t d[4][2];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        float v[4] = {acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+        if (bias) {
+            const float4 bv = *(const float4 *)&bias[co0 + 8 * g + 4 * half];
+            v[0] += bv.x;
+            v[1] += bv.y;
+            v[2] += bv.z;
+            v[3] += bv.w;
+        }
+        if (relu)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = fmaxf(v[e], 0.0f);
+        d[g][0] = f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16);
+        d[g][1] = f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
+    }
+    uint32_t o[2][4];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const auto lo = __builtin_amdgcn_permlane32_swap(d[0][e], d[1][e], false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap(d[2][e], d[3][e], false, false);
+        const auto q0 = __builtin_amdgcn_permlane16_swap(lo[0], hi[0], false, false);
+        const auto q1 = __builtin_amdgcn_permlane16_swap(lo[1], hi[1], false, false);
+        o[0][e] = q0[0];
+        o[1][e] = q0[1];
+        o[0][2 + e] = q1[0];
+        o[1][2 + e] = q1[1];
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const long long at = (p0 + 16 * q + (l32 & 15)) * Cout + co0 + 8 * half + (l32 & 16);
+        uint4 v = make_uint4(o[q][0], o[q][1], o[q][2], o[q][3]);
+        if (gate) {
+            const uint4 y = *(const uint4 *)&gate[at];
+            v = make_uint4(gate2(v.x, y.x), gate2(v.y, y.y), gate2(v.z, y.z), gate2(v.w, y.w));
+        }
+        *(uint4 *)&out[at] = v;
+    }
+}
+
 typedef uint16_t u16x16 __attribute__((ext_vector_type(16)));  // 32 B: one lane's operands for two k-steps
 
 // 1x1 convolution: out[p][co] = act(bias[co] + sum_ci in[p][ci] w[co][ci]),
@@ -124,6 +177,14 @@ __global__ __launch_bounds__(256) void k_conv1x1(const uint16_t *__restrict__ in
         if (kk + 2 < nk) load(kk + 2, A0, B0);
         mma(A1, B1);
     }
+    if (!OUT_F32 && co_store == Cout) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NI; ++j)
+                store_bf16_tile(acc[i][j], bias, RELU, gate, (uint16_t *)out, p0 + 32 * i, Cout, co0 + 32 * j, half, l32);
+        return;
+    }
     // lane l holds pixel l % 32 and channels 8 g + 4 (l / 32) .. + 3: four at a time
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
@@ -143,13 +204,8 @@ __global__ __launch_bounds__(256) void k_conv1x1(const uint16_t *__restrict__ in
                 if (OUT_F32) {
                     *(float4 *)&((float *)out)[p * Cout + co] = make_float4(v[0], v[1], v[2], v[3]);
                 } else {
-                    uint32_t lo = f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16),
-                             hi = f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
-                    if (gate) {
-                        const uint2 y = *(const uint2 *)&gate[p * Cout + co];
-                        lo = gate2(lo, y.x);
-                        hi = gate2(hi, y.y);
-                    }
+                    const uint32_t lo = f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16),
+                                   hi = f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
                     *(uint2 *)&((uint16_t *)out)[p * Cout + co] = make_uint2(lo, hi);
                 }
             }
@@ -161,7 +217,7 @@ __global__ __launch_bounds__(256) void k_conv1x1(const uint16_t *__restrict__ in
 // the A operand and the pixels as B, so a wave's 32 x 32 result is
 // [cout][pixel]: lane l holds pixel l % 32 and output channels
 // 8 (r / 4) + 4 (l / 32) + r % 4, r = 0..15 -- four runs of four consecutive
-// channels, stored as four 8-byte (bf16) or 16-byte (f32) pieces.  gate (input
+// channels, stored as such in f32 and by store_bf16_tile in bf16.  gate (input
 // gradients, bf16): the activation the gradient belongs to, of the output's
 // shape; where it is not positive its ReLU passes nothing on and 0 is stored
 // (a pass of its own read and wrote every gradient once more: 17 launches,
@@ -183,6 +239,13 @@ __device__ __forceinline__ void conv_store_tile(const f32x16 (&acc)[MI][NI], con
         const int y = y_first + i;
         if (y >= H) continue;
         const long long p = (n * H + y) * W + x0 + l32;
+        if (!split && !out_f32 && co_store == Cout) {
+#pragma unroll
+            for (int j = 0; j < NI; ++j)
+                store_bf16_tile(acc[i][j], bias, relu, gate, (uint16_t *)out, p - l32, Cout, co_first + 32 * j, half,
+                                l32);
+            continue;
+        }
 #pragma unroll
         for (int j = 0; j < NI; ++j) {
 #pragma unroll
@@ -207,13 +270,8 @@ __device__ __forceinline__ void conv_store_tile(const f32x16 (&acc)[MI][NI], con
                     if (out_f32) {
                         *(float4 *)&((float *)out)[p * Cout + co] = make_float4(v[0], v[1], v[2], v[3]);
                     } else {
-                        uint32_t lo = f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16),
-                                 hi = f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
-                        if (gate) {
-                            const uint2 y2 = *(const uint2 *)&gate[p * Cout + co];
-                            lo = gate2(lo, y2.x);
-                            hi = gate2(hi, y2.y);
-                        }
+                        const uint32_t lo = f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16),
+                                       hi = f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
                         *(uint2 *)&((uint16_t *)out)[p * Cout + co] = make_uint2(lo, hi);
                     }
                 } else {
@@ -1335,12 +1393,12 @@ void conv_fwd(hipStream_t s, int ks, const ConvIn &in, const uint16_t *w, const 
     ucheck(W % 32 == 0 && in.ca % 32 == 0 && in.cb % 32 == 0 && Cin > 0 && Cout % 32 == 0,
            "convolution shape: W, channel counts must be multiples of 32");
     ucheck(!in.a_up || H % 2 == 0, "upsampled input needs an even height");
-    ucheck(!gate || (!out_f32 && !relu && co_store == Cout && ((uintptr_t)gate & 7) == 0),
+    ucheck(!gate || (!out_f32 && !relu && co_store == Cout && ((uintptr_t)gate & 15) == 0),
            "gate: a whole bf16 gradient's activation");
     if (ks == 1) {
         ucheck(!in.a_up && in.cb == 0 && !pool_out && !head.w, "1x1 convolutions take one plain input only");
-        ucheck(((uintptr_t)bias & 15) == 0 && ((uintptr_t)out & (out_f32 ? 15 : 7)) == 0,
-               "convolution buffers must be 16-byte aligned (8 for bf16 outputs)");
+        ucheck(((uintptr_t)bias & 15) == 0 && ((uintptr_t)out & 15) == 0,
+               "convolution buffers must be 16-byte aligned");
         int mi = 1, ni = 1;
         if (P % 64 == 0 && P / 64 * (Cout / 32) >= 4096) mi = 2;
         else if (Cout % 64 == 0 && P / 32 * (Cout / 64) >= 4096) ni = 2;
@@ -1362,12 +1420,12 @@ void conv_fwd(hipStream_t s, int ks, const ConvIn &in, const uint16_t *w, const 
         HIPCHK(hipGetLastError());
         return;
     }
-    // the 3x3 epilogues move four channels at a time (float4 bias and partial
-    // sums, 8- or 16-byte output and pooled stores)
+    // the 3x3 epilogues move four channels of bias, partial sums and pooled
+    // output at a time and 16 bytes of output
     auto aligned = [](const void *q, uintptr_t a) { return ((uintptr_t)q & (a - 1)) == 0; };
-    ucheck((!bias || aligned(bias, 16)) && aligned(out, out_f32 ? 16 : 8) && (!ws || aligned(ws, 16)) &&
+    ucheck((!bias || aligned(bias, 16)) && aligned(out, 16) && (!ws || aligned(ws, 16)) &&
                (!pool_out || aligned(pool_out, 8)),
-           "convolution buffers must be 16-byte aligned (8 for bf16 outputs)");
+           "convolution buffers must be 16-byte aligned (8 for pooled outputs)");
     ConvPlan pl = conv3_plan(N, H, W, Cin, Cout, pool_out != nullptr);
     if (force.tile) {  // a forced block shape runs on the halo-only kernel unless the kind is forced too
         pl.tile = force.tile - 1;
