@@ -287,6 +287,12 @@ __device__ __forceinline__ void conv_store_tile(const f32x16 (&acc)[MI][NI], con
     }
 }
 
+// the value of lane ^ 1
+__device__ __forceinline__ float other_of_pair(float v) {
+    const int i = __builtin_bit_cast(int, v);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, 0xB1, 0xF, 0xF, false));
+}
+
 // 2 x 2 average pool of a block's bf16 outputs into pout (H / 2 x W / 2 x
 // Cout), with k_pool2's arithmetic on the stored values:
 // bf16(0.25 ((v(y, x) + v(y, x + 1)) + (v(y + 1, x) + v(y + 1, x + 1)))).
@@ -314,30 +320,43 @@ __device__ __forceinline__ void conv_pool_tile(const f32x16 (&acc)[MI][NI], cons
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = bf2f(f2bf(relu ? fmaxf(v[e], 0.0f) : v[e]));
     };
-    auto emit = [&](int y, int j, int g, const float (&top)[4], const float (&bot)[4]) {
+    // the lane's pixel pair's means (both lanes of a pair get them)
+    auto pool = [&](const float (&top)[4], const float (&bot)[4], uint32_t (&d)[2]) {
         float o[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float t1 = __shfl_xor(top[e], 1), b1 = __shfl_xor(bot[e], 1);
-            o[e] = 0.25f * ((top[e] + t1) + (bot[e] + b1));
+        for (int e = 0; e < 4; ++e)
+            o[e] = 0.25f * ((top[e] + other_of_pair(top[e])) + (bot[e] + other_of_pair(bot[e])));
+        d[0] = f2bf(o[0]) | ((uint32_t)f2bf(o[1]) << 16);
+        d[1] = f2bf(o[2]) | ((uint32_t)f2bf(o[3]) << 16);
+    };
+    // as in store_bf16_tile; the even lane of a pair stores channels 0 .. 15, the odd one 16 .. 31
+    auto put = [&](int y, int j, const uint32_t (&d)[4][2]) {
+        const bool odd = (l32 & 1) != 0;
+        uint32_t v[4];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const auto lo = __builtin_amdgcn_permlane32_swap(d[0][e], d[1][e], false, false);
+            const auto hi = __builtin_amdgcn_permlane32_swap(d[2][e], d[3][e], false, false);
+            v[e] = odd ? hi[0] : lo[0];
+            v[2 + e] = odd ? hi[1] : lo[1];
         }
-        if ((l32 & 1) == 0 && y < H) {
-            const int co = co_first + 32 * j + 8 * g + 4 * half;
-            const long long q = (n * Ho + (y >> 1)) * Wo + ((x0 + l32) >> 1);
-            const uint32_t lo = f2bf(o[0]) | ((uint32_t)f2bf(o[1]) << 16), hi = f2bf(o[2]) | ((uint32_t)f2bf(o[3]) << 16);
-            *(uint2 *)&pout[q * Cout + co] = make_uint2(lo, hi);
-        }
+        if (y >= H) return;
+        const long long q = (n * Ho + (y >> 1)) * Wo + ((x0 + l32) >> 1);
+        *(uint4 *)&pout[q * Cout + co_first + 32 * j + 16 * (l32 & 1) + 8 * half] = make_uint4(v[0], v[1], v[2], v[3]);
     };
     if constexpr (MI == 2) {
 #pragma unroll
-        for (int j = 0; j < NI; ++j)
+        for (int j = 0; j < NI; ++j) {
+            uint32_t d[4][2];
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 float top[4], bot[4];
                 vals(0, j, g, top);
                 vals(1, j, g, bot);
-                emit(y_first, j, g, top, bot);
+                pool(top, bot, d[g]);
             }
+            put(y_first, j, d);
+        }
     } else {
         u16x8 *slot = (u16x8 *)scratch + (size_t)(wm >> 1) * NI * 128;
         if (wm & 1) {
@@ -360,7 +379,8 @@ __device__ __forceinline__ void conv_pool_tile(const f32x16 (&acc)[MI][NI], cons
         __syncthreads();
         if (!(wm & 1)) {
 #pragma unroll
-            for (int j = 0; j < NI; ++j)
+            for (int j = 0; j < NI; ++j) {
+                uint32_t d[4][2];
 #pragma unroll
                 for (int h2 = 0; h2 < 2; ++h2) {
                     const u16x8 pk = slot[(j * 2 + h2) * 64 + lane];
@@ -370,9 +390,11 @@ __device__ __forceinline__ void conv_pool_tile(const f32x16 (&acc)[MI][NI], cons
                         vals(0, j, 2 * h2 + gg, top);
 #pragma unroll
                         for (int e = 0; e < 4; ++e) bot[e] = bf2f(pk[4 * gg + e]);
-                        emit(y_first, j, 2 * h2 + gg, top, bot);
+                        pool(top, bot, d[2 * h2 + gg]);
                     }
                 }
+                put(y_first, j, d);
+            }
         }
     }
 }
@@ -1337,32 +1359,28 @@ long long conv3_blocks(int t, int N, int H, int W, int Cout) {
 }
 
 // Block shape, kernel and split by layer shape, from timings of every shape for
-// the network's layers at batches of 1, 3 and 8 (us, old choice -> this one).
+// the network's layers at batches of 1, 3 and 8 (us, the other choice -> this one).
 // Choices differ in how the work is laid out, not in the order of an output's
 // products (32-channel chunk, tap, half chunk; 64-channel chunks for kind 2,
 // where it is the only choice).
-//  - 32 -> 32 channels: one input chunk, the halo-only kernel, which keeps twice
-//    the blocks resident; two rows a wave where that leaves a block per CU.
-//  - 32 -> wider, many pixels: the same kernel with two rows and two channel
-//    tiles a wave (8 x 256 x 256, 32 -> 64: 75.6 -> 49.5), or two rows and two
-//    waves across the channels (3 x 128 x 128: 10.4 -> 8.4; with 256 blocks of
-//    it, 1 x 128 x 256, the LDS weights are as fast: 6.9 against 6.3).
+//  - 32 input channels: weights in registers, two rows a wave (k_conv3_rows)
+//    where that leaves a block per CU (8 x 256 x 256, 32 -> 32: 35.3 -> 20.9), with two
+//    waves across the channels where there are 64 (32 -> 64: 42.8 -> 29.2; 1 x 128 x
+//    256: 6.0 -> 5.6).
 //  - otherwise weights in LDS.  Two rows and two channel tiles a wave read half
-//    the LDS bytes a product (8 x 64 x 64, 256 -> 128: 32.6 -> 27.9; 1 x 128 x
-//    256, 64 -> 128: 14.5 -> 13.0) but need four times the pixels to fill the
-//    chip: from 192 blocks on (3 x 128 x 128, 64 -> 64: 12.5 either way; with
-//    96, 3 x 64 x 64, 128 -> 128: 10.5 against 13), and not with a pooled output,
-//    whose epilogue takes it longer than it saves.  Else one row and tile a
+//    the LDS bytes a product (8 x 64 x 64, 256 -> 128: 31.7 -> 26.6; 1 x 128 x
+//    256, 64 -> 128: 13.5 -> 11.7) but need four times the pixels to fill the
+//    chip: from 192 blocks on (3 x 128 x 128, 64 -> 64: 12.3 -> 11.4; with
+//    96, 3 x 64 x 64, 128 -> 128: 10.0 against 13).  Else one row and tile a
 //    wave, 64-channel chunks where that leaves at most a block a CU anyway, and
 //    the input chunks split over blocks while those cover fewer than half the
 //    CUs (at 128..255 blocks the split's extra pass costs more than it gains).
-ConvPlan conv3_plan(int N, int H, int W, int Cin, int Cout, bool pooled = false) {
+ConvPlan conv3_plan(int N, int H, int W, int Cin, int Cout) {
     constexpr int k111 = 0, k211 = 1, k221 = 4, k212 = 6;  // indices into kTiles3
     if (Cin == 32 && Cout == 32) return {conv3_blocks(k211, N, H, W, Cout) >= 256 ? k211 : k111, 1, 0};
     const bool wide = Cout % 64 == 0;
-    if (Cin == 32 && wide && conv3_blocks(k221, N, H, W, Cout) >= 1024) return {k221, 1, 0};
-    if (Cin == 32 && wide && conv3_blocks(k212, N, H, W, Cout) >= 384) return {k212, 1, 0};
-    if (wide && !pooled && conv3_blocks(k221, N, H, W, Cout) >= 192) return {k221, 1, 1};
+    if (Cin == 32 && wide && conv3_blocks(k212, N, H, W, Cout) >= 256) return {k212, 1, 0};
+    if (wide && conv3_blocks(k221, N, H, W, Cout) >= 192) return {k221, 1, 1};
     const long long blocks = conv3_blocks(k111, N, H, W, Cout);
     const int kind = Cin % 64 == 0 && blocks <= 256 ? 2 : 1;
     int split = 1;
@@ -1420,13 +1438,13 @@ void conv_fwd(hipStream_t s, int ks, const ConvIn &in, const uint16_t *w, const 
         HIPCHK(hipGetLastError());
         return;
     }
-    // the 3x3 epilogues move four channels of bias, partial sums and pooled
-    // output at a time and 16 bytes of output
+    // the 3x3 epilogues move four channels of bias and partial sums and 16 bytes
+    // of output at a time
     auto aligned = [](const void *q, uintptr_t a) { return ((uintptr_t)q & (a - 1)) == 0; };
     ucheck((!bias || aligned(bias, 16)) && aligned(out, 16) && (!ws || aligned(ws, 16)) &&
-               (!pool_out || aligned(pool_out, 8)),
-           "convolution buffers must be 16-byte aligned (8 for pooled outputs)");
-    ConvPlan pl = conv3_plan(N, H, W, Cin, Cout, pool_out != nullptr);
+               (!pool_out || aligned(pool_out, 16)),
+           "convolution buffers must be 16-byte aligned");
+    ConvPlan pl = conv3_plan(N, H, W, Cin, Cout);
     if (force.tile) {  // a forced block shape runs on the halo-only kernel unless the kind is forced too
         pl.tile = force.tile - 1;
         pl.kind = 0;
