@@ -1075,6 +1075,7 @@ __global__ __launch_bounds__(256) void k_wgrad_sum(const float *__restrict__ par
     const size_t i = (size_t)blockIdx.x * 64 + 4 * e;
     float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (i < n)
+#pragma unroll 8
         for (int z = k; z < splits; z += 16) {
             const float4 v = *(const float4 *)(part + (size_t)z * stride + i);
             s.x += v.x;
