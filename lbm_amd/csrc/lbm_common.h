@@ -31,6 +31,11 @@ struct Geom {
     F16Shift sh;        // shift of the binary16 storage (off: f - w)
 };
 
+// f32 values a pixel of the surrogate's output tensor: its three outputs and one
+// that nothing reads (with the head's 32 channels a pixel, three of them used, the
+// last layer and its readers moved whole lines for 12 bytes)
+constexpr int kNetOutStride = 4;
+
 // per-cell bounce-back byte: bit(k) set if population k's upstream is solid or
 // outside the grid; 0xFF marks a cell the fast path does not pull (not streamed,
 // or streamed with all eight upstream cells solid)

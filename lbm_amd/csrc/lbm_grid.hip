@@ -145,7 +145,7 @@ __global__ void k_pack_net_input(const float *__restrict__ mom, const uint8_t *_
 // predicted change, bilinearly interpolated from the nx / F x ny / F output
 // grid at the cell centre (exactly the cell's own pixel for F = 1).
 template <class St, int F>
-__global__ void k_apply_jump(const float *__restrict__ net_out, int C, const float *__restrict__ mom,
+__global__ void k_apply_jump(const float *__restrict__ net_out, const float *__restrict__ mom,
                              const uint8_t *__restrict__ mask, typename St::T *buf, Geom g, float d_rho, float d_u) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x;
     const int y = blockIdx.y;
@@ -157,12 +157,14 @@ __global__ void k_apply_jump(const float *__restrict__ net_out, int C, const flo
     const int i0 = min((int)gx, w - 1), j0 = min((int)gy, h - 1);
     const int i1 = min(i0 + 1, w - 1), j1 = min(j0 + 1, h - 1);
     const float fx = fminf(gx - (float)i0, 1.0f), fy = fminf(gy - (float)j0, 1.0f);
+    auto pixel = [&](int j, int i) { return *(const float4 *)(net_out + ((size_t)j * w + i) * kNetOutStride); };
+    const float4 o00 = pixel(j0, i0), o01 = pixel(j0, i1), o10 = pixel(j1, i0), o11 = pixel(j1, i1);
+    auto part = [](const float4 &v, int c) { return c == 0 ? v.x : c == 1 ? v.y : v.z; };
     float d[3];
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-        const float o00 = net_out[((size_t)j0 * w + i0) * C + c], o01 = net_out[((size_t)j0 * w + i1) * C + c];
-        const float o10 = net_out[((size_t)j1 * w + i0) * C + c], o11 = net_out[((size_t)j1 * w + i1) * C + c];
-        d[c] = (1.0f - fy) * ((1.0f - fx) * o00 + fx * o01) + fy * ((1.0f - fx) * o10 + fx * o11);
+        d[c] = (1.0f - fy) * ((1.0f - fx) * part(o00, c) + fx * part(o01, c)) +
+               fy * ((1.0f - fx) * part(o10, c) + fx * part(o11, c));
     }
     const float rho0 = mom[2 * g.pstride + i];
     const float rho = rho0 + d_rho * d[0];
@@ -1234,10 +1236,10 @@ int lbm_surrogate_jump(lbm_grid *g, lbm_unet *net, uint32_t steps, float s_rho, 
         by_store(g->precision, [&]<class St>() {
             using T = typename St::T;
             if (fine)
-                hipLaunchKernelGGL((k_apply_jump<St, 1>), grid, dim3(256), 0, g->stream, o, 32, g->now, g->mask,
+                hipLaunchKernelGGL((k_apply_jump<St, 1>), grid, dim3(256), 0, g->stream, o, g->now, g->mask,
                                    (T *)g->f[g->cur], g->geom, d_rho, d_u);
             else
-                hipLaunchKernelGGL((k_apply_jump<St, 2>), grid, dim3(256), 0, g->stream, o, 32, g->now, g->mask,
+                hipLaunchKernelGGL((k_apply_jump<St, 2>), grid, dim3(256), 0, g->stream, o, g->now, g->mask,
                                    (T *)g->f[g->cur], g->geom, d_rho, d_u);
         });
         HIPCHK(hipGetLastError());

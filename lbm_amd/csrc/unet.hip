@@ -400,7 +400,7 @@ __device__ __forceinline__ void conv_pool_tile(const f32x16 (&acc)[MI][NI], cons
 }
 
 // A 1x1 convolution applied to a 3x3 convolution's output inside its
-// epilogue (the network's head): out[p * cout + o] = b[o] + sum_c w[o][c] y[p][c]
+// epilogue (the network's head): out[p * stride + o] = b[o] + sum_c w[o][c] y[p][c]
 // in f32 for o < store rounded up to a multiple of 4 (outputs are stored four
 // at a time), y the stored (bf16) output of a 32-channel layer and w
 // [cout = 32][32] bf16.  Null w: none.
@@ -408,7 +408,7 @@ struct ConvHead {
     const uint16_t *w = nullptr;
     const float *b = nullptr;
     float *out = nullptr;
-    int cout = 0, store = 0;
+    int cout = 0, store = 0, stride = 0;
 };
 
 // One more product per row of the wave, on values the wave already holds: the
@@ -452,7 +452,7 @@ __device__ __forceinline__ void conv_head_tile(const f32x16 (&acc)[MI][1], const
                 const int o = 8 * g + 4 * half;  // four consecutive outputs, stored as one vector
                 if (o < hd.store) {
                     const float4 hb = *(const float4 *)&hd.b[o];
-                    *(float4 *)&hd.out[p * hd.cout + o] =
+                    *(float4 *)&hd.out[p * hd.stride + o] =
                         make_float4(d[4 * g] + hb.x, d[4 * g + 1] + hb.y, d[4 * g + 2] + hb.z, d[4 * g + 3] + hb.w);
                 }
             }
@@ -1219,12 +1219,12 @@ __global__ __launch_bounds__(kSumBlocks) void k_weight_inverse(const double *__r
     }
 }
 
-// masked mean-square loss on the first three of 32 output channels and its
-// gradient: loss = sum_p wm[p] sum_{c<3} (out[p][c] - tgt[p][c])^2 / sum_p wm[p].
+// masked mean-square loss on the three outputs and its gradient: loss = sum_p wm[p] sum_{c<3} (out[p][c] - tgt[p][c])^2 / sum_p wm[p].
 // Four threads a pixel, each one 16-byte store of the gradient's 32 channels;
 // kMseBlocks blocks walk over the pixels and end in one atomic each.  (Channel by
 // channel a thread wrote two bytes at a time, and an atomic a wave on the one
-// address of the loss took most of 122 us for 524288 pixels; now 25.)
+// address of the loss took most of 122 us for 524288 pixels; 25 so, and less with
+// four output values a pixel in memory instead of 32.)
 constexpr int kMseBlocks = 512;
 __global__ __launch_bounds__(256) void k_mse(const float *__restrict__ out, const float *__restrict__ tgt,
                                              const float *__restrict__ wm, uint16_t *__restrict__ gout,
@@ -1238,7 +1238,7 @@ __global__ __launch_bounds__(256) void k_mse(const float *__restrict__ out, cons
         u16x8 g = u16x8{};
         if (part == 0) {
             const float w = wm[p];
-            const float4 o = *(const float4 *)(out + p * 32);
+            const float4 o = *(const float4 *)(out + p * kNetOutStride);
             const float v[3] = {o.x, o.y, o.z};
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
@@ -1256,22 +1256,24 @@ __global__ __launch_bounds__(256) void k_mse(const float *__restrict__ out, cons
     if (threadIdx.x == 0) atomicAdd(loss, ((red[0] + red[1]) + (red[2] + red[3])) * inv);
 }
 
-// network input from host fields: x[p] = (the kNetIn host channels, then zeros)
-__global__ void k_pack_input(const float *__restrict__ fields, uint16_t *__restrict__ x, long long P, int C) {
-    const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+// network input from host fields: x[p] = (the kNetIn host channels, then zeros),
+// 32 channels, four threads a pixel
+__global__ void k_pack_input(const float *__restrict__ fields, uint16_t *__restrict__ x, long long P) {
+    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x, p = t >> 2;
     if (p >= P) return;
-    const float4 f0 = *(const float4 *)(fields + p * 8), f1 = *(const float4 *)(fields + p * 8 + 4);
-    u16x8 v;
-    v[0] = f2bf(f0.x);
-    v[1] = f2bf(f0.y);
-    v[2] = f2bf(f0.z);
-    v[3] = f2bf(f0.w);
-    v[4] = f2bf(f1.x);
-    v[5] = f2bf(f1.y);
-    v[6] = f2bf(f1.z);
-    v[7] = f2bf(f1.w);
-    *(u16x8 *)(x + p * C) = v;
-    for (int c = 8; c < C; c += 8) *(u16x8 *)(x + p * C + c) = u16x8{};
+    u16x8 v = u16x8{};
+    if ((t & 3) == 0) {
+        const float4 f0 = *(const float4 *)(fields + p * 8), f1 = *(const float4 *)(fields + p * 8 + 4);
+        v[0] = f2bf(f0.x);
+        v[1] = f2bf(f0.y);
+        v[2] = f2bf(f0.z);
+        v[3] = f2bf(f0.w);
+        v[4] = f2bf(f1.x);
+        v[5] = f2bf(f1.y);
+        v[6] = f2bf(f1.z);
+        v[7] = f2bf(f1.w);
+    }
+    *(u16x8 *)(x + t * 8) = v;
 }
 
 // the network's three outputs per pixel, of `stride` stored ones, as dense
@@ -1397,12 +1399,12 @@ size_t conv_split_elems(int ks, long long P, int N, int H, int W, int Cin, int C
     return pl.split > 1 ? (size_t)pl.split * P * Cout : 0;
 }
 
-// Launch a convolution (also used for input gradients): 3x3 on k_conv3_lds or
-// k_conv3_lw (conv3_plan), 1x1 on k_conv1x1.  Only channels co < co_store are
-// stored (all of them when the K split is taken).  pool_out: also the output's
-// 2 x 2 average pool; head: also a 1x1 head on the output (ConvHead); both in
-// the epilogue where the block shape allows, else as passes of their own.  gate:
-// see conv_store_tile.
+// Launch a convolution (also used for input gradients): 3x3 on k_conv3_rows,
+// k_conv3_lds or k_conv3_lw (conv3_plan), 1x1 on k_conv1x1.  Only channels co <
+// co_store are stored (all of them when the K split is taken).  pool_out: also
+// the output's 2 x 2 average pool, in the epilogue where the block shape allows,
+// else as a pass of its own; head: also a 1x1 head on the output (ConvHead).
+// gate: see conv_store_tile.
 void conv_fwd(hipStream_t s, int ks, const ConvIn &in, const uint16_t *w, const float *bias, void *out, int N, int H,
               int W, int Cout, bool relu, bool out_f32, int co_store, float *ws, size_t ws_elems,
               ConvTile force = ConvTile{}, uint16_t *pool_out = nullptr, ConvHead head = ConvHead{},
@@ -1469,13 +1471,13 @@ void conv_fwd(hipStream_t s, int ks, const ConvIn &in, const uint16_t *w, const 
     ucheck(!pool_out || (!out_f32 && co_store == Cout && H % 2 == 0), "pooled output needs a full bf16 output");
     const bool fuse_pool = pool_out && !split && (kTiles3[t][0] == 2 || (kTiles3[t][0] == 1 && kTiles3[t][2] == 1));
     uint16_t *pout = fuse_pool ? pool_out : nullptr;
-    // a 1x1 head rides in the epilogue of the per-wave-weights kernel when one
-    // wave holds all 32 output channels of its pixels; otherwise its own pass
-    ucheck(!head.w || (Cout == 32 && !out_f32 && co_store == Cout && head.b && head.out && head.store <= 32 &&
-                       head.cout == 32 && aligned(head.w, 8) && aligned(head.b, 16) && aligned(head.out, 16)),
-           "head: a bf16 32-channel layer, 32 x 32 weights, 32 f32 outputs per pixel");
-    const bool fuse_head = head.w && kind == 0 && !split && kTiles3[t][1] == 1 && kTiles3[t][2] == 1;
-    const ConvHead hd = fuse_head ? head : ConvHead{};
+    // a 1x1 head rides in the epilogue of the kernels whose waves hold all 32
+    // output channels of their pixels
+    ucheck(!head.w || (Cout == 32 && !out_f32 && co_store == Cout && head.b && head.out &&
+                       (head.store + 3) / 4 * 4 <= head.stride && head.stride % 4 == 0 && head.cout == 32 &&
+                       aligned(head.w, 8) && aligned(head.b, 16) && aligned(head.out, 16) && kind == 0 && !split &&
+                       kTiles3[t][1] == 1 && kTiles3[t][2] == 1),
+           "head: a bf16 layer of 32 to 32 channels, 32 x 32 weights, f32 outputs four at a time");
     // one plain 32-channel input, two rows a wave: k_conv3_rows, in runs that
     // leave two blocks a CU (its index of a pixel's channels is 32 bits)
     const bool in_rows = kind == 0 && (t == 1 || t == 6) && in.ca == 32 && in.cb == 0 && !in.a_up &&
@@ -1485,11 +1487,11 @@ void conv_fwd(hipStream_t s, int ks, const ConvIn &in, const uint16_t *w, const 
         const int rows = (int)std::max(1ll, std::min<long long>(tiles_y, (long long)grid.x * grid.y / 512));
         const dim3 rgrid((unsigned)(N * (W / 32) * ((tiles_y + rows - 1) / rows)), grid.y);
         if (t == 1)
-            hipLaunchKernelGGL(k_conv3_rows<1>, rgrid, dim3(256), 0, s, in.a, w, bias, out, pout, hd, gate, N, H, W,
-                               Cout, co_store, r, f, rows);
+            hipLaunchKernelGGL(k_conv3_rows<1>, rgrid, dim3(256), 0, s, in.a, w, bias, out, pout, head, gate, N, H,
+                               W, Cout, co_store, r, f, rows);
         else
-            hipLaunchKernelGGL(k_conv3_rows<2>, rgrid, dim3(256), 0, s, in.a, w, bias, out, pout, hd, gate, N, H, W,
-                               Cout, co_store, r, f, rows);
+            hipLaunchKernelGGL(k_conv3_rows<2>, rgrid, dim3(256), 0, s, in.a, w, bias, out, pout, head, gate, N, H,
+                               W, Cout, co_store, r, f, rows);
     }
 #define L3(MI, NI, WN)                                                                                             \
     do {                                                                                                           \
@@ -1500,7 +1502,7 @@ void conv_fwd(hipStream_t s, int ks, const ConvIn &in, const uint16_t *w, const 
             hipLaunchKernelGGL((k_conv3_lw<MI, NI, (32 * NI * WN <= 64 ? WN : 1)>), grid, dim3(256), 0, s, in, w,   \
                                bias, out, ws, pout, gate, N, H, W, Cout, co_store, r, f);                                \
         else                                                                                                       \
-            hipLaunchKernelGGL((k_conv3_lds<MI, NI, WN>), grid, dim3(256), 0, s, in, w, bias, out, ws, pout, hd, gate, \
+            hipLaunchKernelGGL((k_conv3_lds<MI, NI, WN>), grid, dim3(256), 0, s, in, w, bias, out, ws, pout, head, gate, \
                                N, H, W, Cout, co_store, r, f);                                                        \
     } while (0)
     if (!in_rows) switch (t) {
@@ -1536,9 +1538,6 @@ void conv_fwd(hipStream_t s, int ks, const ConvIn &in, const uint16_t *w, const 
                            pool_out, N, H, W, Cout);
         HIPCHK(hipGetLastError());
     }
-    if (head.w && !fuse_head)
-        conv_fwd(s, 1, one_input((const uint16_t *)out, 32), head.w, head.b, head.out, N, H, W, head.cout, false, true,
-                 head.store, ws, ws_elems);
 }
 
 // Tile height and wave grid of the weight gradient: 64 x 64 channels a block
@@ -1741,7 +1740,7 @@ struct lbm_unet {
         wb = (uint16_t *)alloc(nweight * 2);
         wt = (uint16_t *)alloc(nweight * 2);
         const size_t P = (size_t)B * H * W;
-        out32 = (float *)alloc(P * 32 * 4);
+        out32 = (float *)alloc(P * kNetOutStride * 4);
         gout = (uint16_t *)alloc(P * 32 * 2);
         tgt = (float *)alloc(P * 3 * 4);
         wm = (float *)alloc(P * 4);
@@ -1849,6 +1848,7 @@ struct lbm_unet {
         hd.b = w32 + h.boff;
         hd.out = out32;
         hd.cout = h.cout;
+        hd.stride = kNetOutStride;
         hd.store = 3;
         conv_fwd(stream, c16.ks, one_input(d1a.a, d1a.C), wb + c16.wboff, w32 + c16.boff, d1.a, B, H, W, c16.cout,
                  c16.relu, false, c16.cout, ws, ws_elems, ConvTile{}, nullptr, hd);
@@ -1917,7 +1917,7 @@ struct lbm_unet {
         const size_t P = (size_t)B * H * W;
         const Piece in[3] = {{(void *)hx, fields, P * 32}, {(void *)hy, tgt, P * 12}, {(void *)hwm, wm, P * 4}};
         HIPCHK(staging.copy(dev, stream, in, 3, false));
-        hipLaunchKernelGGL(k_pack_input, dim3(nblk(P)), dim3(256), 0, stream, fields, x.a, (long long)P, 32);
+        hipLaunchKernelGGL(k_pack_input, dim3(nblk(4 * P)), dim3(256), 0, stream, fields, x.a, (long long)P);
         forward();
         hipLaunchKernelGGL(k_weight_sum, dim3(kSumBlocks), dim3(256), 0, stream, wm, wsums, P);
         hipLaunchKernelGGL(k_weight_inverse, dim3(1), dim3(kSumBlocks), 0, stream, wsums, wsums + kSumBlocks, inv_wsum,
@@ -2071,11 +2071,11 @@ int lbm_unet_forward(lbm_unet *n, const float *x, float *y) {
         const size_t P = (size_t)n->B * n->H * n->W;
         const Piece in{(void *)x, n->fields, P * 32}, res{y, n->fields, P * 12};
         HIPCHK(n->staging.copy(n->dev, n->stream, &in, 1, false));
-        hipLaunchKernelGGL(k_pack_input, dim3(nblk(P)), dim3(256), 0, n->stream, n->fields, n->x.a, (long long)P, 32);
+        hipLaunchKernelGGL(k_pack_input, dim3(nblk(4 * P)), dim3(256), 0, n->stream, n->fields, n->x.a, (long long)P);
         n->forward();
         // through the host fields' buffer, which the pass has read
         hipLaunchKernelGGL(k_dense_output, dim3(nblk(P)), dim3(256), 0, n->stream, n->out32, n->fields, (long long)P,
-                           32);
+                           kNetOutStride);
         HIPCHK(hipGetLastError());
         HIPCHK(n->staging.copy(n->dev, n->stream, &res, 1, true));
     });
