@@ -580,35 +580,45 @@ __global__ void k_walls(uint8_t *__restrict__ mask, Geom g) {
 // Colour maps (color_map/{inferno,viridis,jet}.wgsl): v is scaled and clamped
 // to [-n, n], its integer block picks two neighbouring control colours and the
 // fraction within the block blends them; solid cells are black.  The control
-// colours are the reference's, block -n first.
-__device__ __forceinline__ void colormap_rgb(int map, float v, bool solid, float *rgb) {
-    constexpr float kInferno[5][3] = {{0.98828125f, 1.0f, 0.64453125f},
-                                      {0.97265625f, 0.55859375f, 0.0390625f},
-                                      {0.73828125f, 0.21875f, 0.33203125f},
-                                      {0.34375f, 0.06640625f, 0.43359375f},
-                                      {0.0f, 0.0f, 0.01853125f}};
-    constexpr float kViridis[5][3] = {{0.9921875f, 0.90625f, 0.1484375f},
-                                      {0.3671875f, 0.7890625f, 0.3828125f},
-                                      {0.1328125f, 0.56640625f, 0.55078125f},
-                                      {0.23046875f, 0.32421875f, 0.546875f},
-                                      {0.265625f, 0.0078125f, 0.33203125f}};
-    constexpr float kJet[9][3] = {{0.0f, 0.0f, 0.5f}, {0.0f, 0.0f, 1.0f}, {0.0f, 0.5f, 1.0f},
-                                  {0.0f, 1.0f, 1.0f}, {0.5f, 1.0f, 0.5f}, {1.0f, 1.0f, 0.0f},
-                                  {1.0f, 0.5f, 0.0f}, {1.0f, 0.0f, 0.0f}, {0.5f, 0.0f, 0.0f}};
+// colours are the reference's, block -n first: kMapColours[map], 2 n + 1 of them.
+__device__ constexpr float kMapColours[3][9][3] = {
+    {{0.98828125f, 1.0f, 0.64453125f},
+     {0.97265625f, 0.55859375f, 0.0390625f},
+     {0.73828125f, 0.21875f, 0.33203125f},
+     {0.34375f, 0.06640625f, 0.43359375f},
+     {0.0f, 0.0f, 0.01853125f}},
+    {{0.9921875f, 0.90625f, 0.1484375f},
+     {0.3671875f, 0.7890625f, 0.3828125f},
+     {0.1328125f, 0.56640625f, 0.55078125f},
+     {0.23046875f, 0.32421875f, 0.546875f},
+     {0.265625f, 0.0078125f, 0.33203125f}},
+    {{0.0f, 0.0f, 0.5f},
+     {0.0f, 0.0f, 1.0f},
+     {0.0f, 0.5f, 1.0f},
+     {0.0f, 1.0f, 1.0f},
+     {0.5f, 1.0f, 0.5f},
+     {1.0f, 1.0f, 0.0f},
+     {1.0f, 0.5f, 0.0f},
+     {1.0f, 0.0f, 0.0f},
+     {0.5f, 0.0f, 0.0f}}};
+__device__ __forceinline__ int colour_table(int map) {
+    return map == LBM_COLORMAP_JET ? 2 : map == LBM_COLORMAP_VIRIDIS ? 1 : 0;
+}
+// tab: the map's 27 table values
+__device__ __forceinline__ void colormap_rgb(int map, const float *tab, float v, bool solid, float *rgb) {
     const bool jet = map == LBM_COLORMAP_JET;
     const int n = jet ? 4 : 2;
     const float c = fminf(fmaxf((jet ? 20.0f : 15.0f) * v, -(float)n), (float)n);
     const int b = (int)floorf(c);
-    const float (*tab)[3] = jet ? kJet : (map == LBM_COLORMAP_VIRIDIS ? kViridis : kInferno);
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         if (solid) {
             rgb[k] = 0.0f;
         } else if (b >= n) {
-            rgb[k] = tab[2 * n][k];
+            rgb[k] = tab[3 * 2 * n + k];
         } else {
             const float w = (float)(-b) + c;  // right_weight = -block + color
-            rgb[k] = (1.0f - w) * tab[b + n][k] + w * tab[b + n + 1][k];
+            rgb[k] = (1.0f - w) * tab[3 * (b + n) + k] + w * tab[3 * (b + n + 1) + k];
         }
     }
 }
@@ -633,45 +643,58 @@ __global__ void k_place_mask(const uint8_t *__restrict__ src, uint8_t *__restric
     mask[(size_t)blockIdx.y * pitch + x] = src[(size_t)blockIdx.y * X + x] == 1 ? 1 : 0;
 }
 
-// summary passes (summary_stats/{curl,ux,uy,rho,speed}.wgsl); out keeps the
-// values of cells a pass skips.  With rgb, the colour map `map` of the whole
-// plane follows in the same pass (3 floats per cell, dense rows); with dense,
-// the plane is also written with dense rows, for the host's copy (see
-// k_dense_planes).
-__global__ void k_summary(const float *__restrict__ mom, float *__restrict__ out, const uint8_t *__restrict__ mask,
-                          float *__restrict__ rgb, float *__restrict__ dense, Geom g, int kind, int map) {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    const int y = blockIdx.y;
-    if (x >= g.X) return;
+// one cell of the summary passes (summary_stats/{curl,ux,uy,rho,speed}.wgsl)
+__device__ __forceinline__ float summary_value(const float *__restrict__ mom, const float *out, const Geom &g, int kind,
+                                               int x, int y) {
     const long long ps = g.pstride;
     const float *jx = mom, *jy = mom + ps, *rho = mom + 2 * ps;
     const size_t i = (size_t)y * g.pitch + x;
-    float v;
     switch (kind) {
     case LBM_SUMMARY_CURL: {
-        if (x == 0 || y >= g.Y - 1) {
-            v = out[i];  // not written by the curl pass: the previous value stays
-            break;
-        }
+        if (x == 0 || y >= g.Y - 1) return out[i];  // not written by the curl pass: the previous value stays
         // flattened neighbours: x+1 at the last column is column 0 of the next row
         const int xe = x + 1 < g.X ? x + 1 : 0, ye = x + 1 < g.X ? y : y + 1;
         const float uye = jy[(size_t)ye * g.pitch + xe];
         const float uyw = jy[i - 1];
         const float uxn = y > 0 ? jx[i - g.pitch] : 0.0f;
         const float uxs = jx[i + g.pitch];
-        v = 10.0f * (uye - uyw - uxn + uxs) / rho[i];
-        break;
+        return 10.0f * (uye - uyw - uxn + uxs) / rho[i];
     }
-    case LBM_SUMMARY_UX: v = jx[i]; break;
-    case LBM_SUMMARY_UY: v = jy[i]; break;
-    case LBM_SUMMARY_RHO: v = 4.0f * fminf(fmaxf(0.15f * rho[i], 0.0f), 1.0f) - 0.5f; break;
-    default: v = fminf(fmaxf(5.0f * sqrtf(jx[i] * jx[i] + jy[i] * jy[i]), 0.0f), 1.0f) - 0.5f; break;
+    case LBM_SUMMARY_UX: return jx[i];
+    case LBM_SUMMARY_UY: return jy[i];
+    case LBM_SUMMARY_RHO: return 4.0f * fminf(fmaxf(0.15f * rho[i], 0.0f), 1.0f) - 0.5f;
+    default: return fminf(fmaxf(5.0f * sqrtf(jx[i] * jx[i] + jy[i] * jy[i]), 0.0f), 1.0f) - 0.5f;
     }
-    out[i] = v;
-    if (dense) dense[(size_t)y * g.X + x] = v;
-    if (rgb) colormap_rgb(map, v, mask[i] == 1, rgb + 3 * ((size_t)y * g.X + x));
 }
 
+// summary passes; out keeps the
+// values of cells a pass skips.  With rgb, the colour map `map` of the whole
+// plane follows in the same pass (3 floats per cell, dense rows); with dense,
+// the plane is also written with dense rows, for the host's copy (see
+// k_dense_planes).  Blocks of 256 cells.  Few bytes, so bound by the chain of its
+// loads: the colours wait in LDS for the value, not the other way round, and leave
+// through it in whole lines (640 x 360: 14.6 -> 4.3 us).
+__global__ __launch_bounds__(256) void k_summary(const float *__restrict__ mom, float *__restrict__ out,
+                                                 const uint8_t *__restrict__ mask, float *__restrict__ rgb,
+                                                 float *__restrict__ dense, Geom g, int kind, int map) {
+    __shared__ float tab[27], row[3 * 256];
+    const int x = blockIdx.x * 256 + threadIdx.x;
+    const int y = blockIdx.y;
+    if (rgb && threadIdx.x < 27) tab[threadIdx.x] = (&kMapColours[colour_table(map)][0][0])[threadIdx.x];
+    const float v = x < g.X ? summary_value(mom, out, g, kind, x, y) : 0.0f;
+    if (x < g.X) {
+        out[(size_t)y * g.pitch + x] = v;
+        if (dense) dense[(size_t)y * g.X + x] = v;
+    }
+    if (!rgb) return;
+    const bool solid = x < g.X && mask[(size_t)y * g.pitch + x] == 1;
+    __syncthreads();
+    colormap_rgb(map, tab, v, solid, row + 3 * threadIdx.x);
+    __syncthreads();
+    const int x0 = blockIdx.x * 256, n = 3 * min(256, g.X - x0);
+    float *const to = rgb + 3 * ((size_t)y * g.X + x0);
+    for (int k = threadIdx.x; k < n; k += 256) to[k] = row[k];
+}
 // rho, u = j / rho, curl into four dense planes
 __global__ void k_fields(const float *__restrict__ mom, float *__restrict__ outp, Geom g) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x;
