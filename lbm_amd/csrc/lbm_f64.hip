@@ -41,7 +41,8 @@ __device__ __forceinline__ double plus(double sum, double v) {
 // the second Newton step on the reciprocal that a double takes before the
 // quotient's residual (12 instead of 22 instructions, one reciprocal instead of
 // two, four for the test).  The residual is exact for numerators down to
-// 2^-900; a smaller quotient changes no bit of the collision's sums.
+// 2^-900; a smaller quotient changes no bit of the collision's sums.  Against the
+// plain divisions 20.8 -> 20.3 us a step at 2048 x 1024, 3.9 -> 3.6 at 640 x 320.
 __device__ __forceinline__ void velocity64(double jx, double jy, double rho, double &ux, double &uy) {
     const double top = fmax(fmax(fabs(jx), fabs(jy)), fabs(rho));
     if (__builtin_expect(__all(rho >= 0x1p-20 && top <= 0x1p20), 1)) {
