@@ -17,7 +17,7 @@
 
 #include <cstdint>
 #include <cstring>
-#include <system_error>
+#include <exception>
 #include <thread>
 #include <vector>
 
@@ -90,7 +90,7 @@ struct Staging {
         int started = 1;
         try {
             for (; started < kThreads; ++started) threads[started] = std::thread(work, started);
-        } catch (const std::system_error &) {  // no more threads: their shares are done here
+        } catch (const std::exception &) {  // no thread, or no memory for one: the shares left are done here
         }
         work(0);
         for (int t = started; t < kThreads; ++t) work(t);
