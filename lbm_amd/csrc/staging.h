@@ -11,6 +11,10 @@
 // An object (grid, batch, network, solver) owns one Staging, made on its first
 // large copy and freed with it; it is used by the object's own calls only, which
 // are not concurrent.
+//
+// Memory the runtime knows (a caller's own pinned buffer) takes the runtime's copy,
+// which is one transfer at the link's rate: three planes of 8192 x 4096 into
+// pinned memory 7.1 ms that way, 12.7 through the chunks.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -63,13 +67,25 @@ struct Staging {
         buf = nullptr;
     }
 
+    // is every piece's host memory the process's own, unknown to the runtime?
+    static bool ordinary(const Piece *pieces, int n) {
+        for (int i = 0; i < n; ++i) {
+            hipPointerAttribute_t a;
+            if (hipPointerGetAttributes(&a, pieces[i].host) != hipSuccess)
+                (void)hipGetLastError();  // (how older runtimes answer for such memory)
+            else if (a.type != hipMemoryTypeUnregistered)
+                return false;
+        }
+        return true;
+    }
+
     // Copies the pieces in stream order after the stream's earlier work.  Out of
     // the device it returns when they are there; into it, the caller waits for
     // the stream before it gives the host memory back.
     hipError_t copy(int dev, hipStream_t s, const Piece *pieces, int n, bool out) {
         size_t total = 0;
         for (int i = 0; i < n; ++i) total += pieces[i].bytes;
-        if (total < (out ? kLeastOut : kLeastIn) || !ready()) {
+        if (total < (out ? kLeastOut : kLeastIn) || !ordinary(pieces, n) || !ready()) {
             for (int i = 0; i < n; ++i) {
                 const Piece &p = pieces[i];
                 const hipError_t e = out ? hipMemcpyAsync(p.host, p.device, p.bytes, hipMemcpyDeviceToHost, s)

@@ -33,6 +33,12 @@ def test_every_byte_arrives(tool, way, sizes, chunked):
 
 
 @pytest.mark.parametrize("way", ["out", "in"])
+def test_pinned_memory_goes_straight(tool, way):
+    """The runtime copies a caller's pinned buffer itself: no chunks, no error left behind."""
+    assert tool("pinned", way, 13 * MB + 11) == (0, "ok host_mallocs=0")
+
+
+@pytest.mark.parametrize("way", ["out", "in"])
 @pytest.mark.parametrize("nth", [0, 1, 2])
 def test_a_thread_that_cannot_be_made(tool, way, nth):
     """Its share is copied by the calling thread; the process goes on."""
