@@ -328,40 +328,6 @@ __global__ __launch_bounds__(64 * NW, NW / 2) void k64_tile(const double *__rest
     }
 }
 
-// Block shapes as in tile.h, fitted to launches of 1 to 8 steps over 0.006 to 4
-// million cells (within 20% / 38% / 44%, the largest errors where a round is
-// barely begun).  Best us per step of each: 300 x 150 1.95 / 2.71 / 3.88, 640 x
-// 320 4.24 / 3.65 / 4.05, 2048 x 1024 32.4 / 22.7 / 20.2.  Taller regions of
-// three and four rows a wave leave one block a CU, whose loads nothing then
-// hides (3 x 12: 25.9, 4 x 12: 25.7).
-constexpr TileShape kTile64[3] = {{1, 16, false, 0.0f, 0.37f, 5.47f, 0.66f},
-                                  {2, 12, false, 0.0f, 0.93f, 6.67f, 0.95f},
-                                  {4, 8, false, 0.0f, 1.17f, 8.21f, 1.48f}};
-
-// A call's launches: their number is odd, as they go from g to f to g ... and
-// the last one has to end in f, which holds the cells the stream does not write.
-TilePlan plan64(int X, int Y, uint32_t n) {
-    TilePlan best{0, 0};
-    float least = 0.0f;
-    for (int i = 0; i < 3; ++i) {
-        const TileShape &sh = kTile64[i];
-        float cost[kTileMaxSteps + 2] = {};
-        for (int s = 1; s <= kTileMaxSteps; ++s)
-            cost[s] = tile_cost(sh, s, (double)tile_nbx(X, s) * tile_nby(Y, sh.waves * sh.m, s));
-        for (int s = 1; s <= kTileMaxSteps; ++s) {
-            const uint32_t launches = ((n + s - 1) / s) | 1u;
-            if (launches > n) continue;
-            const uint32_t low = n / launches, more = n % launches;
-            const float c = cost[low] * (float)(launches - more) + cost[low + 1] * (float)more;
-            if (!best.launches || c < least) {
-                best = TilePlan{i, launches};
-                least = c;
-            }
-        }
-    }
-    return best;
-}
-
 // rho, u = j / rho (uy north-positive, as the reference's uy field)
 __global__ void k64_macro(const double *__restrict__ f, double *__restrict__ out, size_t n) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;

@@ -2,12 +2,11 @@
 // shared by the single grid (k_tile in lbm_grid.hip) and the batched engine.
 #pragma once
 
-#include <algorithm>
 #include <atomic>
-#include <cmath>
 #include <type_traits>
 
 #include "lbm_common.h"
+#include "tile_plan.h"
 
 namespace {
 
@@ -49,89 +48,6 @@ struct TileArgs {
     int nbx, nby;      // regions across and down
     int sform, final;  // A is S_n; the call's last launch
 };
-
-constexpr int kTileMaxSteps = 8;
-// steps an autotuner times a tile variant for at least: launches of a few steps
-// (two of three in a call of six) say little about those of a long call
-constexpr uint32_t kTileTimedSteps = 48;
-
-// Block shapes: rows a wave, waves, where the unstreamed cells' previous
-// populations live, and the launch's cost.  Without `chain` every cell has a
-// place for them in LDS and solid cells are stepped like any other; with it only
-// column 0, column X and the last row have one and solid cells, which nothing
-// pulls from, are stepped on their own at the end (three rows a wave would need
-// 72 KB a block more).
-//
-// us = fixed + step * steps + rounds * (block + block_step * steps), rounds the
-// regions each CU works off one after the other: fitted to launches of 2 to 8
-// steps over 0.06 to 33 million cells (within 9% / 32% / 14% / 16%, the largest
-// errors where a round is barely begun).
-struct TileShape {
-    int m, waves;
-    bool chain;
-    float fixed, step, block, block_step;
-};
-constexpr TileShape kTileF32[2] = {{1, 16, false, 2.18f, 0.58f, 2.43f, 0.26f}, {3, 12, true, 0.0f, 2.28f, 7.6f, 0.53f}};
-constexpr TileShape kTileF16[2] = {{1, 16, false, 2.28f, 0.56f, 2.33f, 0.29f}, {2, 16, false, 1.7f, 1.03f, 4.73f, 0.6f}};
-template <class T>
-constexpr const TileShape &tile_shape(int i) { return sizeof(T) == 4 ? kTileF32[i] : kTileF16[i]; }
-inline const TileShape &tile_shape(int precision, int i) {
-    return precision == LBM_PRECISION_F32 ? kTileF32[i] : kTileF16[i];
-}
-
-// regions that cover n cells when each of `size` cells keeps all but 2 h
-__host__ __device__ inline int tile_regions(int n, int size, int h) {
-    return n <= size ? 1 : 1 + (n - size + (size - 2 * h) - 1) / (size - 2 * h);
-}
-// (column X counts: the outlet's wrapped pulls; so does the row above the grid)
-__host__ __device__ inline int tile_nbx(int X, int steps) { return tile_regions(X + 1, 64, steps - 1); }
-__host__ __device__ inline int tile_nby(int Y, int rows, int steps) { return tile_regions(Y + 1, rows, steps - 1); }
-
-inline float tile_cost(const TileShape &sh, int steps, double blocks) {
-    double rounds = std::max(1.0, blocks / 256.0);
-    if (rounds < 4.0) rounds = std::ceil(rounds);
-    return (float)(sh.fixed + sh.step * steps + rounds * (sh.block + sh.block_step * steps));
-}
-
-// How a call of n >= 2 steps is cut into launches, each of them n / launches
-// steps or one more: the shape (of `first` .. `last`) and number of launches of
-// least cost (no launches: none fits a grid of blocks).  blocks(shape index,
-// steps): the regions of a launch.
-struct TilePlan {
-    int shape;
-    uint32_t launches;
-};
-//
-// even: an even number of launches where n is even.  Every launch trades the
-// state and spare sets, so a call of even length then leaves each where it
-// was, as the one-step kernel's calls do: a caller's graph of such a call can be
-// replayed.
-template <class F>
-TilePlan tile_plan(int precision, int first, int last, uint32_t n, bool even, F &&blocks) {
-    TilePlan best{first, 0};
-    float least = 0.0f;
-    for (int i = first; i <= last; ++i) {
-        const TileShape &sh = tile_shape(precision, i);
-        float cost[kTileMaxSteps + 1] = {};
-        for (int s = 2; s <= kTileMaxSteps; ++s) {
-            const int64_t nb = blocks(i, s);
-            cost[s] = nb * 64 * sh.waves < (int64_t)1 << 32 ? tile_cost(sh, s, (double)nb) : INFINITY;
-        }
-        for (int s = 2; s <= kTileMaxSteps; ++s) {
-            uint32_t launches = (n + s - 1) / s;
-            if (even && n % 2 == 0) launches += launches % 2;
-            const uint32_t low = n / launches;
-            if (low < 2) continue;
-            const uint32_t more = n % launches;
-            const float c = cost[low] * (float)(launches - more) + (more ? cost[low + 1] * (float)more : 0.0f);
-            if (std::isfinite(c) && (!best.launches || c < least)) {
-                best = TilePlan{i, launches};
-                least = c;
-            }
-        }
-    }
-    return best;
-}
 
 constexpr size_t tile_lds(const TileShape &sh, size_t esize) {
     const size_t prev = sh.chain ? 8 * (size_t)(2 * sh.waves * sh.m + 64) : (size_t)sh.waves * sh.m * 8 * 64;
