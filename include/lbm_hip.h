@@ -153,7 +153,9 @@ int lbm_sync(lbm_grid *g);
  * fails, changing nothing, when it cannot) and frees them when it selects
  * another.  A grid for which no variant was ever set or tuned (lbm_get_variant:
  * 0) runs several steps per launch too where two more sets take at most 512
- * MiB; they are allocated with the grid, if there is memory for them.
+ * MiB; they are allocated with the grid, if there is memory for them and for
+ * what the grid may still allocate, and given back where lbm_set_variant or
+ * lbm_autotune would lack their memory.
  * lbm_autotune times each variant for `steps` steps on the grid's
  * own state, restores that state exactly, selects the fastest, and returns it
  * in *best and the per-step time of every variant in ms[LBM_NUM_VARIANTS]

@@ -383,14 +383,38 @@ struct lbm_batch {
             p = nullptr;
         }
     }
-    // a tile variant's sets; setting one does not take over the default path's
+    // a tile variant's sets, the default path's pair and what may still be
+    // allocated: as a single grid's (lbm_grid.hip)
     void ensure_spare(bool take_over = true) {
         if (spare[0] && (take_over || !auto_path)) return;
         void *fresh[2];
-        make_spare(fresh);
+        without_default_pair([&] { make_spare(fresh); });
         release_spare();
         spare[0] = fresh[0];
         spare[1] = fresh[1];
+    }
+    template <class F>
+    void without_default_pair(F &&allocate) {
+        try {
+            return allocate();
+        } catch (const HipError &) {
+            if (!auto_path || !spare[0]) throw;
+        }
+        HIPCHK(hipStreamSynchronize(stream));
+        release_spare();
+        try {
+            allocate();
+        } catch (...) {
+            try {
+                make_spare(spare);
+            } catch (const HipError &) {
+            }
+            throw;
+        }
+    }
+    // a snapshot, the lists, the largest domain's planes
+    size_t later_bytes() const {
+        return 2 * set_bytes() + 4 * aux_elems * sizeof(float) + 9 * (size_t)max_cells * sizeof(float);
     }
 
     static size_t combination(int shape, int steps) { return (size_t)shape * (kTileMaxSteps + 1) + steps; }
@@ -648,7 +672,8 @@ int lbm_batch_create(const lbm_domain *doms, uint32_t n, int32_t precision, int3
             HIPCHK(hipGetLastError());
         }
         b->build_starts();
-        if (2 * b->alloc_bytes() <= lbm_batch::kAutoSpareBytes) {
+        const size_t pair = 2 * b->alloc_bytes();
+        if (pair <= lbm_batch::kAutoSpareBytes && memory_free(pair + b->later_bytes())) {
             try {
                 b->make_spare(b->spare);
             } catch (const HipError &) {  // no memory for them: one step per launch
@@ -791,7 +816,8 @@ int lbm_batch_autotune(lbm_batch *b, uint32_t steps, int *best, float *ms) {
     return bguard(b, [&] {
         bcheck(steps >= 2, "steps must be >= 2");
         const size_t sb = b->f_elems * b->esize, lb = 3 * b->aux_elems * sizeof(float);
-        char *snap = dalloc<char>(2 * sb + lb);
+        char *snap = nullptr;
+        b->without_default_pair([&] { snap = dalloc<char>(2 * sb + lb); });
         const int cur = b->cur;
         const bool pform = b->pform;
         const uint64_t nsteps = b->steps;

@@ -792,12 +792,28 @@ inline size_t test_alloc_limit() {
     return s && *s ? (size_t)std::strtoull(s, nullptr, 10) : SIZE_MAX;
 }
 
+// Test hook: LBM_TEST_MEM_HIDDEN=<bytes> of the device's free memory count as
+// taken, as if another program held them.
+inline size_t test_mem_hidden() {
+    const char *s = std::getenv("LBM_TEST_MEM_HIDDEN");
+    return s && *s ? (size_t)std::strtoull(s, nullptr, 10) : 0;
+}
+
+// are `bytes` free on the current device?
+inline bool memory_free(size_t bytes) {
+    size_t left = 0, all = 0;
+    HIPCHK(hipMemGetInfo(&left, &all));
+    const size_t hidden = test_mem_hidden();
+    return left >= hidden && left - hidden >= bytes;
+}
+
 template <class T>
 T *dalloc(size_t n) {
     void *p = nullptr;
     if (n == 0) n = 1;
     const size_t bytes = n * sizeof(T);
-    hipError_t e = hipMalloc(&p, bytes > test_alloc_limit() ? (size_t)1 << 62 : bytes);
+    const bool deny = bytes > test_alloc_limit() || (test_mem_hidden() && !memory_free(bytes));
+    hipError_t e = hipMalloc(&p, deny ? (size_t)1 << 62 : bytes);
     if (e != hipSuccess) {
         // the runtime keeps a failed call's status as the thread's last error,
         // which the next launch check would report: clear it, the failure is

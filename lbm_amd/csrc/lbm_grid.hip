@@ -394,7 +394,8 @@ struct lbm_grid {
     // A grid nobody has chosen a variant for has k_tile's two output sets from
     // the start if they take at most this (7 million cells in f32): there a step
     // gains most (400 x 160: 3.7 -> 1.6 us; 2048 x 1024: 28 -> 13 us), and
-    // memory for two more sets is not taken unasked on a large grid.
+    // memory for two more sets is not taken unasked on a large grid, nor where
+    // the grid's own later allocations (later_bytes) would lack it.
     static constexpr size_t kAutoSpareBytes = (size_t)512 << 20;
 
     // two more sets (not in place of the default path's: those stay until the
@@ -419,17 +420,42 @@ struct lbm_grid {
             p = nullptr;
         }
     }
-    // k_tile's sets for a tile variant (setting one does not take over the
-    // default path's: it succeeds exactly when two more sets can be allocated);
-    // the state itself is always in f[0], f[1] between calls
+    // k_tile's sets for a tile variant; the state itself is always in f[0], f[1]
+    // between calls.  Setting a variant does not take over the default path's
+    // pair, as it fails where two more sets cannot be allocated; the pair's own
+    // memory counts as free.
     void ensure_spare(bool take_over = true) {
         if (spare[0] && (take_over || !auto_path)) return;
         void *fresh[2];
-        make_spare(fresh);
+        without_default_pair([&] { make_spare(fresh); });
         release_spare();
         spare[0] = fresh[0];
         spare[1] = fresh[1];
     }
+    // `allocate`, and if there is no memory for it once more with the pair that
+    // was taken unasked given back: that must not be why a call is refused
+    template <class F>
+    void without_default_pair(F &&allocate) {
+        try {
+            return allocate();
+        } catch (const HipError &) {
+            if (!auto_path || !spare[0]) throw;
+        }
+        HIPCHK(hipStreamSynchronize(stream));
+        release_spare();
+        try {
+            allocate();
+        } catch (...) {
+            try {
+                make_spare(spare);  // as it was
+            } catch (const HipError &) {  // (other programs took it: one step per launch)
+            }
+            throw;
+        }
+    }
+    // What the grid may still allocate by its own calls: a snapshot, and planes
+    // of moments, staging, colours and marks.
+    size_t later_bytes() const { return 2 * alloc_bytes() + 20 * (size_t)geom.pstride * sizeof(float); }
 
     template <class St, int MODE, int SHAPE>
     void launch_tile(int steps, bool final) {
@@ -771,7 +797,8 @@ int lbm_create(const lbm_config *cfg, lbm_grid **out) {
         hipLaunchKernelGGL(k_walls, dim3((g->X + 255) / 256), dim3(256), 0, g->stream, g->mask, g->geom);
         HIPCHK(hipGetLastError());
         g->build_flags();
-        if (2 * g->alloc_bytes() <= lbm_grid::kAutoSpareBytes) {
+        const size_t pair = 2 * g->alloc_bytes();
+        if (pair <= lbm_grid::kAutoSpareBytes && memory_free(pair + g->later_bytes())) {
             try {
                 g->make_spare(g->spare);
             } catch (const HipError &) {  // no memory for them: one step per launch
@@ -1009,7 +1036,8 @@ int lbm_autotune(lbm_grid *g, uint32_t steps, int *best, float *ms) {
         check(steps > 0, "steps must be > 0");
         // snapshot the whole evolving state so that tuning leaves no trace
         const size_t sb = g->set_bytes(), lb = 3 * (size_t)g->geom.pstride * sizeof(float);
-        char *snap = dalloc<char>(2 * sb + lb);
+        char *snap = nullptr;
+        g->without_default_pair([&] { snap = dalloc<char>(2 * sb + lb); });
         const int cur = g->cur;
         const bool pform = g->pform;
         const uint64_t nsteps = g->steps;
