@@ -9,11 +9,8 @@ A "step" is one lattice update of the whole grid.  The state is resident in HBM
 before the timed region; K steps run between two stream synchronisations.
 
 Printed: ONE JSON line with the FP32 MLUPS as `value`, the roofline of the
-fused step kernel (72 algorithmic bytes per cell update times the updates one
-launch makes -- six in f32 and five in binary16 for the tile variants, which
-read and write the state once per launch -- over the average launch duration of
-that kernel from HIP events recorded on the grid's own stream; `frac_hbm` the same with
-the launch's measured HBM bytes, calibrated FETCH_SIZE + WRITE_SIZE), the same
+fused step kernel (see roofline(); launch durations from HIP events recorded on
+the grid's own stream, steps per launch as the library plans them), the same
 for FP16-shifted storage (36 B per cell update; f - w, and centred on the
 free-stream equilibrium), both again at 4096 x 2048 and 16384 x 8192
 (grid_leg), the batched configuration's MLUPS (batched_leg, 5000 steps), the
@@ -45,29 +42,44 @@ def log(msg):
 
 
 def read_traffic(name):
-    """HBM bytes per launch of the step kernel from a committed rocprofv3 summary."""
+    """HBM bytes per cell update of the step kernel from a committed rocprofv3
+    summary (calibrated FETCH_SIZE + WRITE_SIZE per launch over the launch's updates)."""
     path = os.path.join(ROOT, "profiles", name)
     if not os.path.exists(path):
         return None
-    m = re.search(r"^traffic_bytes_per_launch:\s*([0-9.eE+]+)", open(path).read(), flags=re.M)
-    return float(m.group(1)) if m else None
+    text = open(path).read()
+    m = re.search(r"^traffic_bytes_per_launch:\s*([0-9.eE+]+)", text, flags=re.M)
+    n = re.search(r"\((\d+) cell updates per launch\)", text)
+    return float(m.group(1)) / (8192 * 4096 * (int(n.group(1)) if n else 1)) if m else None
 
 
-def kernel_name(steps_per_launch):
-    if steps_per_launch == 1:
-        return "k_cell (one step per launch)"
-    return f"k_tile ({steps_per_launch} steps per launch: the state read and written once per launch)"
-
-
-def updates_per_launch(variant, f32=True):
-    """Cell updates per cell in one launch of the step kernel: variants 8 and 9
-    (k_tile) run the number of steps a launch that costs least, at the sizes
-    timed here six in f32 and five in binary16."""
-    return (6 if f32 else 5) if variant is not None and variant >= 8 else 1
+def roofline(fmt, bytes_per_update, cells, kernel, at_8192):
+    """The dominant kernel against the HBM peak.  With one step per launch the
+    kernel is bound by HBM and `achieved` is the algorithmic bytes per cell update
+    over its time.  With several the state is read and written once per launch,
+    the bound is VALU issue, and `achieved` is the measured HBM bytes (8192 x 4096
+    only); the algorithmic bytes of the updates made, which are then not moved, are
+    `effective_gbs`."""
+    us, spl = kernel["kernel_us"], kernel["steps_per_launch"]
+    several = spl > 1
+    traffic = None
+    if at_8192 and (not several or kernel["variant"] == 9):  # (the profiled one)
+        traffic = read_traffic(f"traffic_{fmt}_tile_8192x4096.txt" if several else f"traffic_{fmt}_8192x4096.txt")
+    effective = bytes_per_update * cells * spl / us / 1e3
+    hbm = traffic * cells * spl / us / 1e3 if traffic else None
+    achieved = hbm if several else effective
+    return {"bound": "valu" if several else "hbm", "achieved": round(achieved, 1) if achieved else None,
+            "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4) if achieved else None,
+            "kernel": f"k_tile ({spl:g} steps per launch on average: the state read and written once per launch)"
+                      if several else "k_cell (one step per launch)",
+            "steps_per_launch": spl, "kernel_avg_us": us, "cell_updates_per_launch": round(cells * spl),
+            "traffic": round(traffic * cells * spl) if traffic else None,
+            "frac_hbm": round(hbm / HBM_PEAK_GBS, 4) if hbm else None,
+            "effective_gbs": round(effective, 1), "effective_over_peak": round(effective / HBM_PEAK_GBS, 4)}
 
 
 def run_gpu(precision, X, Y, mask, steps, warmup, omega, u_in, variant=None):
-    from lbm_amd import LBM, PRECISION_F32, LbmError
+    from lbm_amd import LBM, LbmError
     g = LBM(omega, X, Y, precision=precision)
     g.mask = mask
     g.custom_speed(u_in)
@@ -89,17 +101,18 @@ def run_gpu(precision, X, Y, mask, steps, warmup, omega, u_in, variant=None):
     except LbmError as e:  # the flow left BGK's stable range: timing stands, sums do not
         log(f"conservation: {e}")
         cons = None
-    tuned["kernel_us"] = launch_us(g, updates_per_launch(tuned["variant"], precision == PRECISION_F32))
+    tuned.update(launch(g))
     g.close()
     return wall, dev_ms, cons, tuned
 
 
-def launch_us(g, steps_per_launch, launches=40):
-    """Average duration of one launch of the step kernel, from HIP events on the
-    grid's stream, over a call of `launches` launches (the last of them also
+def launch(g, steps=240):
+    """Average duration and steps of one launch of the step kernel, from HIP
+    events on the grid's stream, over a call of 240 steps (the last launch also
     writes the other set and the moments)."""
     g.step_timed(2)
-    return round(g.step_timed(launches * steps_per_launch) / launches * 1e3, 2)
+    n = g.launches(steps)
+    return {"kernel_us": round(g.step_timed(steps) / n * 1e3, 2), "steps_per_launch": round(steps / n, 3)}
 
 
 SURROGATE_WEIGHTS = os.path.join(ROOT, "lbm_amd", "data", "surrogate_f2.npy")
@@ -215,7 +228,7 @@ def grid_leg(X, Y, steps):
         k = dev_ms / 1e3 / steps
         out[name] = {"mlups": round(X * Y / k / 1e6, 1), "us_per_step": round(k * 1e6, 2),
                      "achieved_gbs": round(bpc * X * Y / k / 1e9, 1), "variant": tuned["variant"],
-                     "steps_per_launch": updates_per_launch(tuned["variant"], prec == PRECISION_F32), "steps": steps,
+                     "steps_per_launch": tuned["steps_per_launch"], "steps": steps,
                      "state_finite": cons is not None}
     out["f16s_speedup_vs_f32"] = round(out["f16s"]["mlups"] / out["f32"]["mlups"], 3)
     return out
@@ -224,13 +237,13 @@ def grid_leg(X, Y, steps):
 def batched_leg(n_domains=512, steps=5000):
     """The batched configuration: 512 independent domains (sizes 128x64 ..
     1024x512 in multiples of 32, 1-12 circles/rectangles, tau in [0.52, 0.8],
-    u_in in [0.02, 0.1], all from seed 2024) stepped together; tile variant
-    autotuned, hipGraph replay on.  Whole-batch MLUPS per precision."""
+    u_in in [0.02, 0.1], all from seed 2024) stepped together; variant
+    autotuned.  Whole-batch MLUPS per precision."""
     from lbm_amd import PRECISION_F16S, PRECISION_F32, Batch, gen_batch, gen_shapes
     doms = gen_batch(SEED, n_domains)
     masks = [gen_shapes(nx, ny, 10_000 + i, 1, 12) for i, (nx, ny, _, _) in enumerate(doms)]
     out = {"workload": f"{n_domains} domains from seed {SEED} (128x64..1024x512, 1-12 shapes, tau 0.52-0.8, "
-                       f"u_in 0.02-0.1), {steps} timed steps, hipGraph replay"}
+                       f"u_in 0.02-0.1), {steps} timed steps"}
     for name, prec, bpc in (("f32", PRECISION_F32, 72), ("f16s", PRECISION_F16S, 36)):
         b = Batch(doms, precision=prec)
         for i, m in enumerate(masks):
@@ -238,7 +251,6 @@ def batched_leg(n_domains=512, steps=5000):
         b.step(4)
         cells = b.info()["cells"]
         best, _ = b.autotune(10)
-        b.set_graph(True)
         b.step(20)
         b.sync()
         ms = b.step_timed(steps)
@@ -352,14 +364,9 @@ def main():
     wall, dev_ms, cons, tuned = run_gpu(PRECISION_F32, X, Y, mask, args.steps, args.warmup, omega, u_in,
                                        args.variant)
     mlups = cells * args.steps / wall / 1e6
-    upl = updates_per_launch(tuned["variant"])
-    kern_s = tuned["kernel_us"] / 1e6 / upl  # per cell update pass, from the dominant kernel's launches
-    achieved = 72.0 * cells / kern_s / 1e9
-    log(f"f32: {mlups:.0f} MLUPS, {kern_s * 1e6:.1f} us per step, {upl} step(s) per launch, "
-        f"{achieved:.0f} GB/s algorithmic")
-    traffic = None
-    if (X, Y) == (8192, 4096):
-        traffic = read_traffic("traffic_f32_tile_8192x4096.txt" if upl > 1 else "traffic_f32_8192x4096.txt")
+    rl = roofline("f32", 72.0, cells, tuned, (X, Y) == (8192, 4096))
+    log(f"f32: {mlups:.0f} MLUPS, {tuned['kernel_us'] / tuned['steps_per_launch']:.1f} us per step, "
+        f"{tuned['steps_per_launch']:g} step(s) per launch, {rl['effective_gbs']:.0f} GB/s algorithmic")
 
     out = {
         "metric": METRIC,
@@ -380,21 +387,7 @@ def main():
             "nx": X, "ny": Y, "tau": 0.53, "u_in": u_in, "solid_fraction": round(solid_frac, 4),
             "parallelism": "single GPU",
         },
-        "roofline": {
-            "bound": "hbm",
-            "achieved": round(achieved, 1),
-            "peak": HBM_PEAK_GBS,
-            "unit": "GB/s",
-            "frac": round(achieved / HBM_PEAK_GBS, 4),
-            "traffic": traffic,
-            "kernel": kernel_name(upl),
-            "algorithmic_bytes_per_launch": 72 * cells * upl,
-            "cell_updates_per_launch": cells * upl,
-            "kernel_avg_us": tuned["kernel_us"],
-            # measured HBM bytes (calibrated FETCH_SIZE + WRITE_SIZE) per launch over the launch time
-            "achieved_hbm": round(traffic / (tuned["kernel_us"] * 1e-6) / 1e9, 1) if traffic else None,
-            "frac_hbm": round(traffic / (tuned["kernel_us"] * 1e-6) / 1e9 / HBM_PEAK_GBS, 4) if traffic else None,
-        },
+        "roofline": rl,
         "fp64_mass_momentum": [float(c) for c in cons] if cons is not None else None,
         "autotune": tuned,
     }
@@ -404,24 +397,14 @@ def main():
         w16, d16, c16, tuned16 = run_gpu(PRECISION_F16S, X, Y, mask, args.steps, args.warmup, omega,
                                         u_in, args.f16_variant)
         m16 = cells * args.steps / w16 / 1e6
-        u16 = updates_per_launch(tuned16["variant"], False)
-        k16 = tuned16["kernel_us"] / 1e6 / u16
-        a16 = 36.0 * cells / k16 / 1e9
-        log(f"f16s: {m16:.0f} MLUPS, {k16 * 1e6:.1f} us per step, {u16} step(s) per launch, "
-            f"{a16:.0f} GB/s algorithmic")
-        t16 = (read_traffic("traffic_f16s_8192x4096.txt" if u16 == 1 else "traffic_f16s_tile_8192x4096.txt")
-               if (X, Y) == (8192, 4096) else None)
+        k16 = tuned16["kernel_us"] / 1e6 / tuned16["steps_per_launch"]
+        rl16 = roofline("f16s", 36.0, cells, tuned16, (X, Y) == (8192, 4096))
+        log(f"f16s: {m16:.0f} MLUPS, {k16 * 1e6:.1f} us per step, {tuned16['steps_per_launch']:g} step(s) per launch, "
+            f"{rl16['effective_gbs']:.0f} GB/s algorithmic")
         out["f16s"] = {
             "mlups": round(m16, 1),
             "speedup_vs_f32": round(m16 / mlups, 3),
-            "roofline": {"bound": "hbm", "achieved": round(a16, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                         "frac": round(a16 / HBM_PEAK_GBS, 4), "kernel": kernel_name(u16),
-                         "algorithmic_bytes_per_launch": 36 * cells * u16,
-                         "cell_updates_per_launch": cells * u16, "kernel_avg_us": tuned16["kernel_us"],
-                         "traffic": t16,
-                         "achieved_hbm": round(t16 / (tuned16["kernel_us"] * 1e-6) / 1e9, 1) if t16 else None,
-                         "frac_hbm": round(t16 / (tuned16["kernel_us"] * 1e-6) / 1e9 / HBM_PEAK_GBS, 4)
-                         if t16 else None},
+            "roofline": rl16,
             "fp64_mass_momentum": [float(c) for c in c16] if c16 is not None else None,
             "autotune": tuned16,
         }
@@ -436,7 +419,8 @@ def main():
                                           args.f16_variant)
         m16e = cells * args.steps / w16e / 1e6
         out["f16e"] = {"mlups": round(m16e, 1), "speedup_vs_f32": round(m16e / mlups, 3),
-                       "kernel_avg_us": tuned16e["kernel_us"], "variant": tuned16e["variant"],
+                       "kernel_avg_us": tuned16e["kernel_us"], "steps_per_launch": tuned16e["steps_per_launch"],
+                       "variant": tuned16e["variant"],
                        "fp64_mass_momentum": [float(c) for c in c16e] if c16e is not None else None}
 
     if not args.no_large and not args.no_f16:

@@ -174,6 +174,9 @@ int lbm_autotune(lbm_grid *g, uint32_t steps, int *best, float *ms);
  * rename.  A cached variant that cannot get its spare sets counts as a miss.  LBM_EINVAL when the file cannot be written (the tuned variant is
  * selected all the same).  best and hit may be NULL. */
 int lbm_autotune_cached(lbm_grid *g, const char *cache_path, uint32_t steps, int *best, int *hit);
+/* The launches of the step kernel that lbm_step(g, n) would make now: n with one
+ * step per launch, fewer where several steps share one. */
+int lbm_launches(const lbm_grid *g, uint32_t n, uint32_t *launches);
 /* lbm_step(g, n) bracketed by two hipEvents recorded on the grid's stream;
  * waits for the second and returns the elapsed device time in *ms.  (No
  * reference counterpart: the reference has no timing, lbm.rs:1166-1172.) */
@@ -286,6 +289,8 @@ int lbm_batch_set_graph(lbm_batch *b, int enable);
 int lbm_batch_set_variant(lbm_batch *b, int variant);
 int lbm_batch_get_variant(const lbm_batch *b, int *variant);
 int lbm_batch_autotune(lbm_batch *b, uint32_t steps, int *best, float *ms);
+/* as lbm_launches; a single step of a batch is two kernels, counted as one */
+int lbm_batch_launches(const lbm_batch *b, uint32_t n, uint32_t *launches);
 /* as lbm_autotune_cached; the shape class is the domain count and the total
  * cells in MiB-cells, each rounded up to a power of two */
 int lbm_batch_autotune_cached(lbm_batch *b, const char *cache_path, uint32_t steps, int *best, int *hit);

@@ -86,6 +86,7 @@ SIGNATURES = {
     "lbm_step_timed": (_i32, [_P, _u32, _fp]),
     "lbm_set_variant": (_i32, [_P, _i32]),
     "lbm_get_variant": (_i32, [_P, ctypes.POINTER(ctypes.c_int)]),
+    "lbm_launches": (_i32, [_P, _u32, ctypes.POINTER(_u32)]),
     "lbm_autotune": (_i32, [_P, _u32, ctypes.POINTER(ctypes.c_int), _fp]),
     "lbm_autotune_cached": (_i32, [_P, ctypes.c_char_p, _u32, ctypes.POINTER(ctypes.c_int),
                                    ctypes.POINTER(ctypes.c_int)]),
@@ -115,6 +116,7 @@ SIGNATURES = {
     "lbm_batch_set_graph": (_i32, [_P, _i32]),
     "lbm_batch_set_variant": (_i32, [_P, _i32]),
     "lbm_batch_get_variant": (_i32, [_P, ctypes.POINTER(ctypes.c_int)]),
+    "lbm_batch_launches": (_i32, [_P, _u32, ctypes.POINTER(_u32)]),
     "lbm_batch_autotune": (_i32, [_P, _u32, ctypes.POINTER(ctypes.c_int), _fp]),
     "lbm_batch_autotune_cached": (_i32, [_P, ctypes.c_char_p, _u32, ctypes.POINTER(ctypes.c_int),
                                          ctypes.POINTER(ctypes.c_int)]),

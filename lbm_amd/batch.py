@@ -106,6 +106,12 @@ class Batch:
     def variant(self, v: int):
         self._chk(self._lib.lbm_batch_set_variant(self._h, v))
 
+    def launches(self, n: int) -> int:
+        """Launches of the step kernel that step(n) would make now."""
+        v = ctypes.c_uint32()
+        self._chk(self._lib.lbm_batch_launches(self._h, n, ctypes.byref(v)))
+        return v.value
+
     def autotune(self, steps: int = 10):
         best = ctypes.c_int()
         ms = (ctypes.c_float * N.BATCH_NUM_VARIANTS)()

@@ -812,6 +812,13 @@ int lbm_batch_get_variant(const lbm_batch *b, int *variant) {
     return LBM_OK;
 }
 
+int lbm_batch_launches(const lbm_batch *b, uint32_t n, uint32_t *launches) {
+    if (!b || !launches) return LBM_EINVAL;
+    const TilePlan plan = b->plan_tile(n);
+    *launches = plan.launches ? plan.launches : n;
+    return LBM_OK;
+}
+
 int lbm_batch_autotune(lbm_batch *b, uint32_t steps, int *best, float *ms) {
     return bguard(b, [&] {
         bcheck(steps >= 2, "steps must be >= 2");

@@ -1031,6 +1031,13 @@ int lbm_get_variant(const lbm_grid *g, int *variant) {
     return LBM_OK;
 }
 
+int lbm_launches(const lbm_grid *g, uint32_t n, uint32_t *launches) {
+    if (!g || !launches) return LBM_EINVAL;
+    const TilePlan plan = g->plan_tile(n);
+    *launches = plan.launches ? plan.launches : n;
+    return LBM_OK;
+}
+
 int lbm_autotune(lbm_grid *g, uint32_t steps, int *best, float *ms) {
     return guarded(g, [&] {
         check(steps > 0, "steps must be > 0");

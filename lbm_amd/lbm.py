@@ -236,6 +236,12 @@ class LBM:
     def variant(self, v: int):
         self._chk(self._lib.lbm_set_variant(self._h, v))
 
+    def launches(self, n: int) -> int:
+        """Launches of the step kernel that step(n) would make now."""
+        v = ctypes.c_uint32()
+        self._chk(self._lib.lbm_launches(self._h, n, ctypes.byref(v)))
+        return v.value
+
     def autotune(self, steps: int = 20):
         """Time every step-kernel variant on this grid (state restored), keep the
         fastest; returns (best, ms_per_step list)."""

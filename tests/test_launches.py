@@ -1,0 +1,35 @@
+"""lbm_launches / lbm_batch_launches name the launches a call makes: one a step
+with the one-step kernels and for calls too short to share one, fewer (an even
+number for an even call once the stream is pending) with several steps a launch."""
+import ctypes
+
+import pytest
+
+
+def test_null_arguments():
+    from lbm_amd import _native as N
+    lib, n = N.load(), ctypes.c_uint32()
+    assert lib.lbm_launches(None, 5, ctypes.byref(n)) == N.LBM_EINVAL
+    assert lib.lbm_batch_launches(None, 5, ctypes.byref(n)) == N.LBM_EINVAL
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch", [False, True])
+def test_launches_of_a_call(batch):
+    from lbm_amd import LBM, Batch
+    print(f"case: launches, batch {batch}", flush=True)
+    o = Batch([(400, 160, 1.6, 0.05), (96, 64, 1.5, 0.04)]) if batch else LBM(1.6, 400, 160)
+    several = 6 if batch else 8
+    o.step(3)  # a stream is pending
+    for variant in (None, several, several + 1, 0, several - 1):
+        if variant is not None:
+            o.variant = variant
+        one = variant is not None and variant < several
+        assert [o.launches(n) for n in (0, 1, 2)] == [0, 1, 2]
+        for n in range(3, 70):
+            k = o.launches(n)
+            if one:
+                assert k == n
+            else:
+                assert 2 * k <= n <= 8 * k and (n % 2 or k % 2 == 0)
+    o.close()
