@@ -151,8 +151,8 @@ int lbm_sync(lbm_grid *g);
  * All variants compute the same bits.  The variants of several steps need two
  * more state sets: lbm_set_variant allocates them when it selects one (and
  * fails, changing nothing, when it cannot) and frees them when it selects
- * another.  A grid for which no variant was ever set or tuned (lbm_get_variant:
- * 0) runs several steps per launch too where two more sets take at most 512
+ * another.  A grid for which no variant was ever set, or tuned over three steps
+ * or more, runs several steps per launch by default where two more sets take at most 512
  * MiB; they are allocated with the grid, if there is memory for them and for
  * what the grid may still allocate, and given back where lbm_set_variant or
  * lbm_autotune would lack their memory.
@@ -160,7 +160,8 @@ int lbm_sync(lbm_grid *g);
  * own state, restores that state exactly, selects the fastest, and returns it
  * in *best and the per-step time of every variant in ms[LBM_NUM_VARIANTS]
  * (either pointer may be NULL; +inf for a variant of several steps whose sets
- * could not be allocated, or with steps < 3). */
+ * could not be allocated, or with steps < 3: a call that short picks the
+ * variant of single steps and leaves the default for longer calls as it was). */
 #define LBM_NUM_VARIANTS 10
 int lbm_set_variant(lbm_grid *g, int variant);
 int lbm_get_variant(const lbm_grid *g, int *variant);
@@ -282,10 +283,9 @@ int lbm_batch_set_graph(lbm_batch *b, int enable);
  * launch (one row a wave; two or three), which need two more state sets:
  * lbm_batch_set_variant allocates them (and fails, changing nothing, when it
  * cannot) and frees them when another variant is selected.  A batch for which
- * no variant was ever set or tuned (lbm_batch_get_variant: 0) runs several
- * steps per launch too where two more sets take at most 512 MiB.  All variants
- * give the same bits.  lbm_batch_autotune as lbm_autotune (+inf for a variant
- * of several steps without memory or with steps < 3). */
+ * no variant was ever set, or tuned over three steps or more, runs several
+ * steps per launch by default where two more sets take at most 512 MiB.  All variants
+ * give the same bits.  lbm_batch_autotune as lbm_autotune. */
 int lbm_batch_set_variant(lbm_batch *b, int variant);
 int lbm_batch_get_variant(const lbm_batch *b, int *variant);
 int lbm_batch_autotune(lbm_batch *b, uint32_t steps, int *best, float *ms);

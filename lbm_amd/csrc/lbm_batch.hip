@@ -842,7 +842,7 @@ int lbm_batch_autotune(lbm_batch *b, uint32_t steps, int *best, float *ms) {
             HIPCHK(hipEventCreate(&e1));
             for (int v = 0; v < LBM_BATCH_NUM_VARIANTS; ++v) {
                 if (lbm_batch::tile_variant(v)) {
-                    if (steps < 3) {  // too few steps a call for what these variants are for
+                    if (steps < kTileTunedFrom) {
                         t[v] = INFINITY;
                         continue;
                     }
@@ -887,7 +887,8 @@ int lbm_batch_autotune(lbm_batch *b, uint32_t steps, int *best, float *ms) {
         b->pform = pform;
         b->steps = nsteps;
         b->variant = v_best;
-        if (!lbm_batch::tile_variant(v_best)) b->release_spare();  // tried, not kept
+        if (steps < kTileTunedFrom && auto_path) b->auto_path = true;  // the default was not compared
+        else if (!lbm_batch::tile_variant(v_best)) b->release_spare();  // tried, not kept
         if (best) *best = v_best;
         if (ms)
             for (int v = 0; v < LBM_BATCH_NUM_VARIANTS; ++v) ms[v] = t[v] / steps;

@@ -1063,8 +1063,7 @@ int lbm_autotune(lbm_grid *g, uint32_t steps, int *best, float *ms) {
             HIPCHK(hipEventCreate(&e0));
             HIPCHK(hipEventCreate(&e1));
             for (int v = 0; v < LBM_NUM_VARIANTS; ++v) {
-                if (g->tile_variant(v) && steps < 3) {
-                    // too few steps a call for what these variants are for
+                if (g->tile_variant(v) && steps < kTileTunedFrom) {
                     t[v] = INFINITY;
                     continue;
                 }
@@ -1121,7 +1120,8 @@ int lbm_autotune(lbm_grid *g, uint32_t steps, int *best, float *ms) {
         g->pform = pform;
         g->steps = nsteps;
         g->variant = v_best;
-        if (!g->tile_variant(v_best)) g->release_spare();  // tried, not kept
+        if (steps < kTileTunedFrom && auto_path) g->auto_path = true;  // the default was not compared
+        else if (!g->tile_variant(v_best)) g->release_spare();  // tried, not kept
         if (best) *best = v_best;
         if (ms)
             for (int v = 0; v < LBM_NUM_VARIANTS; ++v) ms[v] = t[v] / steps;

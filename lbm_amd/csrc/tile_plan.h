@@ -16,6 +16,9 @@ constexpr int kTileMaxSteps = 8;
 // steps an autotuner times a tile variant for at least: launches of a few steps
 // (two of three in a call of six) say little about those of a long call
 constexpr uint32_t kTileTimedSteps = 48;
+// A tuning call of fewer steps does not time the tile variants (it asks for the
+// fastest single step); then neither do its results turn the default path off.
+constexpr uint32_t kTileTunedFrom = 3;
 
 // Block shapes of k_tile: rows a wave, waves, where the unstreamed cells' previous
 // populations live, and the launch's cost.  Without `chain` every cell has a

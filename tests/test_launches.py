@@ -33,3 +33,27 @@ def test_launches_of_a_call(batch):
             else:
                 assert 2 * k <= n <= 8 * k and (n % 2 or k % 2 == 0)
     o.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch", [False, True])
+def test_a_short_tuning_call_keeps_the_default(batch):
+    """Two steps cannot compare the several-step kernels: they pick the variant
+    of single steps and no more.  Three and above decide for every call; a
+    variant that was set is replaced as before."""
+    from lbm_amd import LBM, Batch
+    print(f"case: short tuning call, batch {batch}", flush=True)
+    o = Batch([(400, 160, 1.6, 0.05), (96, 64, 1.5, 0.04)]) if batch else LBM(1.6, 400, 160)
+    several = 6 if batch else 8
+    o.step(3)
+    untuned = [o.launches(n) for n in range(70)]
+    assert untuned[60] < 60
+    best, _ = o.autotune(2)
+    assert best < several and o.variant == best
+    assert [o.launches(n) for n in range(70)] == untuned
+    best, _ = o.autotune(3)
+    assert o.variant == best and (o.launches(60) == 60) == (best < several)
+    o.variant = several
+    best, _ = o.autotune(2)
+    assert best < several and o.launches(60) == 60
+    o.close()
