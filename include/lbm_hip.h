@@ -168,12 +168,14 @@ int lbm_get_variant(const lbm_grid *g, int *variant);
 int lbm_autotune(lbm_grid *g, uint32_t steps, int *best, float *ms);
 /* lbm_autotune through a JSON file (no reference counterpart): the file maps
  * (device architecture and CU count, shape class = the grid's width and height
- * rounded up to powers of two, precision, boundary, number of variants) to the
- * variant that was fastest.  A key found in the file selects its variant
- * without timing (*hit = 1); otherwise the call tunes as lbm_autotune and
+ * rounded up to powers of two, precision, boundary, number and generation of the
+ * variants) to the variant that was fastest.  A key found in the file selects its
+ * variant without timing (*hit = 1); otherwise the call tunes as lbm_autotune and
  * adds the key (*hit = 0), rewriting the file through a temporary file and a
- * rename.  A cached variant that cannot get its spare sets counts as a miss.  LBM_EINVAL when the file cannot be written (the tuned variant is
- * selected all the same).  best and hit may be NULL. */
+ * rename.  A cached variant that cannot get its spare sets counts as a miss, and
+ * so does the choice of a call of fewer than three steps for one of more.
+ * LBM_EINVAL when the file cannot be written (the tuned variant is selected all
+ * the same).  best and hit may be NULL. */
 int lbm_autotune_cached(lbm_grid *g, const char *cache_path, uint32_t steps, int *best, int *hit);
 /* The launches of the step kernel that lbm_step(g, n) would make now: n with one
  * step per launch, fewer where several steps share one. */
@@ -284,8 +286,8 @@ int lbm_batch_set_graph(lbm_batch *b, int enable);
  * lbm_batch_set_variant allocates them (and fails, changing nothing, when it
  * cannot) and frees them when another variant is selected.  A batch for which
  * no variant was ever set, or tuned over three steps or more, runs several
- * steps per launch by default where two more sets take at most 512 MiB.  All variants
- * give the same bits.  lbm_batch_autotune as lbm_autotune. */
+ * steps per launch by default where two more sets take at most 512 MiB.  All
+ * variants give the same bits.  lbm_batch_autotune as lbm_autotune. */
 int lbm_batch_set_variant(lbm_batch *b, int variant);
 int lbm_batch_get_variant(const lbm_batch *b, int *variant);
 int lbm_batch_autotune(lbm_batch *b, uint32_t steps, int *best, float *ms);

@@ -440,6 +440,16 @@ struct lbm_batch {
         HIPCHK(hipStreamSynchronize(stream));
     }
 
+    // `keep_default`: a one-step variant leaves the default path for longer calls
+    void select(int v, bool keep_default) {
+        HIPCHK(hipStreamSynchronize(stream));
+        keep_default = keep_default && auto_path && !tile_variant(v);
+        if (tile_variant(v)) ensure_spare(false);  // may fail: then nothing changes
+        else if (!keep_default) release_spare();
+        variant = v;
+        auto_path = keep_default;
+    }
+
     template <class St, int MODE, int SHAPE>
     void launch_tile(int steps, bool final) {
         using T = typename St::T;
@@ -798,11 +808,7 @@ int lbm_batch_set_graph(lbm_batch *b, int enable) {
 int lbm_batch_set_variant(lbm_batch *b, int variant) {
     return bguard(b, [&] {
         bcheck(variant >= 0 && variant < LBM_BATCH_NUM_VARIANTS, "unknown variant");
-        HIPCHK(hipStreamSynchronize(b->stream));
-        if (lbm_batch::tile_variant(variant)) b->ensure_spare(false);  // may fail: then nothing changes
-        else b->release_spare();
-        b->variant = variant;
-        b->auto_path = false;
+        b->select(variant, false);
     });
 }
 
@@ -902,24 +908,17 @@ int lbm_batch_autotune_cached(lbm_batch *b, const char *cache_path, uint32_t ste
     int rc = bguard(b, [&] {
         bcheck(cache_path && *cache_path, "null or empty cache path");
         bcheck(steps >= 2, "steps must be >= 2");
-        uint64_t cells = 0;
-        for (const DomainDev &d : b->table) cells += (uint64_t)d.g.X * d.g.Y;
-        const uint32_t mcells = (uint32_t)std::min<uint64_t>((cells + (1u << 20) - 1) >> 20, 1u << 30);
-        key = tune_cache::clean_key(device_tag(b->dev) + "/batch/" +
-                                    std::to_string(tune_cache::pow2_ceil((uint32_t)b->table.size())) + "d/" +
-                                    std::to_string(tune_cache::pow2_ceil(mcells)) + "Mcells/" +
-                                    precision_tag(b->precision) +
-                                    (b->boundary == LBM_BOUNDARY_REFERENCE ? "/ref" : "/zg") + "/v" +
-                                    std::to_string(LBM_BATCH_NUM_VARIANTS));
-        found = tune_cache::lookup(cache_path, key, e) && e.variant >= 0 && e.variant < LBM_BATCH_NUM_VARIANTS;
+        key = tune_cache::batch_key(device_tag(b->dev), (uint32_t)b->table.size(), b->cells, precision_tag(b->precision),
+                                    b->boundary == LBM_BOUNDARY_REFERENCE, LBM_BATCH_NUM_VARIANTS);
+        found = tune_cache::lookup(cache_path, key, e) &&
+                tune_cache::answers(e, steps, kTileTunedFrom, LBM_BATCH_NUM_VARIANTS);
     });
     if (rc != LBM_OK) return rc;
     if (hit) *hit = 0;
     // a cached variant whose spare sets cannot be allocated here is a miss
-    if (found && lbm_batch_set_variant(b, e.variant) == LBM_OK) {
+    if (found && bguard(b, [&] { b->select(e.variant, e.steps < kTileTunedFrom); }) == LBM_OK) {
         if (hit) *hit = 1;
         if (best) *best = e.variant;
-        b->err.clear();
         return LBM_OK;
     }
     e.ms.assign(LBM_BATCH_NUM_VARIANTS, 0.0f);

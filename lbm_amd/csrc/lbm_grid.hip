@@ -457,6 +457,16 @@ struct lbm_grid {
     // of moments, staging, colours and marks.
     size_t later_bytes() const { return 2 * alloc_bytes() + 20 * (size_t)geom.pstride * sizeof(float); }
 
+    // `keep_default`: a one-step variant leaves the default path for longer calls
+    void select(int v, bool keep_default) {
+        HIPCHK(hipStreamSynchronize(stream));
+        keep_default = keep_default && auto_path && !tile_variant(v);
+        if (tile_variant(v)) ensure_spare(false);  // may fail: then nothing changes
+        else if (!keep_default) release_spare();
+        variant = v;
+        auto_path = keep_default;
+    }
+
     template <class St, int MODE, int SHAPE>
     void launch_tile(int steps, bool final) {
         using T = typename St::T;
@@ -1017,11 +1027,7 @@ int lbm_step_timed(lbm_grid *g, uint32_t n, float *ms) {
 int lbm_set_variant(lbm_grid *g, int variant) {
     return guarded(g, [&] {
         check(variant >= 0 && variant < LBM_NUM_VARIANTS, "unknown kernel variant");
-        HIPCHK(hipStreamSynchronize(g->stream));
-        if (g->tile_variant(variant)) g->ensure_spare(false);  // may fail: then nothing changes
-        else g->release_spare();
-        g->variant = variant;
-        g->auto_path = false;
+        g->select(variant, false);
     });
 }
 
@@ -1135,20 +1141,17 @@ int lbm_autotune_cached(lbm_grid *g, const char *cache_path, uint32_t steps, int
     int rc = guarded(g, [&] {
         check(cache_path && *cache_path, "null or empty cache path");
         check(steps > 0, "steps must be > 0");
-        key = tune_cache::clean_key(device_tag(g->dev) + "/grid/" + std::to_string(tune_cache::pow2_ceil(g->X)) +
-                                    "x" + std::to_string(tune_cache::pow2_ceil(g->Y)) + "/" +
-                                    precision_tag(g->precision) +
-                                    (g->boundary == LBM_BOUNDARY_REFERENCE ? "/ref" : "/zg") + "/v" +
-                                    std::to_string(LBM_NUM_VARIANTS));
-        found = tune_cache::lookup(cache_path, key, e) && e.variant >= 0 && e.variant < LBM_NUM_VARIANTS;
+        key = tune_cache::grid_key(device_tag(g->dev), g->X, g->Y, precision_tag(g->precision),
+                                   g->boundary == LBM_BOUNDARY_REFERENCE, LBM_NUM_VARIANTS);
+        found = tune_cache::lookup(cache_path, key, e) &&
+                tune_cache::answers(e, steps, kTileTunedFrom, LBM_NUM_VARIANTS);
     });
     if (rc != LBM_OK) return rc;
     if (hit) *hit = 0;
     // a cached variant whose spare sets cannot be allocated here is a miss
-    if (found && lbm_set_variant(g, e.variant) == LBM_OK) {
+    if (found && guarded(g, [&] { g->select(e.variant, e.steps < kTileTunedFrom); }) == LBM_OK) {
         if (hit) *hit = 1;
         if (best) *best = e.variant;
-        g->err.clear();
         return LBM_OK;
     }
     e.ms.assign(LBM_NUM_VARIANTS, 0.0f);

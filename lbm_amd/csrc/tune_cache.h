@@ -6,7 +6,7 @@
 //
 // The file is one JSON object, one entry per line, as store() writes it:
 //   {
-//   "gfx950:sramecc+:xnack-/256cu/grid/8192x4096/f32/ref/v10": {"variant": 8, "steps": 20, "ms": [0.93, ...]},
+//   "gfx950:sramecc+:xnack-/256cu/grid/8192x4096/f32/ref/v10/g2": {"variant": 8, "steps": 20, "ms": [0.93, ...]},
 //   ...
 //   }
 // "ms" holds the per-step time of every candidate (null for one that could not
@@ -50,6 +50,36 @@ inline std::string clean_key(const std::string &s) {
         if (!ok || c == '\0') c = '_';
     }
     return k;
+}
+
+// What the variants' numbers stand for: raised whenever one of them names another
+// kernel or the path of an untuned object changes, so that choices made among
+// other kernels are made again (2: variants 8 and 9 of a grid, 6 and 7 of a batch
+// became the register tiles, the default of small objects).
+constexpr int kGeneration = 2;
+
+inline std::string versioned(const std::string &s, const char *precision, bool reference, int variants) {
+    return clean_key(s + precision + (reference ? "/ref" : "/zg") + "/v" + std::to_string(variants) + "/g" +
+                     std::to_string(kGeneration));
+}
+inline std::string grid_key(const std::string &device, uint32_t X, uint32_t Y, const char *precision, bool reference,
+                            int variants) {
+    return versioned(device + "/grid/" + std::to_string(pow2_ceil(X)) + "x" + std::to_string(pow2_ceil(Y)) + "/",
+                     precision, reference, variants);
+}
+inline std::string batch_key(const std::string &device, uint32_t domains, uint64_t cells, const char *precision,
+                             bool reference, int variants) {
+    const uint64_t m = (cells + (1u << 20) - 1) >> 20;
+    return versioned(device + "/batch/" + std::to_string(pow2_ceil(domains)) + "d/" +
+                         std::to_string(pow2_ceil((uint32_t)(m < (1u << 30) ? m : 1u << 30))) + "Mcells/",
+                     precision, reference, variants);
+}
+
+// May a call that tunes over `steps` steps take the entry's choice?  An entry of
+// a call too short to time every variant (fewer than `all_from` steps) answers
+// only calls as short.
+inline bool answers(const Entry &e, uint32_t steps, uint32_t all_from, int variants) {
+    return e.variant >= 0 && e.variant < variants && (e.steps >= all_from || steps < all_from);
 }
 
 inline const char *skip_ws(const char *p) {
