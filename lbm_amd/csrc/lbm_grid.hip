@@ -323,8 +323,10 @@ struct lbm_grid {
         staging.release();
         for (void *p : {f[0], f[1], spare[0], spare[1], (void *)mask, (void *)flags, (void *)lag,
                         (void *)now, (void *)out, (void *)dense, (void *)partials, (void *)sums,
-                        (void *)snap, (void *)umark, (void *)vpart})
+                        (void *)rgb, (void *)snap, (void *)umark, (void *)vpart})
             if (p) (void)hipFree(p);
+        rgb = nullptr;
+        rgb_elems = 0;
         snap = nullptr;
         umark = nullptr;
         vpart = nullptr;
