@@ -404,7 +404,8 @@ int lbm_velocity_skill(lbm_grid *g, double out[2]);
  * chunks (block shape (1,1,1) only, input channels a multiple of 64).  Bit 12
  * with mode 0: a bf16 output and its
  * 2 x 2 average pool, returned as out[0, N H W Cout) and out[N H W Cout,
- * + N H W Cout / 4) (H even). */
+ * + N H W Cout / 4) (H even).  Bit 14 with mode 1: the input gradient in bf16,
+ * zero where the N H W Cin activations `g` are not positive. */
 int lbm_conv3x3_test(int mode, int n, int h, int w, int cin, int cout, const float *in, const float *g,
                      const float *weights, const float *bias, float *out, int device);
 

@@ -2131,7 +2131,8 @@ int lbm_unet_time_forward(lbm_unet *n, int reps, float *ms) {
 // Test entry point for the convolution primitives on host arrays (f32 in,
 // rounded to bf16 on the device).  mode 0: out = conv(in, w) + bias (no ReLU;
 // with bit 12 also its pooled bf16 output); mode 1: out = input gradient for
-// output gradient `in`; mode 2: out = weight gradient dw[tap][co][ci] for input
+// output gradient `in` (with bit 14 in bf16 through the ReLU of the activation
+// `g`); mode 2: out = weight gradient dw[tap][co][ci] for input
 // `in` and output gradient `g`; mode 3: timing.  Bits 4..11 force the block
 // shape, split and kernel.
 int lbm_conv3x3_test(int mode, int N, int H, int W, int Cin, int Cout, const float *in, const float *g,
@@ -2143,7 +2144,9 @@ int lbm_conv3x3_test(int mode, int N, int H, int W, int Cin, int Cout, const flo
         force.split = (mode >> 8) & 7;
         force.kind = (mode >> 13) & 1 ? 2 : (mode >> 11) & 1 ? 1 : -1;
         const bool pooled = (mode >> 12) & 1;
-        ucheck(force.tile <= 13 && (mode >> 14) == 0, "mode");
+        const bool gated = (mode >> 14) & 1;
+        ucheck(force.tile <= 13 && (mode >> 15) == 0, "mode");
+        ucheck(!gated || ((mode & 3) == 1 && g), "mode: a gate needs the input gradient and an activation");
         ucheck(!pooled || ((mode & 3) == 0 && H % 2 == 0), "mode: pooled output needs the forward and an even height");
         ucheck(force.split == 0 || force.split == 1 || force.split == 2 || force.split == 4, "mode: split");
         mode = op;
@@ -2160,7 +2163,7 @@ int lbm_conv3x3_test(int mode, int N, int H, int W, int Cin, int Cout, const flo
             return p;
         };
         try {
-            float *d32 = (float *)alloc(std::max({P * cin_in, P * Cout, nw}) * sizeof(float));
+            float *d32 = (float *)alloc(std::max({P * cin_in, P * Cout, P * cout_out, nw}) * sizeof(float));
             uint16_t *din = (uint16_t *)alloc(P * cin_in * 2);
             uint16_t *dw = (uint16_t *)alloc(nw * 2);
             HIPCHK(hipMemcpy(d32, in, P * cin_in * sizeof(float), hipMemcpyHostToDevice));
@@ -2212,8 +2215,17 @@ int lbm_conv3x3_test(int mode, int N, int H, int W, int Cin, int Cout, const flo
             } else if (mode == 1) {
                 uint16_t *dwt = (uint16_t *)alloc(nw * 2);
                 hipLaunchKernelGGL(k_flip_transpose, dim3(nblk(nw)), dim3(256), 0, 0, dw, dwt, Cin, Cout, 9);
-                conv_fwd(0, 3, one_input(din, Cout), dwt, nullptr, dout, N, H, W, Cin, false, true, Cin, ws, wsn,
-                         force);
+                if (gated) {  // bf16 through the activation's ReLU, returned as f32
+                    uint16_t *act = (uint16_t *)alloc(P * Cin * 2), *o16 = (uint16_t *)alloc(P * Cin * 2);
+                    HIPCHK(hipMemcpy(d32, g, P * Cin * sizeof(float), hipMemcpyHostToDevice));
+                    hipLaunchKernelGGL(k_f32_to_bf16, dim3(nblk(P * Cin)), dim3(256), 0, 0, d32, act, P * Cin);
+                    conv_fwd(0, 3, one_input(din, Cout), dwt, nullptr, o16, N, H, W, Cin, false, false, Cin, ws, wsn,
+                             force, nullptr, ConvHead{}, act);
+                    hipLaunchKernelGGL(k_bf16_to_f32, dim3(nblk(P * Cin)), dim3(256), 0, 0, o16, dout, P * Cin);
+                } else {
+                    conv_fwd(0, 3, one_input(din, Cout), dwt, nullptr, dout, N, H, W, Cin, false, true, Cin, ws, wsn,
+                             force);
+                }
                 HIPCHK(hipMemcpy(out, dout, P * Cin * sizeof(float), hipMemcpyDeviceToHost));
             } else {
                 uint16_t *dg = (uint16_t *)alloc(P * Cout * 2);
