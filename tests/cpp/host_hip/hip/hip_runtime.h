@@ -1,6 +1,6 @@
 // The few runtime calls of lbm_amd/csrc/staging.h on the host, for
-// staging_check.cpp: a stream is a queue whose copies run only when something
-// waits for them, as late as the real runtime may run them, so that a chunk
+// staging_check.cpp: a stream is a queue whose copies and kernels (every thread of
+// every block in turn) run only when something waits for them, as late as the real runtime may run them, so that a chunk
 // refilled or read without a wait gives wrong bytes.
 #pragma once
 
@@ -39,9 +39,9 @@ typedef FakeEvent *hipEvent_t;
 struct FakeHip {
     std::recursive_mutex lock;
     std::map<const char *, size_t> pinned;  // host allocations
-    hipError_t last = hipSuccess;
-    int host_mallocs = 0, copies = 0, fail_copy = -1, device = -1;
+    int host_mallocs = 0, copies = 0, launches = 0, fail_launch = -1, device = -1;
 };
+inline thread_local hipError_t fake_last = hipSuccess;
 inline FakeHip &fake() {
     static FakeHip f;
     return f;
@@ -49,13 +49,12 @@ inline FakeHip &fake() {
 #define FAKE_LOCK std::lock_guard<std::recursive_mutex> guard_(fake().lock)
 
 inline hipError_t fake_error(hipError_t e) {
-    if (e != hipSuccess) fake().last = e;
+    if (e != hipSuccess) fake_last = e;
     return e;
 }
 inline hipError_t hipGetLastError() {
-    FAKE_LOCK;
-    const hipError_t e = fake().last;
-    fake().last = hipSuccess;
+    const hipError_t e = fake_last;
+    fake_last = hipSuccess;
     return e;
 }
 inline hipError_t hipSetDevice(int dev) {
@@ -110,7 +109,27 @@ inline hipError_t hipStreamSynchronize(hipStream_t s) {
 }
 inline hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind, hipStream_t s) {
     FAKE_LOCK;
-    if (fake().copies++ == fake().fail_copy) return fake_error(hipErrorUnknown);
+    ++fake().copies;
     s->ops.push_back([=] { std::memcpy(dst, src, n); });
     return hipSuccess;
 }
+
+#define __global__
+struct dim3 {
+    unsigned x, y, z;
+    dim3(unsigned x_ = 1, unsigned y_ = 1, unsigned z_ = 1) : x(x_), y(y_), z(z_) {}
+};
+inline thread_local dim3 blockIdx, threadIdx;
+template <class... P, class... A>
+void fake_launch(void (*kernel)(P...), dim3 grid, dim3 block, size_t, hipStream_t s, A... args) {
+    FAKE_LOCK;
+    if (fake().launches++ == fake().fail_launch) {
+        fake_error(hipErrorUnknown);
+        return;
+    }
+    s->ops.push_back([=] {
+        for (blockIdx.x = 0; blockIdx.x < grid.x; ++blockIdx.x)
+            for (threadIdx.x = 0; threadIdx.x < block.x; ++threadIdx.x) kernel(args...);
+    });
+}
+#define hipLaunchKernelGGL fake_launch

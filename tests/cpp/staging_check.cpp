@@ -1,10 +1,11 @@
 // Drives lbm_amd/csrc/staging.h over a host stand-in of the runtime
 // (host_hip/hip/hip_runtime.h) for tests/test_staging.py:
 //   staging_check copy out|in BYTES [BYTES ...]   the pieces of one call, twice
+//   staging_check odd out|in BYTES                device memory at an odd address
 //   staging_check pinned out|in BYTES             pinned caller memory
 //   staging_check nothread out|in BYTES N         the N-th thread cannot be made
-//   staging_check error out|in BYTES N            the N-th chunk's copy fails
-// Prints "ok" and what was counted; any wrong byte ends it with status 1.
+//   staging_check error out|in BYTES N            the N-th chunk's launch fails
+// Prints "ok", whether chunks were made, and the runtime's copies and the launches; any wrong byte ends it with status 1.
 #include <cstdio>
 #include <cstdlib>
 #include <new>
@@ -32,29 +33,29 @@ static char byte_at(size_t b, unsigned seed) {
 }
 
 static bool fill_and_compare(Staging &st, bool out, const std::vector<size_t> &sizes, bool pinned, unsigned seed,
-                             hipError_t expect) {
+                             hipError_t expect, size_t shift = 0) {
     constexpr size_t kGuard = 64;
     std::vector<std::vector<char>> dev(sizes.size()), ref(sizes.size());
     std::vector<char *> host(sizes.size());
     std::vector<Piece> pieces;
     for (size_t i = 0; i < sizes.size(); ++i) {
-        const size_t n = sizes[i] + 2 * kGuard;
+        const size_t n = sizes[i] + 2 * kGuard + shift;
         if (pinned) (void)hipHostMalloc((void **)&host[i], n, hipHostMallocDefault);
         else host[i] = (char *)std::malloc(n);
-        dev[i].assign(n, 'd');
+        dev[i].assign(n, 'd');  // (device memory from dev + shift on)
         std::memset(host[i], 'h', n);
         ref[i].resize(sizes[i]);
         for (size_t b = 0; b < sizes[i]; ++b) ref[i][b] = byte_at(b, 97 * seed + (unsigned)i);
-        char *const from = out ? dev[i].data() : host[i];
+        char *const from = out ? dev[i].data() + shift : host[i];
         std::memcpy(from + kGuard, ref[i].data(), sizes[i]);
-        pieces.push_back({host[i] + kGuard, dev[i].data() + kGuard, sizes[i]});
+        pieces.push_back({host[i] + kGuard, dev[i].data() + shift + kGuard, sizes[i]});
     }
     const hipError_t e = st.copy(3, &s, pieces.data(), (int)pieces.size(), out);
     if (e == hipSuccess && !out) (void)hipStreamSynchronize(&s);
     bool ok = e == expect;
     if (e == hipSuccess)
         for (size_t i = 0; i < sizes.size(); ++i) {
-            const char *to = out ? host[i] : dev[i].data();
+            const char *to = out ? host[i] : dev[i].data() + shift;
             const char mark = out ? 'h' : 'd';
             ok = ok && std::memcmp(to + kGuard, ref[i].data(), sizes[i]) == 0;
             for (size_t b = 0; b < kGuard; ++b) ok = ok && to[b] == mark && to[kGuard + sizes[i] + b] == mark;
@@ -77,6 +78,8 @@ int main(int argc, char **argv) {
         for (int i = 4; i < argc; ++i) sizes.push_back(std::strtoull(argv[i], nullptr, 10));
         for (unsigned seed = 1; seed <= 2; ++seed)  // the second call meets the first one's chunks
             ok = ok && fill_and_compare(st, out, sizes, false, seed, hipSuccess);
+    } else if (cmd == "odd") {
+        ok = fill_and_compare(st, out, sizes, false, 1, hipSuccess, 1);
     } else if (cmd == "pinned") {
         ok = fill_and_compare(st, out, sizes, true, 1, hipSuccess);
         --fake().host_mallocs;  // the caller's own
@@ -96,15 +99,16 @@ int main(int argc, char **argv) {
         (void)hipStreamSynchronize(&s);
         ok = ok && e == hipSuccess && to == want;
     } else if (cmd == "error" && argc == 5) {
-        fake().fail_copy = std::atoi(argv[4]);
+        fake().fail_launch = std::atoi(argv[4]);
         ok = fill_and_compare(st, out, sizes, false, 1, hipErrorUnknown);
-        fake().fail_copy = -1;
+        fake().fail_launch = -1;
         ok = ok && fill_and_compare(st, out, sizes, false, 2, hipSuccess);  // and the next call is whole
     } else {
         return 2;
     }
     const bool clean = hipGetLastError() == hipSuccess || cmd == "error";
     st.release();
-    std::printf("%s host_mallocs=%d\n", ok ? (clean ? "ok" : "an error is left behind") : "wrong", fake().host_mallocs);
+    std::printf("%s chunks=%d copies=%d launches=%d\n", ok ? (clean ? "ok" : "an error is left behind") : "wrong",
+                fake().host_mallocs, fake().copies, fake().launches);
     return ok && clean ? 0 : 1;
 }
