@@ -203,7 +203,8 @@ struct lbm_batch {
         drop_graphs();
         staging.release();
         release_spare();
-        for (void *p : {f[0], f[1], (void *)starts, (void *)mask, (void *)flags, (void *)segs, (void *)lag, (void *)dense,
+        free_sets(f);
+        for (void *p : {(void *)starts, (void *)mask, (void *)flags, (void *)segs, (void *)lag, (void *)dense,
                         (void *)dtable, (void *)ilist, (void *)blist, (void *)alist})
             if (p) (void)hipFree(p);
         if (stream) (void)hipStreamDestroy(stream);
@@ -364,25 +365,16 @@ struct lbm_batch {
     static constexpr size_t kAutoSpareBytes = (size_t)512 << 20;
 
     void make_spare(void *out[2]) {
-        out[0] = out[1] = nullptr;
+        alloc_sets(out, alloc_bytes());
         try {
-            for (int i = 0; i < 2; ++i) {
-                out[i] = dalloc<char>(alloc_bytes());
-                // the rows' padding is never written by k_batch_tile: keep it defined
-                HIPCHK(hipMemsetAsync(out[i], 0, set_bytes(), stream));
-            }
+            // the rows' padding is never written by k_batch_tile: keep it defined
+            HIPCHK(hipMemsetAsync(out[0], 0, set_stride(alloc_bytes()) + set_bytes(), stream));
         } catch (...) {
-            for (int i = 0; i < 2; ++i)
-                if (out[i]) (void)hipFree(out[i]);
+            free_sets(out);
             throw;
         }
     }
-    void release_spare() {
-        for (void *&p : spare) {
-            if (p) (void)hipFree(p);
-            p = nullptr;
-        }
-    }
+    void release_spare() { free_sets(spare); }
     // a tile variant's sets, the default path's pair and what may still be
     // allocated: as a single grid's (lbm_grid.hip)
     void ensure_spare(bool take_over = true) {
@@ -667,8 +659,7 @@ int lbm_batch_create(const lbm_domain *doms, uint32_t n, int32_t precision, int3
     b->seg_bytes = so;
     int rc = bguard(b, [&] {
         HIPCHK(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
-        b->f[0] = dalloc<char>(b->alloc_bytes());
-        b->f[1] = dalloc<char>(b->alloc_bytes());
+        alloc_sets(b->f, b->alloc_bytes());
         b->mask = dalloc<uint8_t>(b->aux_elems);
         b->flags = dalloc<uint8_t>(b->aux_elems);
         b->segs = dalloc<uint8_t>(b->seg_bytes);
@@ -724,14 +715,13 @@ int lbm_batch_reset(lbm_batch *b) {
             host_feq(b->doms[i].u_in, 0.0f, 1.0f, v);
             const float4 a = make_float4(v[0], v[1], v[2], v[3]);
             const float4 c = make_float4(v[4], v[5], v[6], v[7]);
-            const dim3 grid((unsigned)(((size_t)d.g.ys * d.g.Y + 255) / 256));
-            for (int s = 0; s < 2; ++s) {
-                by_store(b->precision, [&]<class St>() {
-                    hipLaunchKernelGGL(k_fill<St>, grid, dim3(256), 0, b->stream, (typename St::T *)b->fptr(s, d), d.g,
-                                       a, c, v[8]);
-                });
-                HIPCHK(hipGetLastError());
-            }
+            const dim3 grid((unsigned)(((size_t)d.g.ys * d.g.Y + 255) / 256), 2);
+            by_store(b->precision, [&]<class St>() {
+                using T = typename St::T;
+                hipLaunchKernelGGL(k_fill<St>, grid, dim3(256), 0, b->stream, (T *)b->fptr(0, d), (T *)b->fptr(1, d),
+                                   d.g, a, c, v[8]);
+            });
+            HIPCHK(hipGetLastError());
         }
         b->cur = 0;
         b->pform = false;

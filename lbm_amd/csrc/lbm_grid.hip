@@ -321,8 +321,10 @@ struct lbm_grid {
     void release() {
         (void)hipSetDevice(dev);
         staging.release();
-        for (void *p : {f[0], f[1], spare[0], spare[1], (void *)mask, (void *)flags, (void *)lag,
-                        (void *)now, (void *)out, (void *)dense, (void *)partials, (void *)sums,
+        free_sets(f);
+        free_sets(spare);
+        for (void *p : {(void *)mask, (void *)flags, (void *)lag, (void *)now,
+                        (void *)out, (void *)dense, (void *)partials, (void *)sums,
                         (void *)rgb, (void *)snap, (void *)umark, (void *)vpart})
             if (p) (void)hipFree(p);
         rgb = nullptr;
@@ -330,8 +332,6 @@ struct lbm_grid {
         snap = nullptr;
         umark = nullptr;
         vpart = nullptr;
-        f[0] = f[1] = nullptr;
-        spare[0] = spare[1] = nullptr;
         mask = flags = nullptr;
         lag = now = out = dense = nullptr;
         partials = sums = nullptr;
@@ -403,25 +403,16 @@ struct lbm_grid {
     // two more sets (not in place of the default path's: those stay until the
     // new ones are there)
     void make_spare(void *out[2]) {
-        out[0] = out[1] = nullptr;
+        alloc_sets(out, alloc_bytes());
         try {
-            for (int i = 0; i < 2; ++i) {
-                out[i] = dalloc<char>(alloc_bytes());
-                // the rows' padding is never written by k_tile: keep it defined
-                HIPCHK(hipMemsetAsync(out[i], 0, set_bytes(), stream));
-            }
+            // the rows' padding is never written by k_tile: keep it defined
+            HIPCHK(hipMemsetAsync(out[0], 0, set_stride(alloc_bytes()) + set_bytes(), stream));
         } catch (...) {
-            for (int i = 0; i < 2; ++i)
-                if (out[i]) (void)hipFree(out[i]);
+            free_sets(out);
             throw;
         }
     }
-    void release_spare() {
-        for (void *&p : spare) {
-            if (p) (void)hipFree(p);
-            p = nullptr;
-        }
-    }
+    void release_spare() { free_sets(spare); }
     // k_tile's sets for a tile variant; the state itself is always in f[0], f[1]
     // between calls.  Setting a variant does not take over the default path's
     // pair, as it fails where two more sets cannot be allocated; the pair's own
@@ -527,13 +518,12 @@ struct lbm_grid {
     void fill_both(const float v[9]) {
         const float4 a = make_float4(v[0], v[1], v[2], v[3]);
         const float4 b = make_float4(v[4], v[5], v[6], v[7]);
-        const dim3 grid((unsigned)(((size_t)geom.ys * Y + 255) / 256));
-        for (int s = 0; s < 2; ++s) {
-            by_store(precision, [&]<class St>() {
-                hipLaunchKernelGGL(k_fill<St>, grid, dim3(256), 0, stream, (typename St::T *)f[s], geom, a, b, v[8]);
-            });
-            HIPCHK(hipGetLastError());
-        }
+        const dim3 grid((unsigned)(((size_t)geom.ys * Y + 255) / 256), 2);
+        by_store(precision, [&]<class St>() {
+            using T = typename St::T;
+            hipLaunchKernelGGL(k_fill<St>, grid, dim3(256), 0, stream, (T *)f[0], (T *)f[1], geom, a, b, v[8]);
+        });
+        HIPCHK(hipGetLastError());
     }
 
     void ensure_now() {
@@ -793,8 +783,7 @@ int lbm_create(const lbm_config *cfg, lbm_grid **out) {
     g->geom = Geom{(int)cfg->nx, (int)cfg->ny, pitch, pstride, 9LL * pitch, (long long)pitch, cfg->omega};
     int rc = guarded(g, [&] {
         HIPCHK(hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking));
-        g->f[0] = dalloc<char>(g->alloc_bytes());
-        g->f[1] = dalloc<char>(g->alloc_bytes());
+        alloc_sets(g->f, g->alloc_bytes());
         g->mask = dalloc<uint8_t>(pstride);
         g->flags = dalloc<uint8_t>(pstride);
         g->lag = dalloc<float>(3 * (size_t)pstride);
