@@ -1757,9 +1757,13 @@ struct lbm_unet {
                 const long long Pl = (long long)B * h * w;
                 ws_elems = std::max({ws_elems, conv_split_elems(c.ks, Pl, B, h, w, c.cin, c.cout),
                                      conv_split_elems(c.ks, Pl, B, h, w, c.cout, c.cin)});
-                wgrad_ws_elems = std::max(wgrad_ws_elems, wgrad_elems(c.ks, B, h, w, c.cin, c.cout));
             }
         }
+        // (by each layer's own level: at the full resolution a 256-channel layer would ask for 38 MB)
+        constexpr int levels[18] = {0, 0, 1, 1, 2, 2, 3, 3, 3, 2, 2, 2, 1, 1, 1, 0, 0, 0};
+        for (size_t i = 0; i < convs.size(); ++i)
+            wgrad_ws_elems = std::max(wgrad_ws_elems, wgrad_elems(convs[i].ks, B, H >> levels[i], W >> levels[i],
+                                                                  convs[i].cin, convs[i].cout));
         if (ws_elems) ws = (float *)alloc(ws_elems * 4);
         wgrad_ws = (float *)alloc(wgrad_ws_elems * 4);
         // He-normal weights (fan-in = taps * real input channels), zero biases; the

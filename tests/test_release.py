@@ -35,3 +35,20 @@ def test_no_buffer_outlives_its_grid():
         use()
     # (a plane kept back would be 8 MB a grid, 100 MB in all)
     assert before - _free() < 16 << 20
+
+
+def test_network_memory():
+    """A network holds 36 MB of parameters, optimiser state and bf16 copies, its
+    tensors, and workspaces for its own layers (55 MB in all at 8 x 256), not 38 MB
+    more for a 256-channel layer at the full resolution, which it has none of."""
+    from lbm_amd.surrogate import UNet
+    print("case: network memory", flush=True)
+    first = UNet(1, 8, 256, seed=1)  # (modules and the runtime's own buffers)
+    nets, before = [], _free()
+    for _ in range(4):
+        nets.append(UNet(1, 8, 256, seed=1))
+    held = (before - _free()) / 4
+    print(f"held per network: {held / 2 ** 20:.1f} MB", flush=True)
+    for n in nets + [first]:
+        n.close()
+    assert held < 64 << 20
