@@ -255,7 +255,7 @@ struct lbm_batch {
             const DomainDev &d = table[i];
             const int srow = d.g.pitch / 64 + kSegSlack;
             hipLaunchKernelGGL(k_build_segments, dim3((srow + 255) / 256, d.g.Y), dim3(256), 0, stream,
-                               flags + d.aux_off, segs + d.seg_off, nullptr, nullptr, d.g);
+                               flags + d.aux_off, segs + d.seg_off, d.g);
             HIPCHK(hipGetLastError());
         }
         std::vector<uint8_t> hs(seg_bytes);

@@ -91,8 +91,7 @@ __global__ void k_build_flags(const uint8_t *__restrict__ mask, uint8_t *__restr
 // pitch / 64 + 8 entries; the extra ones stay 0.
 constexpr int kSegSlack = 8;
 
-__global__ void k_build_segments(const uint8_t *__restrict__ flags, uint8_t *__restrict__ segs,
-                                 uint32_t *__restrict__ list, uint32_t *__restrict__ count, Geom g) {
+__global__ void k_build_segments(const uint8_t *__restrict__ flags, uint8_t *__restrict__ segs, Geom g) {
     const int srow = g.pitch / 64 + kSegSlack;
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     const int y = blockIdx.y;
@@ -109,7 +108,6 @@ __global__ void k_build_segments(const uint8_t *__restrict__ flags, uint8_t *__r
         clear = acc == 0;
     }
     segs[(size_t)y * srow + s] = clear;
-    if (list && !clear && 64 * s < g.X) list[atomicAdd(count, 1u)] = (uint32_t)((size_t)y * srow + s);
 }
 
 // fn.template operator()<St>() with the storage format of `precision`

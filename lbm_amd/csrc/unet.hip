@@ -124,14 +124,13 @@ typedef uint16_t u16x16 __attribute__((ext_vector_type(16)));  // 32 B: one lane
 // eight and the second k-step their last eight (the same permutation of K for
 // A and B).  The next chunk's operands are loaded while the current one is
 // multiplied.  Requirements: P % (32 * MI) == 0, Cin % 32 == 0,
-// Cout % (32 * NI) == 0.  Only channels co < co_store, rounded up to a multiple
-// of four, are stored: the weights are the A operand, as in the 3x3 kernels, so
+// Cout % (32 * NI) == 0.  The weights are the A operand, as in the 3x3 kernels, so
 // that a lane holds runs of four channels of one pixel (with the pixels in A it
 // held one channel and stored two bytes at a time).
-template <int MI, int NI, bool RELU, bool OUT_F32>
+template <int MI, int NI, bool RELU>
 __global__ __launch_bounds__(256) void k_conv1x1(const uint16_t *__restrict__ in, const uint16_t *__restrict__ w,
-                                                 const float *__restrict__ bias, void *__restrict__ out, long long P,
-                                                 int Cin, int Cout, int co_store, const uint16_t *__restrict__ gate) {
+                                                 const float *__restrict__ bias, uint16_t *__restrict__ out,
+                                                 long long P, int Cin, int Cout, const uint16_t *__restrict__ gate) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int half = lane >> 5, l32 = lane & 31;
     const long long p0 = ((long long)blockIdx.x * 4 + wave) * (32 * MI);
@@ -177,40 +176,11 @@ __global__ __launch_bounds__(256) void k_conv1x1(const uint16_t *__restrict__ in
         if (kk + 2 < nk) load(kk + 2, A0, B0);
         mma(A1, B1);
     }
-    if (!OUT_F32 && co_store == Cout) {
 #pragma unroll
-        for (int i = 0; i < MI; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
-            for (int j = 0; j < NI; ++j)
-                store_bf16_tile(acc[i][j], bias, RELU, gate, (uint16_t *)out, p0 + 32 * i, Cout, co0 + 32 * j, half, l32);
-        return;
-    }
-    // lane l holds pixel l % 32 and channels 8 g + 4 (l / 32) .. + 3: four at a time
-#pragma unroll
-    for (int i = 0; i < MI; ++i) {
-        const long long p = p0 + 32 * i + l32;
-#pragma unroll
-        for (int j = 0; j < NI; ++j) {
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int co = co0 + 32 * j + 8 * g + 4 * half;
-                if (co >= co_store) continue;
-                const float4 bv = bias ? *(const float4 *)&bias[co] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                float v[4] = {acc[i][j][4 * g] + bv.x, acc[i][j][4 * g + 1] + bv.y, acc[i][j][4 * g + 2] + bv.z,
-                              acc[i][j][4 * g + 3] + bv.w};
-                if (RELU)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = fmaxf(v[e], 0.0f);
-                if (OUT_F32) {
-                    *(float4 *)&((float *)out)[p * Cout + co] = make_float4(v[0], v[1], v[2], v[3]);
-                } else {
-                    const uint32_t lo = f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16),
-                                   hi = f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
-                    *(uint2 *)&((uint16_t *)out)[p * Cout + co] = make_uint2(lo, hi);
-                }
-            }
-        }
-    }
+        for (int j = 0; j < NI; ++j)
+            store_bf16_tile(acc[i][j], bias, RELU, gate, out, p0 + 32 * i, Cout, co0 + 32 * j, half, l32);
 }
 
 // Epilogue of the 3x3 kernels.  The products are issued with the weights as
@@ -1418,25 +1388,25 @@ void conv_fwd(hipStream_t s, int ks, const ConvIn &in, const uint16_t *w, const 
     ucheck(!gate || (!out_f32 && !relu && co_store == Cout && ((uintptr_t)gate & 15) == 0),
            "gate: a whole bf16 gradient's activation");
     if (ks == 1) {
-        ucheck(!in.a_up && in.cb == 0 && !pool_out && !head.w, "1x1 convolutions take one plain input only");
+        ucheck(!in.a_up && in.cb == 0 && !pool_out && !head.w && !out_f32 && co_store == Cout,
+               "1x1 convolutions take one plain input and store whole bf16 outputs");
         ucheck(((uintptr_t)bias & 15) == 0 && ((uintptr_t)out & 15) == 0,
                "convolution buffers must be 16-byte aligned");
         int mi = 1, ni = 1;
         if (P % 64 == 0 && P / 64 * (Cout / 32) >= 4096) mi = 2;
         else if (Cout % 64 == 0 && P / 32 * (Cout / 64) >= 4096) ni = 2;
         const dim3 grid((unsigned)((P + 128 * mi - 1) / (128 * mi)), (unsigned)(Cout / (32 * ni)), 1);
-#define K1(MI, NI, R, F)                                                                                     \
-    hipLaunchKernelGGL((k_conv1x1<MI, NI, R, F>), grid, dim3(256), 0, s, in.a, w, bias, out, P, Cin, Cout, \
-                       co_store, gate)
-#define PICK(R, F)                       \
-    do {                                 \
-        if (mi == 2) K1(2, 1, R, F);     \
-        else if (ni == 2) K1(1, 2, R, F); \
-        else K1(1, 1, R, F);             \
+#define K1(MI, NI, R)                                                                                         \
+    hipLaunchKernelGGL((k_conv1x1<MI, NI, R>), grid, dim3(256), 0, s, in.a, w, bias, (uint16_t *)out, P, Cin, Cout, \
+                       gate)
+#define PICK(R)                       \
+    do {                              \
+        if (mi == 2) K1(2, 1, R);     \
+        else if (ni == 2) K1(1, 2, R); \
+        else K1(1, 1, R);             \
     } while (0)
-        if (out_f32) PICK(false, true);
-        else if (relu) PICK(true, false);
-        else PICK(false, false);
+        if (relu) PICK(true);
+        else PICK(false);
 #undef PICK
 #undef K1
         HIPCHK(hipGetLastError());
