@@ -282,15 +282,28 @@ struct lbm_batch {
                 }
             }
         }
-        auto upload = [&](uint2 *&dptr, const std::vector<uint2> &v) {
-            if (dptr) (void)hipFree(dptr);
-            dptr = dalloc<uint2>(std::max<size_t>(1, v.size()));
-            if (!v.empty()) HIPCHK(hipMemcpyAsync(dptr, v.data(), v.size() * sizeof(uint2), hipMemcpyHostToDevice, stream));
-        };
-        upload(ilist, il);
-        upload(blist, bl);
-        upload(alist, al);
-        HIPCHK(hipStreamSynchronize(stream));
+        // all three new before an old one goes: a list that cannot be allocated
+        // leaves the batch with those it has
+        uint2 *made[3] = {};
+        const std::vector<uint2> *from[3] = {&il, &bl, &al};
+        try {
+            for (int i = 0; i < 3; ++i) {
+                const std::vector<uint2> &v = *from[i];
+                made[i] = dalloc<uint2>(std::max<size_t>(1, v.size()));
+                if (!v.empty())
+                    HIPCHK(hipMemcpyAsync(made[i], v.data(), v.size() * sizeof(uint2), hipMemcpyHostToDevice, stream));
+            }
+            HIPCHK(hipStreamSynchronize(stream));
+        } catch (...) {
+            for (uint2 *p : made)
+                if (p) (void)hipFree(p);
+            throw;
+        }
+        for (uint2 *p : {ilist, blist, alist})
+            if (p) (void)hipFree(p);
+        ilist = made[0];
+        blist = made[1];
+        alist = made[2];
         n_interior = (uint32_t)il.size();
         n_boundary = (uint32_t)bl.size();
         n_all = (uint32_t)al.size();
