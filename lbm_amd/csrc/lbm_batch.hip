@@ -841,11 +841,13 @@ int lbm_batch_autotune(lbm_batch *b, uint32_t steps, int *best, float *ms) {
         const bool auto_path = b->auto_path, had_spare = b->spare[0] != nullptr;
         float t[LBM_BATCH_NUM_VARIANTS];
         int v_best = 0;
+        bool saved = false;
         b->auto_path = false;  // time each variant's own kernels
         try {
             HIPCHK(hipMemcpyAsync(snap, b->f[0], sb, hipMemcpyDeviceToDevice, b->stream));
             HIPCHK(hipMemcpyAsync(snap + sb, b->f[1], sb, hipMemcpyDeviceToDevice, b->stream));
             HIPCHK(hipMemcpyAsync(snap + 2 * sb, b->lag, lb, hipMemcpyDeviceToDevice, b->stream));
+            saved = true;
             hipEvent_t e0, e1;
             HIPCHK(hipEventCreate(&e0));
             HIPCHK(hipEventCreate(&e1));
@@ -881,7 +883,14 @@ int lbm_batch_autotune(lbm_batch *b, uint32_t steps, int *best, float *ms) {
             HIPCHK(hipMemcpyAsync(b->lag, snap + 2 * sb, lb, hipMemcpyDeviceToDevice, b->stream));
             HIPCHK(hipStreamSynchronize(b->stream));
         } catch (...) {
+            // as it was: whichever two sets are current now hold the state
             (void)hipStreamSynchronize(b->stream);
+            if (saved) {
+                (void)hipMemcpyAsync(b->f[0], snap, sb, hipMemcpyDeviceToDevice, b->stream);
+                (void)hipMemcpyAsync(b->f[1], snap + sb, sb, hipMemcpyDeviceToDevice, b->stream);
+                (void)hipMemcpyAsync(b->lag, snap + 2 * sb, lb, hipMemcpyDeviceToDevice, b->stream);
+                (void)hipStreamSynchronize(b->stream);
+            }
             (void)hipFree(snap);
             b->cur = cur;
             b->pform = pform;
