@@ -251,8 +251,9 @@ int lbm_load_state(lbm_grid *g, const void *buf, size_t bytes);
  * the single-grid semantics above (walls on rows 0 and ny-1, equilibrium inlet,
  * the selected outlet) with its own omega and inflow speed, and equals a single
  * grid of the same size and mask bit for bit.  All domains share one precision,
- * one boundary mode and one step count.  A step launches one interior and one
- * boundary kernel for all domains; lbm_batch_step replays them from a hipGraph
+ * one boundary mode and one step count.  One launch makes several steps of all
+ * domains (see the variants below); a single step is one interior and one
+ * boundary kernel for all domains, which lbm_batch_step replays from a hipGraph
  * two steps at a time. */
 typedef struct lbm_batch lbm_batch;
 
@@ -278,7 +279,8 @@ int lbm_batch_sync(lbm_batch *b);
 int lbm_batch_step_count(const lbm_batch *b, uint64_t *n);
 /* total cells, interior tiles and boundary segments of the current work lists */
 int lbm_batch_info(lbm_batch *b, uint64_t *cells, uint32_t *interior_tiles, uint32_t *boundary_segments);
-/* hipGraph replay on (default) or off */
+/* hipGraph replay of the single steps on (default) or off; launches of several
+ * steps are made directly either way */
 int lbm_batch_set_graph(lbm_batch *b, int enable);
 /* Batch variants: 0..5 the interior kernel's tile (cells per thread 1, 2, 4
  * -- twice that for binary16 -- in two list orders), 6 and 7 several steps per

@@ -35,8 +35,9 @@ namespace {
 // step at 8192 x 4096 in f32) and by the launch on small ones (3.7 us at 400 x
 // 160); two steps a launch from a ring of rows in LDS by its loads' latency and
 // halo rows (265 us).  Here a step of a large grid moves 16 bytes a cell and the
-// kernel is bound by VALU issue, 200 instructions a cell and step in f32 and 171
-// in binary16 counting the halo, 1.4 times the cells (158 and 134 us), and a
+// kernel is bound by VALU issue, 200 instructions a cell and step in f32, 171 in
+// binary16 and 206 centred on the free stream, counting the halo, 1.4 times the
+// cells (158, 134 and 155 us: the same time an instruction, not a byte), and a
 // small grid by the 2 us a launch and the 1 us of a region's step (1.6 us a
 // step).  More rows a wave mean less halo and fewer waves in flight: measured
 // at 8192 x 4096 in f32, us per step of 6 steps a launch, for 2 x 16, 3 x 12 and
