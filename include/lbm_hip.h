@@ -186,7 +186,12 @@ int lbm_launches(const lbm_grid *g, uint32_t n, uint32_t *launches);
 int lbm_step_timed(lbm_grid *g, uint32_t n, float *ms);
 /* Replaces LBM::get_compute_num (lbm.rs:1170-1172). */
 int lbm_step_count(const lbm_grid *g, uint64_t *n);
-/* The grid's hipStream_t, as an opaque pointer. */
+/* The grid's hipStream_t, as an opaque pointer.  A caller may capture lbm_step
+ * calls of even length on it, made while a stream is pending (after any step and
+ * before a mask change or read_f), and replay the graph whenever the steps made
+ * by other calls since are even in number and a stream is pending again.  After
+ * this call every lbm_step leaves the grid's sets where they were, which costs
+ * short calls a launch, and the sets are kept until the grid is destroyed. */
 int lbm_get_stream(const lbm_grid *g, void **stream);
 
 /* ---- fields ---------------------------------------------------------------------- */

@@ -489,7 +489,7 @@ struct lbm_batch {
         if (n < 2 || !spare[0] || !(auto_path || tile_variant(variant))) return {0, 0};
         const bool any = !tile_variant(variant);
         const int first = any ? 0 : variant - kTileFirst, last = any ? 1 : first;
-        return tile_plan(precision, first, last, n, pform,
+        return tile_plan(precision, first, last, n, false,
                          [&](int i, int s) { return (int64_t)tile_blocks[combination(i, s)]; });
     }
 

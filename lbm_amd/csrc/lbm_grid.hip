@@ -285,6 +285,9 @@ struct lbm_grid {
     uint64_t steps = 0;
     int variant = 0;  // step-kernel variant (cells per thread, non-temporal access)
     bool auto_path = true;  // no variant was ever set or tuned: steps go through k_tile where `spare` is there
+    // the caller has the stream and may hold graphs of calls: calls then leave the
+    // sets where they were, and none is given back
+    mutable bool stream_shared = false;
     std::string err;
     // device snapshot of the evolving state (both sets, fields, form, step count)
     char *snap = nullptr;
@@ -412,13 +415,15 @@ struct lbm_grid {
             throw;
         }
     }
-    void release_spare() { free_sets(spare); }
+    void release_spare() {
+        if (!stream_shared) free_sets(spare);
+    }
     // k_tile's sets for a tile variant; the state itself is always in f[0], f[1]
     // between calls.  Setting a variant does not take over the default path's
     // pair, as it fails where two more sets cannot be allocated; the pair's own
     // memory counts as free.
     void ensure_spare(bool take_over = true) {
-        if (spare[0] && (take_over || !auto_path)) return;
+        if (spare[0] && (take_over || !auto_path || stream_shared)) return;
         void *fresh[2];
         without_default_pair([&] { make_spare(fresh); });
         release_spare();
@@ -432,7 +437,7 @@ struct lbm_grid {
         try {
             return allocate();
         } catch (const HipError &) {
-            if (!auto_path || !spare[0]) throw;
+            if (!auto_path || !spare[0] || stream_shared) throw;
         }
         HIPCHK(hipStreamSynchronize(stream));
         release_spare();
@@ -559,7 +564,7 @@ struct lbm_grid {
             return {0, 0};
         const bool any = !tile_variant(variant);
         const int first = any ? 0 : variant - kTileFirst, last = any ? 1 : first;
-        return tile_plan(precision, first, last, n, pform, [&](int i, int s) {
+        return tile_plan(precision, first, last, n, stream_shared, [&](int i, int s) {
             const TileShape &sh = tile_shape(precision, i);
             return (int64_t)tile_nbx((int)X, s) * tile_nby((int)Y, sh.waves * sh.m, s);
         });
@@ -1290,6 +1295,7 @@ int lbm_step_count(const lbm_grid *g, uint64_t *n) {
 int lbm_get_stream(const lbm_grid *g, void **stream) {
     if (!g || !stream) return LBM_EINVAL;
     *stream = (void *)g->stream;
+    g->stream_shared = true;
     return LBM_OK;
 }
 

@@ -70,10 +70,10 @@ struct TilePlan {
     uint32_t launches;
 };
 //
-// even: an even number of launches where n is even.  Every launch trades the
-// state and spare sets, so a call of even length then leaves each where it
-// was, as the one-step kernel's calls do: a caller's graph of such a call can be
-// replayed.
+// even: an even number of launches, whatever n is (none for calls of two or three
+// steps).  Every launch trades the state and spare sets; after an even number
+// each is where it was, as after the one-step kernel's calls.  A caller's graph
+// of a call holds the sets it was captured with, and needs that of every call.
 template <class F>
 TilePlan tile_plan(int precision, int first, int last, uint32_t n, bool even, F &&blocks) {
     TilePlan best{first, 0};
@@ -87,7 +87,7 @@ TilePlan tile_plan(int precision, int first, int last, uint32_t n, bool even, F 
         }
         for (int s = 2; s <= kTileMaxSteps; ++s) {
             uint32_t launches = launches_of(n, s);
-            if (even && n % 2 == 0) launches += launches % 2;
+            if (even) launches += launches % 2;
             const uint32_t low = n / launches;
             if (low < 2) continue;
             const uint32_t more = n % launches;

@@ -26,10 +26,10 @@ int main(int argc, char **argv) {
                                 const TileShape &sh = tile_shape(precision, s);
                                 return (int64_t)tile_nbx(X, steps) * tile_nby(Y, sh.waves * sh.m, steps);
                             });
-                            // (two steps in an even number of launches: none)
+                            // (two or three steps in an even number of launches: none)
                             const bool ok = p.launches ? adds_up(n, p.launches, 2) && p.shape >= first && p.shape <= last
-                                                       : n == 2 && even;
-                            if (!ok || (even && n % 2 == 0 && p.launches % 2)) {
+                                                       : n <= 3 && even;
+                            if (!ok || (even && p.launches % 2)) {
                                 std::printf("n %u precision %d shapes %d..%d even %d: shape %d, %u launches\n", n,
                                             precision, first, last, even, p.shape, p.launches);
                                 return 1;
