@@ -1601,6 +1601,8 @@ struct lbm_unet {
     uint16_t *wb = nullptr, *wt = nullptr;
     float *out32 = nullptr, *tgt = nullptr, *wm = nullptr, *fields = nullptr, *loss = nullptr, *inv_wsum = nullptr;
     double *wsums = nullptr;  // partial sums of the loss weights, then their sum
+    double *wsum_host = nullptr;  // that sum, in pinned memory, and the event of its arrival
+    hipEvent_t wsum_there = nullptr;
     uint16_t *gout = nullptr;
     Act x, e1a, e1, p1, e2a, e2, p2, e3a, e3, p3, e4a, e4, d3u, k3, d3a, d3, d2u, k2, d2a, d2, d1u, k1, d1a, d1;
     float *ws = nullptr;  // split-K partial sums
@@ -1657,6 +1659,10 @@ struct lbm_unet {
         }
         drop_graph();
         staging.release();
+        if (wsum_there) (void)hipEventDestroy(wsum_there);
+        if (wsum_host) (void)hipHostFree(wsum_host);
+        wsum_there = nullptr;
+        wsum_host = nullptr;
         for (void *p : mem) (void)hipFree(p);
         mem.clear();
         if (stream) (void)hipStreamDestroy(stream);
@@ -1719,6 +1725,8 @@ struct lbm_unet {
         loss = (float *)alloc(4);
         inv_wsum = (float *)alloc(4);
         wsums = (double *)alloc((kSumBlocks + 1) * sizeof(double));
+        HIPCHK(hipHostMalloc((void **)&wsum_host, sizeof(double), hipHostMallocDefault));
+        HIPCHK(hipEventCreateWithFlags(&wsum_there, hipEventDisableTiming));
         // split-K workspace: the largest need over the forward and input-gradient convolutions
         for (const Conv &c : convs) {
             // level of the layer from its output (forward) / input (gradient) channel count
@@ -1890,23 +1898,31 @@ struct lbm_unet {
     // host inputs -> device; returns the loss
     float loss_and_grad(const float *hx, const float *hy, const float *hwm) {
         const size_t P = (size_t)B * H * W;
-        const Piece in[3] = {{(void *)hx, fields, P * 32}, {(void *)hy, tgt, P * 12}, {(void *)hwm, wm, P * 4}};
-        HIPCHK(staging.copy(dev, stream, in, 3, false));
-        hipLaunchKernelGGL(k_pack_input, dim3(nblk(4 * P)), dim3(256), 0, stream, fields, x.a, (long long)P);
-        forward();
+        // the weights first: their sum is there, and a call without any refused,
+        // before the network has anything to do, while the other inputs are copied
+        const Piece in[3] = {{(void *)hwm, wm, P * 4}, {(void *)hx, fields, P * 32}, {(void *)hy, tgt, P * 12}};
+        HIPCHK(staging.copy(dev, stream, in, 1, false));
         hipLaunchKernelGGL(k_weight_sum, dim3(kSumBlocks), dim3(256), 0, stream, wm, wsums, P);
         hipLaunchKernelGGL(k_weight_inverse, dim3(1), dim3(kSumBlocks), 0, stream, wsums, wsums + kSumBlocks, inv_wsum,
                            loss);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipMemcpyAsync(wsum_host, wsums + kSumBlocks, 8, hipMemcpyDeviceToHost, stream));
+        HIPCHK(hipEventRecord(wsum_there, stream));
+        HIPCHK(staging.copy(dev, stream, in + 1, 2, false));
+        HIPCHK(hipEventSynchronize(wsum_there));
+        if (!(*wsum_host > 0.0)) {
+            HIPCHK(hipStreamSynchronize(stream));  // the host inputs go back to the caller
+            ucheck(false, "loss weights sum to zero");
+        }
+        hipLaunchKernelGGL(k_pack_input, dim3(nblk(4 * P)), dim3(256), 0, stream, fields, x.a, (long long)P);
+        forward();
         hipLaunchKernelGGL(k_mse, dim3(std::min<unsigned>(kMseBlocks, nblk(4 * P))), dim3(256), 0, stream, out32, tgt, wm, gout, loss, (long long)P,
                            inv_wsum);
         HIPCHK(hipGetLastError());
         backward();
         float l = 0.0f;
-        double wsum = 0.0;
         HIPCHK(hipMemcpyAsync(&l, loss, 4, hipMemcpyDeviceToHost, stream));
-        HIPCHK(hipMemcpyAsync(&wsum, wsums + kSumBlocks, 8, hipMemcpyDeviceToHost, stream));
         HIPCHK(hipStreamSynchronize(stream));
-        ucheck(wsum > 0.0, "loss weights sum to zero");
         return l;
     }
 
